@@ -49,3 +49,15 @@ def test_consensus_alignment_like(eng):
                 r[k] = "-"
         rows.append("".join(r))
     assert eng.consensus(rows) == po.consensus(rows)
+
+
+@pytest.mark.parametrize("n, L", [(1, 1), (1, 64), (2, 65), (7, 63), (8, 129), (15, 64), (16, 1), (17, 200), (127, 65),
+                                  (128, 64), (129, 3), (257, 191), (3000, 2)])
+def test_consensus_row_shares(eng, n, L):
+    # rows dealt to 16 waves of 8 loads each, columns to workgroups of 64: one
+    # below, at and above the shares' edges; few letters, so classes tie and
+    # the first sequence decides
+    rng = random.Random(1000 * n + L)
+    rows = ["".join(rng.choice("AST-") for _ in range(L)) for _ in range(n)]
+    for pl in (-1.0, 0.0):
+        assert eng.consensus(rows, pl) == po.consensus(rows, pl)

@@ -8,9 +8,9 @@
 // reaches the plurality (else '?').
 //
 // A sequence's score depends only on the class of its residue (23 BLOSUM62
-// rows or "not a letter"), so one thread per column counts the classes in
-// one pass over the rows (coalesced: consecutive threads read consecutive
-// columns of a row) and scores each class present against the counts,
+// rows or "not a letter"), so a column's classes are counted in one pass over
+// the rows (coalesced: consecutive lanes read consecutive columns of a row)
+// and each class present is scored against the counts,
 // O(nseq + 24^2) per column: score(k) = sum_j cnt[j] * S(k, j) - S(k, k),
 // the self pairing removed.  The winner is the class of best score whose
 // first sequence comes first -- the reference's strict ">" over sequences in
@@ -28,7 +28,8 @@
 namespace {
 
 constexpr int CK = 24;       // 23 BLOSUM62 rows, then "not a letter"
-constexpr int CT = 256;      // threads (columns) per workgroup
+constexpr int CW = 16;       // waves per workgroup: shares of the rows
+constexpr int CU = 8;        // row loads a lane has in flight
 
 struct ConsArgs {
   const uint8_t *msa;        // row s at msa + s * len
@@ -40,45 +41,68 @@ struct ConsArgs {
   const int8_t *match;       // CK x CK: 1 when a pairing counts as a match
 };
 
-__global__ __launch_bounds__(CT) void consensus_kernel(ConsArgs A) {
+// A workgroup takes 64 columns (a lane each) and deals its rows to CW waves,
+// which count classes into shared LDS tables (a lane's column is its own bank,
+// so the atomics never conflict inside a wave).  Bound by the latency of the
+// row loads: a thread per column alone, reading its rows one after the other,
+// took 233 us for 512 x 2,000 (8 workgroups in all); 16 waves of 8 loads in
+// flight take about 14 us.  The scores are dealt by class, one or two a wave.
+__global__ __launch_bounds__(64 * CW) void consensus_kernel(ConsArgs A) {
   __shared__ int8_t cls[256];
   __shared__ int32_t sc[CK * CK], mt[CK * CK];
-  __shared__ int32_t cnt[CK][CT], first[CK][CT];
-  const int tid = threadIdx.x;
-  cls[tid] = A.cls[tid];
-  for (int x = tid; x < CK * CK; x += CT) {
+  __shared__ int32_t cnt[CK][64], first[CK][64], sco[CK][64], mat[CK][64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if (tid < 256) cls[tid] = A.cls[tid];
+  for (int x = tid; x < CK * CK; x += 64 * CW) {
     sc[x] = A.score[x];
     mt[x] = A.match[x];
   }
+  for (int x = tid; x < CK * 64; x += 64 * CW) {
+    (&cnt[0][0])[x] = 0;
+    (&first[0][0])[x] = INT_MAX;
+  }
   __syncthreads();
-  const int c = blockIdx.x * CT + tid;
-  if (c >= A.len) return;
+  const int c = blockIdx.x * 64 + lane;
+  const bool in = c < A.len;
+  const uint8_t *col = A.msa + (in ? c : 0);
+  const int per = (A.nseq + CW - 1) / CW, s0 = wave * per, s1 = s0 + per < A.nseq ? s0 + per : A.nseq;
+  for (int s = s0; s < s1; s += CU) {
+    uint8_t v[CU];
 #pragma unroll
-  for (int k = 0; k < CK; ++k) {
-    cnt[k][tid] = 0;
-    first[k][tid] = INT_MAX;
+    for (int u = 0; u < CU; ++u) v[u] = col[(size_t)(s + u < s1 ? s + u : s1 - 1) * A.len];
+#pragma unroll
+    for (int u = 0; u < CU; ++u) {
+      if (s + u < s1) {
+        const int k = cls[v[u]];
+        atomicAdd(&cnt[k][lane], 1);
+        atomicMin(&first[k][lane], s + u);
+      }
+    }
   }
-  const uint8_t *col = A.msa + c;
-  for (int s = 0; s < A.nseq; ++s) {
-    const int k = cls[col[(size_t)s * A.len]];
-    if (cnt[k][tid]++ == 0) first[k][tid] = s;
-  }
-  int best = INT_MIN, best_first = INT_MAX, best_match = 0;
-  for (int k = 0; k < CK; ++k) {
-    const int ck = cnt[k][tid];
-    if (ck == 0) continue;
+  __syncthreads();
+  int32_t cj[CK];
+#pragma unroll
+  for (int j = 0; j < CK; ++j) cj[j] = cnt[j][lane];
+  for (int k = wave; k < CK; k += CW) {
     int s = -sc[k * CK + k], m = -mt[k * CK + k];  // no pairing with itself
 #pragma unroll
     for (int j = 0; j < CK; ++j) {
-      const int cj = cnt[j][tid];
-      s += cj * sc[k * CK + j];
-      m += cj * mt[k * CK + j];
+      s += cj[j] * sc[k * CK + j];
+      m += cj[j] * mt[k * CK + j];
     }
-    const int f = first[k][tid];
-    if (s > best || (s == best && f < best_first)) {
+    sco[k][lane] = s;
+    mat[k][lane] = m;
+  }
+  __syncthreads();
+  if (wave != 0 || !in) return;
+  int best = INT_MIN, best_first = INT_MAX, best_match = 0;
+#pragma unroll
+  for (int k = 0; k < CK; ++k) {
+    const int f = first[k][lane], s = sco[k][lane];
+    if (f != INT_MAX && (s > best || (s == best && f < best_first))) {
       best = s;
       best_first = f;
-      best_match = m;
+      best_match = mat[k][lane];
     }
   }
   A.out[c] = (double)best_match >= A.plurality ? (char)col[(size_t)best_first * A.len] : '?';
@@ -144,7 +168,7 @@ int ta_consensus(ta_ctx *ctx, const char *const *rows, int32_t nseq, int32_t len
     a.score = tb + offsetof(ConsTables, score);
     a.match = tb + offsetof(ConsTables, match);
     (void)hipGetLastError();
-    hipLaunchKernelGGL(consensus_kernel, dim3((len + CT - 1) / CT), dim3(CT), 0, st, a);
+    hipLaunchKernelGGL(consensus_kernel, dim3((len + 63) / 64), dim3(64 * CW), 0, st, a);
     if (hipGetLastError() != hipSuccess ||
         hipMemcpyAsync(out, d_out, (size_t)len, hipMemcpyDeviceToHost, st) != hipSuccess)
       rc = TA_E_DEVICE;
