@@ -140,3 +140,34 @@ def test_bad_letters_and_small_buffer(eng):
     rc = ta.lib().ta_align_pair(eng.ctx, ctypes.byref(params), b"ACDEFGHIK", 9, b"ACDGHIK", 7, ctypes.byref(res),
                                 buf, 2, ctypes.byref(used))
     assert rc == -3 and used.value == res.cigar_len > 2
+
+
+# Rows per lane change at 256 and 512 rows, strips at 64, 128 and 256; the largest pairs (256 x 921, 512 x 489,
+# 640 x 385, 1025 x 193) keep their codes in device memory; |extend| > |open| makes a border value positive.
+@pytest.mark.parametrize("la, lb", [(1, 1), (1, 63), (63, 1), (64, 64), (65, 8), (66, 129), (127, 70), (128, 65),
+                                    (192, 7), (193, 130), (255, 256), (256, 257), (257, 100), (384, 63), (385, 71),
+                                    (511, 300), (512, 489), (256, 921), (640, 385), (600, 380), (1025, 193), (1025, 64),
+                                    (2050, 9), (128, 1553)])
+@pytest.mark.parametrize("mode", [ta.GLOBAL, ta.LOCAL])
+def test_strip_edges(eng, la, lb, mode):
+    rng = random.Random(la * 10007 + lb)
+    a = rand_prot(rng, la)
+    b = (mutate(rng, a) + rand_prot(rng, lb))[:lb]
+    tie = rand_prot(rng, lb, "AGW")
+    for go, ge in ((-11, -1), (-2, -7), (0, 0)):
+        check(eng, [(a, b), (rand_prot(rng, la, "AGW"), tie)], "edges %d %d" % (go, ge), mode=mode, gap_open=go,
+              gap_extend=ge)
+    d = rand_prot(rng, la, "ACGT")
+    e = (mutate(rng, d, 0.1, 0.02, "ACGT") + rand_prot(rng, lb, "ACGT"))[:lb]
+    check(eng, [(d, e)], "edges dna", mode=mode, alphabet=ta.DNA, gap_open=-1000, gap_extend=-1000, match=100,
+          mismatch=-100)
+    check(eng, [(d, e)], "edges dna", mode=mode, alphabet=ta.DNA, gap_open=-5, gap_extend=-2, match=2, mismatch=-3)
+
+
+def test_large_keeps_flags(eng):
+    # the largest pairs of the low-latency path and the first beyond it: F_I32 marks the former
+    params = ta.engine.make_params(mode=ta.GLOBAL, gap_open=-11)
+    rng = random.Random(5)
+    for la, lb, on in ((512, 489, True), (512, 490, False), (640, 385, True), (640, 386, False)):
+        g = eng.align_pair(rand_prot(rng, la), rand_prot(rng, lb), params)
+        assert bool(g.flags & ta.F_I32) == on, (la, lb)

@@ -7,19 +7,20 @@
 namespace ta {
 
 constexpr int PAIR_WAVES = 4;                // waves of the workgroup (one per SIMD)
-constexpr int PAIR_R = 2;                    // query rows per lane
-constexpr int PAIR_STRIP = 64 * PAIR_R;      // rows per strip
-constexpr int PAIR_PAD = 31;                 // code of a row / column outside the sequences
+constexpr int PAIR_PAD_LINE = 31;            // table line of a row outside the query
 constexpr int PAIR_BAD_LETTER = 1;           // PairOut::status bits
 constexpr int PAIR_GAVE_UP = 2;
 
-// LDS byte offsets of the kernel's arrays for an m x n pair.
+// Rows per lane, and LDS byte offsets of the kernel's arrays, for an m x n pair.
 struct PairLayout {
+  int32_t R;                // rows per lane: 1, 2 or 4
   int32_t T, S;             // steps per strip (n + 63, rounded to 8), strips
-  int32_t ring_len;         // int2 entries per ring slot
+  int32_t slot_bytes;       // score slot of a wave
+  int32_t ring_len;         // int2 entries per ring
   int32_t runs_cap;         // CIGAR run slots
-  int32_t acode, bcode, sync, ring, planes, runs;
+  int32_t acode, bcode, sync, slots, ring, planes, runs, window;
   int32_t bytes;            // total LDS
+  int32_t plane_bytes;      // direction codes of all strips in device memory; 0: they are in LDS
 };
 
 // Written by the kernel: the result, then nruns CIGAR runs ((len << 2) | op,
@@ -39,10 +40,12 @@ struct PairArgs {
   int32_t spin_limit;
   int32_t walk_cap;         // most steps the walk may take before it ends flagged (above any walk normally)
   PairLayout lay;
+  uint8_t *planes;          // lay.plane_bytes of device memory, where the codes do not fit in LDS
   PairOut *out;             // device-writable; m + n + 2 run slots follow it
 };
 
-PairLayout pair_layout(int m, int n);
+// The form for an m x n pair of an alphabet of K letters within lds_max bytes of LDS.
+PairLayout pair_layout(int m, int n, int K, int lds_max);
 // One workgroup on stream st; TA_E_DEVICE when the launch fails.
 int pair_launch(const PairArgs &A, hipStream_t st);
 

@@ -6,23 +6,26 @@
 // one launch of one workgroup that takes the letters and returns the CIGAR
 // runs, with nothing else on the device:
 //  * the letters are read straight from host staging (mapped, pinned
-//    memory) and encoded in LDS, the substitution table is built in LDS
-//    from a copy compiled into the kernel;
-//  * the fill is the striped form of the batch fill in int32 with PR rows
-//    per lane: a strip is 64 lanes x PR rows, strip s runs on wave s % PW
-//    and trails strip s-1 through a ring of bottom rows in LDS (progress
-//    counters, workgroup scope, bounded waits);
-//  * direction codes (4 bits per cell) stay in LDS, so the walk never
-//    touches HBM: wave 0 loads a 16 x 16-cell window of codes into its
-//    lanes (one byte per lane per row pair) and steps through it with
-//    readlane on wave-uniform coordinates, reloading when the walk leaves
-//    the window;
+//    memory) and encoded in LDS, beside a substitution table compiled in;
+//  * the fill is strip.h's int32 sweep: strips of 64 lanes x 1, 2 or 4 rows,
+//    strip s on wave s % 4, trailing strip s-1 through a ring of bottom rows
+//    in LDS (progress counters, workgroup scope, bounded waits);
+//  * direction codes (4 bits per cell) stay in LDS (in device memory where
+//    they do not fit beside the tables), and wave 0 walks them back a CIGAR
+//    run at a time (walk.h);
 //  * the result and the runs go straight back to host staging.
-// Pairs whose codes do not fit in LDS take the batch path (the caller's
-// entry point decides).  Recurrence, boundaries and tie-breaks are those of
-// the specification the CPU oracle implements (oracle/gotoh.c); the local
+// Pairs larger than that take the batch path (the caller's entry point
+// decides).  Recurrence, boundaries and tie-breaks are those of the
+// specification the CPU oracle implements (oracle/gotoh.c); the local
 // stop cell (H = 0) is marked in its code as d = 0, x = 1 (a combination
 // the H-source never takes), since no walk reads another bit of such a cell.
+//
+// Bound by dependent steps: n + 80 (strips) of the fill, each as long as one
+// wave takes to issue it, and a lookup per CIGAR run of the walk.  Call to
+// CIGAR, with two rows per lane, 322 cycles a step and a walk of 430 cycles a
+// cell, and now: 24 x 28 global protein 36 / 24 us, 300 x 320 155 / 76 us (of
+// 2.4 GHz cycles: fill 117,000, walk 28,000, tables and letters 7,500),
+// 400 x 420 local DNA 217 / 105 us.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -37,78 +40,232 @@
 #include "common.h"
 #include "pair.h"
 #include "runtime_internal.h"
+#include "strip.h"
+#include "walk.h"
 
 namespace ta {
 
-__constant__ int8_t kBlosumDev[] = {TA_BLOSUM62_LOWER};
-__constant__ char kProtOrderDev[] = TA_PROT_ORDER;
-
 namespace {
 
+// Substitution lines (32 bytes a residue, pads at PAD_SCORE) and letter maps,
+// compiled in and loaded as they are.
+struct alignas(16) PairTables {
+  int8_t prot[32 * 32];
+  int8_t map[2][256];  // TA_PROTEIN, TA_DNA: letter -> code, -1 outside the alphabet
+};
+constexpr PairTables pair_tables() {
+  constexpr int8_t lower[] = {TA_BLOSUM62_LOWER};
+  constexpr char order[] = TA_PROT_ORDER;
+  PairTables t{};
+  for (int x = 0; x < 32 * 32; ++x) t.prot[x] = PAD_SCORE;
+  for (int r = 0; r < TA_PROT_K; ++r)
+    for (int c = 0; c < TA_PROT_K; ++c) {
+      const int hi = r > c ? r : c, lo = r > c ? c : r;
+      t.prot[32 * r + c] = lower[hi * (hi + 1) / 2 + lo];
+    }
+  for (int x = 0; x < 256; ++x) {
+    const int u = (x >= 'a' && x <= 'z') ? x - 32 : x;
+    int p = -1;
+    for (int r = 0; r < TA_PROT_K; ++r)
+      if (order[r] == u) p = r;
+    if (u == 'J' || u == 'O' || u == 'U') p = TA_PROT_K - 1;  // scored as X
+    t.map[0][x] = (int8_t)p;
+    t.map[1][x] = (int8_t)(u == 'A' ? 0 : u == 'C' ? 1 : u == 'G' ? 2 : u == 'T' ? 3 : -1);
+  }
+  return t;
+}
+static_assert(TA_PROTEIN == 0 && TA_DNA == 1 && TA_PROT_K + 1 <= STRIP_NC, "alphabet codes");
+__device__ const PairTables kPairTables = pair_tables();
+
 // LDS words of the sync area.
-enum { SY_STATUS = 0, SY_SCORE = 1, SY_PROG = 4, SY_BEST = 8, SY_WORDS = 64 };
+enum { SY_STATUS = 0, SY_SCORE = 1, SY_PROG = 4, SY_BEST = 8, SY_DUMP = 24, SY_READY = 25, SY_ZERO = 32, SY_EDGE = 48,
+       SY_WORDS = 64 };
 
-__device__ __forceinline__ int wave_shr1(int old, int v) {
-  return __builtin_amdgcn_update_dpp(old, v, 0x138, 0xf, 0xf, false);  // wave_shr:1, lane 0 takes old
+// 16 letters of a sequence (positions x .. x + 15, those past len ignored) as
+// codes, `pad` past its end; bad: a letter outside the alphabet.
+__device__ __forceinline__ uint4 encode16(const int8_t *lmap, uint4 v, int x, int len, int pad, int &bad) {
+  uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    uint32_t o = 0;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      const bool in = x + 4 * q + b < len;
+      const int c = lmap[(w[q] >> (8 * b)) & 0xff];
+      bad |= in && c < 0;
+      o |= (uint32_t)(in && c >= 0 ? c : pad) << (8 * b);
+    }
+    w[q] = o;
+  }
+  return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
-// (h desc, i asc, j asc): the local end-cell order.
-__device__ __forceinline__ bool better(int h, int i, int j, int bh, int bi, int bj) {
-  return h > bh || (h == bh && (i < bi || (i == bi && j < bj)));
-}
+// A strip's surroundings in the workgroup's LDS (strip.h): the ring of the
+// strip above, its progress counter, the pair's column codes.  The ring
+// holds column x at entry x + 64.
+template <int PR, bool GP>
+struct PairIO {
+  const uint8_t *bcode;      // this lane's first column code, at step 0
+  uint32_t slot_add;
+  int32_t *pin, *pout, *status;
+  int2 *rin, *rout;          // rin: lane 0's entries (strip 0: 8 border entries), the others' 8 zero entries
+  int rin_step, need0, cols, s, spin_limit, seen = 0;
+  uint32_t *pl;              // this lane's next dword, pl_step apart (a lane past the query: one unused dword)
+  int pl_step;
+  bool lost = false;         // a wait gave up: no more waits
 
-__device__ __forceinline__ int load_code(const int8_t *lmap, char ch, int &bad) {
-  const int c = lmap[(uint8_t)ch];
-  bad |= c < 0;
-  return c < 0 ? PAIR_PAD : c;
-}
+  __device__ __forceinline__ uint64_t codes(int b) const {
+    uint64_t w;
+    __builtin_memcpy(&w, bcode + 8 * b, 8);
+    return w;
+  }
+  __device__ __forceinline__ int need(int b) const { return need0 | (8 * b + 8 < cols ? 8 * b + 8 : cols); }
+  __device__ __forceinline__ void peek() {
+    seen = __hip_atomic_load(pin, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+  __device__ __forceinline__ void await(int b) {
+    const int want = need(b);
+    int spins = 0;
+    while (!lost && __builtin_amdgcn_readfirstlane(seen) < want) {
+      if (++spins > spin_limit) {
+        if ((threadIdx.x & 63) == 0) atomicOr(status, PAIR_GAVE_UP);
+        lost = true;
+      }
+      __builtin_amdgcn_s_sleep(1);
+      peek();
+    }
+    asm volatile("" ::: "memory");  // the ring's reads stay below (a wave's LDS accesses keep their order)
+  }
+  __device__ __forceinline__ void tops(int b, int half, int (&g)[8], int (&f)[8]) const {
+    const int4 *r = (const int4 *)(rin + b * rin_step) + 2 * half;
+    const int4 v = r[0], w = r[1];
+    const int q = 4 * half;
+    g[q] = v.x; f[q] = v.y; g[q + 1] = v.z; f[q + 1] = v.w;
+    g[q + 2] = w.x; f[q + 2] = w.y; g[q + 3] = w.z; f[q + 3] = w.w;
+  }
+  __device__ __forceinline__ void bottom(int b, const int (&g)[8], const int (&f)[8]) {
+    if ((threadIdx.x & 63) == 63) {
+      int2 *r = rout + 8 * b + 1;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) r[q] = make_int2(g[q], f[q]);
+      int done = 8 * b + 8 - 63;
+      done = done < 0 ? 0 : done;
+      asm volatile("" ::: "memory");  // the entries first (a wave's LDS accesses keep their order)
+      __hip_atomic_store(pout, ((s + 1) << 20) | done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+  }
+  __device__ __forceinline__ void planes(uint32_t dw) {
+    *pl = dw;
+    pl += pl_step;
+  }
+};
 
-template <bool LOCAL>
-__global__ __launch_bounds__(64 * PAIR_WAVES) void pair_kernel(PairArgs A) {
-  extern __shared__ __align__(16) uint8_t lds[];
+// Direction codes in LDS, all at hand: dwords [strip][t / SPD][lane], the
+// last strip as wide as it has lanes.
+template <int PR>
+struct PairCodes {
+  const uint32_t *pl;
+  uint32_t strip_dw;         // dwords of a full strip
+  uint32_t last, last_lanes; // the last strip, and its width
+  __device__ __forceinline__ int code(int i, int j) const {
+    constexpr uint32_t SPD = strip_spd(PR);
+    const uint32_t r = (uint32_t)i - 1, L = r / PR, s = L >> 6, l = L & 63, t = (uint32_t)j - 1 + l;
+    const uint32_t dw = pl[__umul24(s, strip_dw) + __umul24(t / SPD, s == last ? last_lanes : 64u) + l];
+    return strip_code<PR>(dw, t % SPD, r % PR);
+  }
+  __device__ __forceinline__ bool refill(int, int) { return false; }
+};
+
+// Codes in device memory ([strip][t / SPD][64 lanes]): a window of them in
+// LDS, 32 lanes' rows up from the walk's cell, for each lane WD dwords
+// around the diagonal through it.
+template <int PR>
+struct StripWindow {
+  static constexpr int SPD = strip_spd(PR), WL = 32, WD = 32 / SPD + 1;
+  const uint32_t *pl;
+  uint32_t *win;  // WL x WD
+  int T;
+  int L0, u0;     // the window's first (lowest) lane, counted over all strips, and its 0-based column
+  // first staged dword of lane L0 - q
+  __device__ __forceinline__ int first(int q) const {
+    const int t = u0 - q * PR + ((L0 - q) & 63), d = t / SPD - WD / 2, top = T / SPD - WD;
+    return d > top ? (top < 0 ? 0 : top) : (d < 0 ? 0 : d);
+  }
+  __device__ __forceinline__ int code(int i, int j) const {
+    const int L = (int)((uint32_t)(i - 1) / PR), q = L0 - L, t = j - 1 + (L & 63);
+    const int d = (int)((uint32_t)t / SPD) - first(q);
+    if (q < 0 || q >= WL || d < 0 || d >= WD) return -1;
+    return strip_code<PR>(win[q * WD + d], (uint32_t)t % SPD, (uint32_t)(i - 1) % PR);
+  }
+  __device__ __forceinline__ bool refill(int i, int j) {
+    const bool moved = (i - 1) / PR != L0 || j - 1 != u0;
+    L0 = (i - 1) / PR;
+    u0 = j - 1;
+    constexpr int N = WL * WD, U = (N + 63) / 64;
+    uint32_t v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int x = u * 64 + (int)(threadIdx.x & 63), q = x / WD, d = first(q) + x % WD, L = L0 - q;
+      v[u] = x < N && L >= 0 && d < T / SPD ? pl[((size_t)(L >> 6) * (T / SPD) + d) * 64 + (L & 63)] : 0;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int x = u * 64 + (int)(threadIdx.x & 63);
+      if (x < N) win[x] = v[u];
+    }
+    return moved;
+  }
+};
+
+template <int PR, bool LOCAL, bool GP>
+__global__ __launch_bounds__(64 * PAIR_WAVES) __attribute__((amdgpu_waves_per_eu(1, 1))) void pair_kernel(PairArgs A) {
+  extern __shared__ __align__(256) uint8_t lds[];
   const PairLayout &Y = A.lay;
-  int8_t *tab = (int8_t *)lds;                   // [a code][b code], 32 x 32
+  uint8_t *tab = lds;                            // 32-byte line per residue code
   int8_t *lmap = (int8_t *)(lds + 1024);         // letter -> code, -1 outside the alphabet
   uint8_t *acode = lds + Y.acode;
-  uint8_t *bcode = lds + Y.bcode;
+  uint8_t *bcode = lds + Y.bcode;                // 64 pads, the columns, pads
   int32_t *sy = (int32_t *)(lds + Y.sync);
-  int2 *ring = (int2 *)(lds + Y.ring);
-  uint8_t *planes = lds + Y.planes;
-  uint32_t *runs = (uint32_t *)(lds + Y.runs);
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int m = A.m, n = A.n, T = Y.T, S = Y.S;
-  const int open = A.open, ext = A.ext;
+  const int m = A.m, n = A.n, T = Y.T, S = Y.S, nthr = blockDim.x;
+  const bool prot = A.alphabet == TA_PROTEIN;
+  const int K = prot ? TA_PROT_K : 4, pad = K;
 
-  for (int x = tid; x < 1024; x += blockDim.x) {
-    const int r = x >> 5, c = x & 31;
-    int v = 0;
-    if (A.alphabet == TA_PROTEIN) {
-      if (r < TA_PROT_K && c < TA_PROT_K) {
-        const int hi = r > c ? r : c, lo = r > c ? c : r;
-        v = kBlosumDev[hi * (hi + 1) / 2 + lo];
+  // Tables and letters: every load before the first use (the letters come
+  // over the host link).  Each thread takes 16 letters of either sequence.
+  const uint4 *ga = (const uint4 *)A.a, *gb = (const uint4 *)A.b;
+  uint4 va = make_uint4(0, 0, 0, 0), vb = va;
+  if (16 * tid < m) va = ga[tid];
+  if (16 * tid < n) vb = gb[tid];
+  for (int x = tid; x < 256; x += nthr) {
+    uint32_t v = ((const uint32_t *)kPairTables.prot)[x];
+    if (!prot) {
+      v = 0;
+      for (int b = 0; b < 4; ++b) {
+        const int r = x >> 3, c = ((x & 7) << 2) + b;
+        v |= (uint32_t)(uint8_t)(r < 4 && c < 4 ? (r == c ? A.match : A.mismatch) : PAD_SCORE) << (8 * b);
       }
-    } else if (r < 4 && c < 4) {
-      v = r == c ? A.match : A.mismatch;
     }
-    tab[x] = (int8_t)v;
+    ((uint32_t *)tab)[x] = v;
+    if (x < 64) ((uint32_t *)lmap)[x] = ((const uint32_t *)kPairTables.map[prot ? 0 : 1])[x];
   }
-  for (int x = tid; x < 256; x += blockDim.x) {
-    const int u = (x >= 'a' && x <= 'z') ? x - 32 : x;
-    int code = -1;
-    if (A.alphabet == TA_PROTEIN) {
-      for (int r = 0; r < TA_PROT_K; ++r)
-        if (kProtOrderDev[r] == u) code = r;
-      if (u == 'J' || u == 'O' || u == 'U') code = TA_PROT_K - 1;  // scored as X
-    } else {
-      code = u == 'A' ? 0 : (u == 'C' ? 1 : (u == 'G' ? 2 : (u == 'T' ? 3 : -1)));
-    }
-    lmap[x] = (int8_t)code;
+  if (tid < SY_WORDS) sy[tid] = tid == SY_READY ? 0x7fffffff : tid >= SY_EDGE && !LOCAL ? 2 * (A.open - A.ext) : 0;
+  if (LOCAL && S > 1) {  // ring columns no strip stores (from T - 63 on): 0
+    int2 *tail = (int2 *)(lds + Y.ring) + T + 1;
+    const int rings = S - 1 < PAIR_WAVES ? S - 1 : PAIR_WAVES, w = Y.ring_len - T - 1;
+    for (int x = tid; x < rings * w; x += nthr) tail[(x / w) * Y.ring_len + x % w] = make_int2(0, 0);
   }
-  if (tid < SY_WORDS) sy[tid] = 0;
+  if (tid < 16) ((uint32_t *)bcode)[tid] = 0x01010101u * (uint32_t)pad;
   __syncthreads();
   int bad = 0;
-  for (int x = tid; x < m; x += blockDim.x) acode[x] = (uint8_t)load_code(lmap, A.a[x], bad);
-  for (int x = tid; x < T + 8; x += blockDim.x) bcode[x] = x < n ? (uint8_t)load_code(lmap, A.b[x], bad) : PAIR_PAD;
+  for (int x = 16 * tid; x < m || x < T + 16; x += 16 * nthr) {
+    if (x != 16 * tid) {
+      if (x < m) va = ga[x / 16];
+      if (x < n) vb = gb[x / 16];
+    }
+    if (x < m) *(uint4 *)(acode + x) = encode16(lmap, va, x, m, pad, bad);
+    if (x < T + 16) *(uint4 *)(bcode + 64 + x) = encode16(lmap, vb, x, n, pad, bad);
+  }
   if (bad) atomicOr(&sy[SY_STATUS], PAIR_BAD_LETTER);
   __syncthreads();
   if (sy[SY_STATUS] & PAIR_BAD_LETTER) {
@@ -117,147 +274,54 @@ __global__ __launch_bounds__(64 * PAIR_WAVES) void pair_kernel(PairArgs A) {
   }
 
   // ---- fill
-  int bh = 0, bi = 0x7fffffff, bj = 0x7fffffff;  // lane's best cell (local), 1-based
+  constexpr int SPD = strip_spd(PR);
+  const int slot = Y.slots + wv * Y.slot_bytes;
+  int2 *const ring = (int2 *)(lds + Y.ring);
+  const int last_lanes = (m - (S - 1) * 64 * PR + PR - 1) / PR;
+  StripEnd end;
   for (int s = wv; s < S; s += PAIR_WAVES) {
-    const int r0 = s * PAIR_STRIP + PAIR_R * lane;  // 0-based row of the lane's first row
-    const int8_t *t0 = tab + ((r0 < m ? acode[r0] : PAIR_PAD) << 5);
-    const int8_t *t1 = tab + ((r0 + 1 < m ? acode[r0 + 1] : PAIR_PAD) << 5);
-    auto left = [&](int i) { return (LOCAL || i == 0) ? 0 : open + (i - 1) * ext; };  // H(i, 0), 1-based
-    int H0 = left(r0 + 1), H1 = left(r0 + 2), E0 = NEG32, E1 = NEG32;
-    int hd = left(r0);  // H(r0, c - 1) of the step to come (1-based row r0 = the row above)
-    int Hbot = 0, Fbot = NEG32;
-    // Local: one key per row, (H << 16) | (0xFFFF - column): the maximum is
-    // the best H at its first column (columns and H stay below 2^16 here).
-    uint32_t key0 = 0, key1 = 0;
-    const int2 *rin = ring + ((s + PAIR_WAVES - 1) % PAIR_WAVES) * Y.ring_len;
-    int2 *rout = ring + (s % PAIR_WAVES) * Y.ring_len;
-    int32_t *pin = sy + SY_PROG + (s + PAIR_WAVES - 1) % PAIR_WAVES, *pout = sy + SY_PROG + s % PAIR_WAVES;
-    const bool wr = s + 1 < S;
-    uint32_t *pl = (uint32_t *)(planes + (size_t)s * T * 64) + lane;  // [t / 4][lane] dwords, byte t % 4
-    // the column code of step 0 (lane 0: column 0; the others idle) and its
-    // scores; later steps read theirs one step ahead
-    int code = wave_shr1(bcode[0], PAIR_PAD);
-    int s0n = t0[code], s1n = t1[code];
-    uint32_t pk = 0;  // plane bytes of the current 4 steps
-    for (int tb = 0; tb < T; tb += 8) {
-      int topH[8], topF[8];
-      if (s == 0) {
+    const int r0 = (s * 64 + lane) * PR;
+    const uint8_t *line[PR];
 #pragma unroll
-        for (int q = 0; q < 8; ++q) {
-          topH[q] = LOCAL ? 0 : open + (tb + q) * ext;  // H(0, tb + q + 1)
-          topF[q] = NEG32;
-        }
-      } else {
-        // ring columns [tb, tb + 8) of the strip above: wait for them (bounded)
-        const int need = (s << 20) | (tb + 8 < n ? tb + 8 : n);
-        int spins = 0;
-        while (__hip_atomic_load(pin, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < need) {
-          if (++spins > A.spin_limit) {
-            if (lane == 0) atomicOr(&sy[SY_STATUS], PAIR_GAVE_UP);
-            break;
-          }
-          __builtin_amdgcn_s_sleep(1);
-        }
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-          const int2 v = rin[tb + q < n ? tb + q : n - 1];
-          topH[q] = v.x;
-          topF[q] = v.y;
-        }
-      }
-      const uint2 bw0 = *(const uint2 *)(bcode + tb), bw1 = *(const uint2 *)(bcode + tb + 8);
-      const uint32_t bw[4] = {bw0.x, bw0.y, bw1.x, bw1.y};
-      // The 8 steps, in two forms: with the per-lane column test, and without
-      // it where every lane is inside the columns (most blocks).
-      auto steps = [&](auto full_tag) {
-        constexpr bool FULL = decltype(full_tag)::value;
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-          const int t = tb + q;
-          const int S0 = s0n, S1 = s1n;
-          // the next step's column code (lane l takes lane l-1's) and scores
-          const int bnext = (int)((bw[(q + 1) >> 2] >> (8 * ((q + 1) & 3))) & 0xff);
-          const int cnext = wave_shr1(bnext, code);
-          s0n = t0[cnext];
-          s1n = t1[cnext];
-          code = cnext;
-          const int Hup = wave_shr1(topH[q], Hbot), Fup = wave_shr1(topF[q], Fbot);
-          const int c0 = t - lane;  // 0-based column of this lane at this step
-          if (FULL || (c0 >= 0 && c0 < n)) {
-            // Direction bits are sign bits of differences (|values| < 2^30),
-            // pushed into acc: e0 f0 d0 x0 e1 f1 d1 x1 from bit 0 up.  x (F
-            // above E) is kept only where d (H not from the diagonal) is set,
-            // so that d = 0, x = 1 marks a local stop cell (H = 0), whose
-            // other bits no walk reads.
-            uint32_t acc = 0;
-            // row r0 + 1 (1-based)
-            const int HdS0 = hd + S0;
-            const int Eo0 = H0 + open, Ee0 = E0 + ext, En0 = max(Eo0, Ee0);
-            const int Fo0 = Hup + open, Fe0 = Fup + ext, Fn0 = max(Fo0, Fe0);
-            int Hn0 = max(HdS0, max(En0, Fn0));
-            if (LOCAL) Hn0 = max(Hn0, 0);
-            // row r0 + 2: the row above is the one just computed
-            const int HdS1 = H0 + S1;
-            const int Eo1 = H1 + open, Ee1 = E1 + ext, En1 = max(Eo1, Ee1);
-            const int Fo1 = Hn0 + open, Fe1 = Fn0 + ext, Fn1 = max(Fo1, Fe1);
-            int Hn1 = max(HdS1, max(En1, Fn1));
-            if (LOCAL) Hn1 = max(Hn1, 0);
-            const uint32_t dD0 = (uint32_t)(HdS0 - Hn0), dD1 = (uint32_t)(HdS1 - Hn1);
-            uint32_t xd0 = (uint32_t)(En0 - Fn0) & dD0, xd1 = (uint32_t)(En1 - Fn1) & dD1;
-            uint32_t dd0 = dD0, dd1 = dD1;
-            if (LOCAL) {  // H >= 0: H = 0 sets x and clears d
-              xd0 |= (uint32_t)(Hn0 - 1); xd1 |= (uint32_t)(Hn1 - 1);
-              dd0 &= (uint32_t)(-Hn0); dd1 &= (uint32_t)(-Hn1);
-              key0 = max(key0, ((uint32_t)Hn0 << 16) | (uint32_t)(0xFFFF - c0));
-              key1 = max(key1, ((uint32_t)Hn1 << 16) | (uint32_t)(0xFFFF - c0));
-            }
-            acc = __builtin_amdgcn_alignbit(acc, xd1, 31);
-            acc = __builtin_amdgcn_alignbit(acc, dd1, 31);
-            acc = __builtin_amdgcn_alignbit(acc, (uint32_t)(Fo1 - Fe1), 31);
-            acc = __builtin_amdgcn_alignbit(acc, (uint32_t)(Eo1 - Ee1), 31);
-            acc = __builtin_amdgcn_alignbit(acc, xd0, 31);
-            acc = __builtin_amdgcn_alignbit(acc, dd0, 31);
-            acc = __builtin_amdgcn_alignbit(acc, (uint32_t)(Fo0 - Fe0), 31);
-            acc = __builtin_amdgcn_alignbit(acc, (uint32_t)(Eo0 - Ee0), 31);
-            pk = (pk & ~(0xffu << (8 * (q & 3)))) | ((acc & 0xffu) << (8 * (q & 3)));
-            if (wr && lane == 63) rout[c0] = make_int2(Hn1, Fn1);
-            hd = Hup;
-            H0 = Hn0; H1 = Hn1; E0 = En0; E1 = En1;
-            Hbot = Hn1; Fbot = Fn1;
-          }
-          if ((q & 3) == 3) pl[(size_t)(t >> 2) * 64] = pk;
-        }
-      };
-      if (tb >= 63 && tb + 8 <= n) steps(std::true_type{});
-      else steps(std::false_type{});
-      if (wr) {
-        int done = tb + 8 - 63;  // lane 63 has stored columns 0 .. tb + 7 - 63
-        done = done < 0 ? 0 : (done > n ? n : done);
-        if (lane == 63)
-          __hip_atomic_store(pout, ((s + 1) << 20) | done, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-      }
-    }
-    if (LOCAL) {
-      const int rb0 = (int)(key0 >> 16), rc0 = 0x10000 - (int)(key0 & 0xffff);  // 1-based column
-      const int rb1 = (int)(key1 >> 16), rc1 = 0x10000 - (int)(key1 & 0xffff);
-      if (r0 < m && rb0 > 0 && better(rb0, r0 + 1, rc0, bh, bi, bj)) { bh = rb0; bi = r0 + 1; bj = rc0; }
-      if (r0 + 1 < m && rb1 > 0 && better(rb1, r0 + 2, rc1, bh, bi, bj)) { bh = rb1; bi = r0 + 2; bj = rc1; }
+    for (int k = 0; k < PR; ++k) line[k] = tab + 32 * (r0 + k < m ? acode[r0 + k] : PAIR_PAD_LINE);
+    strip_slot<PR>(lds + slot, line, K, LOCAL ? 0 : -A.open - A.ext, LOCAL ? PAD_SCORE : A.ext - A.open);
+    PairIO<PR, GP> io;
+    io.bcode = bcode + 64 - lane;
+    io.slot_add = 0x01010101u * ((uint32_t)((uint32_t)(uintptr_t)(lds_u8 *)lds + slot) >> 8);
+    io.status = sy + SY_STATUS;
+    io.pin = sy + (s ? SY_PROG + (s + PAIR_WAVES - 1) % PAIR_WAVES : SY_READY);
+    io.pout = sy + SY_PROG + s % PAIR_WAVES;
+    io.rin = lane ? (int2 *)(sy + SY_ZERO)
+                  : s ? ring + ((s + PAIR_WAVES - 1) % PAIR_WAVES) * Y.ring_len + 64 : (int2 *)(sy + SY_EDGE);
+    io.rin_step = lane == 0 && s ? 8 : 0;
+    io.rout = ring + (s % PAIR_WAVES) * Y.ring_len;
+    io.need0 = s << 20;
+    io.cols = T - 63;
+    io.s = s;
+    io.spin_limit = A.spin_limit;
+    if constexpr (GP) {
+      io.pl = (uint32_t *)A.planes + (size_t)s * (T / SPD) * 64 + lane;
+      io.pl_step = 64;
     } else {
-      if (r0 + 1 == m) sy[SY_SCORE] = H0;
-      if (r0 + 2 == m) sy[SY_SCORE] = H1;
+      const bool own = s + 1 < S || lane < last_lanes;
+      io.pl = own ? (uint32_t *)(lds + Y.planes) + s * (T / SPD) * 64 + lane : (uint32_t *)sy + SY_DUMP;
+      io.pl_step = !own ? 0 : s + 1 < S ? 64 : last_lanes;
     }
+    strip_sweep<PR, LOCAL>(io, s, s + 1 == S, m, n, T, A.open, A.ext, end);
   }
   if (LOCAL) {
 #pragma unroll
     for (int w = 32; w >= 1; w >>= 1) {
-      const int oh = __shfl_xor(bh, w, 64), oi = __shfl_xor(bi, w, 64), oj = __shfl_xor(bj, w, 64);
-      if (better(oh, oi, oj, bh, bi, bj)) { bh = oh; bi = oi; bj = oj; }
+      const int oh = __shfl_xor(end.h, w, 64), oi = __shfl_xor(end.i, w, 64), oj = __shfl_xor(end.j, w, 64);
+      if (strip_better(oh, oi, oj, end.h, end.i, end.j)) { end.h = oh; end.i = oi; end.j = oj; }
     }
     if (lane == 0) {
-      sy[SY_BEST + 3 * wv] = bh; sy[SY_BEST + 3 * wv + 1] = bi; sy[SY_BEST + 3 * wv + 2] = bj;
+      sy[SY_BEST + 3 * wv] = end.h; sy[SY_BEST + 3 * wv + 1] = end.i; sy[SY_BEST + 3 * wv + 2] = end.j;
     }
+  } else if (end.has) {
+    sy[SY_SCORE] = end.h;
   }
-  __syncthreads();
+  __syncthreads();  // (GP: and every plane store of the workgroup is visible to it)
   if (wv != 0) return;
 
   // ---- end cell and walk (wave 0)
@@ -265,10 +329,10 @@ __global__ __launch_bounds__(64 * PAIR_WAVES) void pair_kernel(PairArgs A) {
   r.flags = TA_F_I32;
   int i = m, j = n;
   if (LOCAL) {
-    bh = 0; bi = 0x7fffffff; bj = 0x7fffffff;
-    for (int w = 0; w < PAIR_WAVES; ++w) {
+    int bh = 0, bi = 0x7fffffff, bj = 0x7fffffff;
+    for (int w = 0; w < PAIR_WAVES && w < S; ++w) {
       const int oh = sy[SY_BEST + 3 * w], oi = sy[SY_BEST + 3 * w + 1], oj = sy[SY_BEST + 3 * w + 2];
-      if (oh > 0 && better(oh, oi, oj, bh, bi, bj)) { bh = oh; bi = oi; bj = oj; }
+      if (oh > 0 && strip_better(oh, oi, oj, bh, bi, bj)) { bh = oh; bi = oi; bj = oj; }
     }
     r.score = bh;
     if (bh <= 0) {
@@ -277,72 +341,43 @@ __global__ __launch_bounds__(64 * PAIR_WAVES) void pair_kernel(PairArgs A) {
       r.flags |= TA_F_EMPTY;
       i = j = 0;
     } else {
-      i = bi; j = bj;
-      r.a_end = bi - 1; r.b_end = bj - 1;
+      i = __builtin_amdgcn_readfirstlane(bi);
+      j = __builtin_amdgcn_readfirstlane(bj);
+      r.a_end = i - 1; r.b_end = j - 1;
     }
   } else {
     r.score = sy[SY_SCORE];
     r.a_begin = 0; r.a_end = m - 1; r.b_begin = 0; r.b_end = n - 1;
   }
   const bool walk = LOCAL ? r.score > 0 : A.traceback != 0;
+  uint32_t *runs = (uint32_t *)(lds + Y.runs);  // over the slots, which only the fill read
   const int cap = Y.runs_cap;
-  int wp = cap, op = -1, len = 0, state = 0, steps = 0;
-  bool fail = false, stop = false;
-  auto flush = [&]() {
-    if (len) {
-      --wp;
-      runs[wp] = ((uint32_t)len << 2) | (uint32_t)op;  // every lane stores the same word
+  WaveRuns rw;
+  rw.end = runs + cap;
+  rw.cap = cap;
+  if (walk) {
+    constexpr int KIND = LOCAL ? WALK_MARKED : WALK_GLOBAL;
+    int state = 0, h = 0, steps = 0, how;
+    if constexpr (GP) {
+      StripWindow<PR> src{(const uint32_t *)A.planes, (uint32_t *)(lds + Y.window), T, -1, -1};
+      src.refill(i, j);
+      how = wave_walk<KIND>(src, rw, i, j, state, h, A.open, A.ext, A.walk_cap, steps);
+    } else {
+      PairCodes<PR> src{(const uint32_t *)(lds + Y.planes), (uint32_t)(T / SPD) * 64, (uint32_t)S - 1,
+                        (uint32_t)last_lanes};
+      how = wave_walk<KIND>(src, rw, i, j, state, h, A.open, A.ext, A.walk_cap, steps);
     }
-  };
-  auto emit = [&](int o, int k) {
-    if (o != op) { flush(); op = o; len = 0; }
-    len += k;
-  };
-  while (walk && !stop && !fail && i > 0 && j > 0) {
-    // the 16 x 16 cells above-left of (i, j): lane q holds row pairs rp0 - (q >> 4) (- 4 in v1),
-    // column j - 1 - (q & 15) (0-based), one code byte (both rows of the pair)
-    const int rp0 = (i - 1) >> 1, cw0 = j - 1;
-    int v[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int rp = rp0 - (lane >> 4) - 4 * h, cj = cw0 - (lane & 15);
-      int byte = 0;
-      if (rp >= 0 && cj >= 0) {
-        const int ss = rp >> 6, ll = rp & 63;
-        const int t = cj + ll;
-        byte = planes[((size_t)ss * T + (t & ~3)) * 64 + 4 * ll + (t & 3)];
-      }
-      v[h] = byte;
+    if (how == WALK_GAVE_UP) {
+      r.flags |= TA_F_WALK_FAILED;
+    } else if (!LOCAL) {
+      if (i == 0 && j > 0) rw.emit(1, j);
+      if (j == 0 && i > 0) rw.emit(2, i);
+      i = j = 0;
     }
-    // Steps inside the window, all on wave-uniform (scalar) values: the
-    // code by readlane, the transition by selects.
-    for (;;) {
-      const int dyp = rp0 - ((i - 1) >> 1), dx = cw0 - (j - 1);
-      if (i == 0 || j == 0 || dyp > 7 || dx > 15) break;
-      const int lo = __builtin_amdgcn_readlane(v[0], ((dyp & 3) << 4) | dx);
-      const int hi = __builtin_amdgcn_readlane(v[1], ((dyp & 3) << 4) | dx);
-      const int cd = ((dyp < 4 ? lo : hi) >> (((i - 1) & 1) << 2)) & 15;
-      if (LOCAL && state == 0 && (cd & 12) == 8) { stop = true; break; }  // entered a cell whose H is 0
-      const int src = ((cd >> 2) & 1) * (1 + ((cd >> 3) & 1));  // H-source: 0 diag, 1 E, 2 F
-      const int g = state ? state : src;
-      const int xb = g ? (cd >> (g - 1)) & 1 : 0;              // E: bit 0, F: bit 1 (extend)
-      if (g != op) { flush(); op = g; len = 0; }
-      ++len;
-      state = xb ? g : 0;
-      j -= g != 2;
-      i -= g != 1;
-      if (++steps > A.walk_cap) { fail = true; break; }
-    }
+    if (!rw.finish()) r.flags |= TA_F_WALK_FAILED;
   }
-  if (walk && !fail && !LOCAL) {
-    if (i == 0 && j > 0) emit(1, j);
-    if (j == 0 && i > 0) emit(2, i);
-    i = j = 0;
-  }
-  if (walk) flush();
   if (LOCAL && r.score > 0) { r.a_begin = i; r.b_begin = j; }
-  if (fail) r.flags |= TA_F_WALK_FAILED;
-  const int nr = cap - wp;
+  const int nr = rw.n < cap ? rw.n : cap, wp = cap - nr;
   uint32_t *dst = (uint32_t *)(A.out + 1);
   if (A.traceback)
     for (int q = lane; q < nr; q += 64) dst[q] = runs[wp + q];
@@ -355,32 +390,59 @@ __global__ __launch_bounds__(64 * PAIR_WAVES) void pair_kernel(PairArgs A) {
   }
 }
 
+template <int PR>
+void launch_rows(const PairArgs &A, hipStream_t st) {
+  void (*k)(PairArgs) = A.local ? (A.lay.plane_bytes ? pair_kernel<PR, true, true> : pair_kernel<PR, true, false>)
+                                : (A.lay.plane_bytes ? pair_kernel<PR, false, true> : pair_kernel<PR, false, false>);
+  hipLaunchKernelGGL(k, dim3(1), dim3(64 * std::min(PAIR_WAVES, A.lay.S)), A.lay.bytes, st, A);
+}
+
 }  // namespace
 
-PairLayout pair_layout(int m, int n) {
+PairLayout pair_layout(int m, int n, int K, int lds_max) {
   PairLayout L{};
-  auto up16 = [](long x) { return (int)((x + 15) & ~15L); };
+  auto up = [](long x, int to) { return (x + to - 1) / to * to; };
+  // Rows per lane.  A strip's step takes about 16 instructions and 13 more
+  // per row, and every wave is one SIMD's: the fewest rows that give each of
+  // the four waves at most one strip.
+  L.R = m <= 64 * PAIR_WAVES ? 1 : m <= 128 * PAIR_WAVES ? 2 : 4;
   L.T = (n + 63 + 7) & ~7;
-  L.S = (m + PAIR_STRIP - 1) / PAIR_STRIP;
-  L.ring_len = n + 8;
+  L.S = (m + 64 * L.R - 1) / (64 * L.R);
+  const int waves = std::min(PAIR_WAVES, L.S);
+  L.ring_len = L.T + 80;
   L.runs_cap = m + n + 2;
   long off = 1280;
-  L.acode = (int)off; off += up16(m);
-  L.bcode = (int)off; off += up16(L.T + 8);
   L.sync = (int)off; off += 4 * SY_WORDS;
-  L.ring = (int)off; off += (long)PAIR_WAVES * L.ring_len * 8;
-  L.planes = (int)off; off += (long)L.S * L.T * 64;
-  L.runs = (int)off; off += 4L * L.runs_cap;
-  L.bytes = off > (1L << 30) ? (1 << 30) : (int)off;
+  L.slots = (int)off;  // in the first 64 KB (strip.h addresses a slot's rows in one byte)
+  static_assert((1280 + 4 * SY_WORDS) % STRIP_ROW == 0 &&
+                1280 + 4 * SY_WORDS + PAIR_WAVES * strip_slot_bytes(4) <= 256 * STRIP_ROW, "slot rows");
+  const int rows = (int)up(K + 1, 4);
+  L.slot_bytes = (L.R == 4 ? STRIP_NC + rows : rows) * STRIP_ROW;
+  off += (long)waves * L.slot_bytes;
+  L.acode = (int)off; off += up(m, 16);
+  L.bcode = (int)off; off += up(64 + L.T + 32, 16);
+  L.ring = (int)off; off += (long)std::min(PAIR_WAVES, L.S - 1) * L.ring_len * 8;
+  // after the fill: the CIGAR runs and, with the codes in device memory, the walk's window
+  L.runs = L.slots;
+  L.window = (int)(L.slots + up(4L * L.runs_cap, 16));
+  const long spd = strip_spd(L.R), after = L.window + 32 * (32 / spd + 1) * 4, strips = (long)L.T / spd * 4;
+  const long last = (m - (long)(L.S - 1) * 64 * L.R + L.R - 1) / L.R;
+  L.planes = (int)std::max(off, (long)L.window);
+  const long with = L.planes + strips * ((L.S - 1) * 64L + last);
+  if (with <= lds_max) {
+    L.bytes = (int)with;
+  } else {
+    L.bytes = (int)std::min(std::max(off, after), 1L << 30);
+    L.plane_bytes = (int)std::min(strips * 64 * L.S, 1L << 30);
+  }
   return L;
 }
 
 int pair_launch(const PairArgs &A, hipStream_t st) {
   (void)hipGetLastError();
-  if (A.local)
-    hipLaunchKernelGGL(pair_kernel<true>, dim3(1), dim3(64 * PAIR_WAVES), A.lay.bytes, st, A);
-  else
-    hipLaunchKernelGGL(pair_kernel<false>, dim3(1), dim3(64 * PAIR_WAVES), A.lay.bytes, st, A);
+  if (A.lay.R == 1) launch_rows<1>(A, st);
+  else if (A.lay.R == 2) launch_rows<2>(A, st);
+  else launch_rows<4>(A, st);
   return hipGetLastError() == hipSuccess ? TA_OK : TA_E_DEVICE;
 }
 
@@ -417,8 +479,17 @@ int pair_finish(const PairOut &o, const uint32_t *runs, const ta_params *p, ta_r
   return (r.flags & TA_F_WALK_FAILED) ? TA_E_WALK : TA_OK;
 }
 
-// The pair path takes pairs whose codes fit in LDS; others (and empty
-// sides, and forced long-pair lanes) go through the batch path.
+// The pair path takes pairs whose codes take about a CU's LDS at most (codes
+// that do not fit beside the fill's tables go to device memory); others (and
+// empty sides, and forced long-pair lanes) go through the batch path.  Which
+// pairs these are shows in their results (TA_F_I32), so the bound is a fixed
+// function of the lengths.
+bool pair_fits(int32_t m, int32_t n, int64_t lds_max) {
+  const int64_t T = (n + 63 + 7) & ~7, S = ((int64_t)m + 127) / 128;
+  auto up16 = [](int64_t x) { return (x + 15) & ~15ll; };
+  return 1536 + up16(m) + up16(T + 8) + 32 * ((int64_t)n + 8) + S * T * 64 + 4 * ((int64_t)m + n + 2) <= lds_max;
+}
+
 bool pair_path(const ta_ctx *ctx, const ta_params *p, int32_t la, int32_t lb) {
   if (la <= 0 || lb <= 0 || p->lanes == TA_LANES_LONG) return false;
   if (p->mode == TA_GLOBAL && (int64_t)(la + lb + 2) * -p->gap_extend + 2 * (int64_t)-p->gap_open >= (1ll << 28))
@@ -427,10 +498,10 @@ bool pair_path(const ta_ctx *ctx, const ta_params *p, int32_t la, int32_t lb) {
     const int maxS = p->alphabet == TA_PROTEIN ? 11 : std::max(0, std::max(p->match, p->mismatch));
     if ((int64_t)std::min(la, lb) * maxS >= 65535) return false;
   }
-  return pair_layout(la, lb).bytes <= ctx->lds_max;
+  return pair_fits(la, lb, ctx->lds_max);
 }
 
-PairArgs pair_args(const ta_params *p, int32_t la, int32_t lb) {
+PairArgs pair_args(const ta_ctx *ctx, const ta_params *p, int32_t la, int32_t lb) {
   PairArgs A{};
   A.m = la; A.n = lb;
   A.alphabet = p->alphabet; A.match = p->match; A.mismatch = p->mismatch;
@@ -439,9 +510,13 @@ PairArgs pair_args(const ta_params *p, int32_t la, int32_t lb) {
   A.spin_limit = 1 << 22;
   A.walk_cap = la + lb;  // a walk takes at most la + lb steps
   if (const char *e = getenv("TWEAKALIGN_WALK_GUARD")) A.walk_cap = std::min(A.walk_cap, std::max(0, atoi(e)));
-  A.lay = pair_layout(la, lb);
+  A.lay = pair_layout(la, lb, p->alphabet == TA_PROTEIN ? TA_PROT_K : 4, ctx->lds_max);
   return A;
 }
+
+// Device memory for the codes of a pair that fits: at most the codes' 4 bits
+// a cell over whole strips and steps, some 200 KB.
+constexpr size_t kPairPlanes = 256 << 10;
 
 }  // namespace
 
@@ -454,7 +529,11 @@ int ta_align_pair(ta_ctx *ctx, const ta_params *p, const char *a, int32_t la, co
     return ta_align_batch(ctx, p, &q, 1, out, cigar_buf, cap, used);
   }
   if (hipSetDevice(ctx->device) != hipSuccess) return TA_E_DEVICE;
-  PairArgs A = pair_args(p, la, lb);
+  PairArgs A = pair_args(ctx, p, la, lb);
+  if (A.lay.plane_bytes) {
+    if (!ctx->pair_planes && !(ctx->pair_planes = device_alloc(kPairPlanes))) return TA_E_NOMEM;
+    A.planes = (uint8_t *)ctx->pair_planes;
+  }
   // staging: [PairOut][runs][a][b]
   const size_t o_runs = sizeof(PairOut), o_a = (o_runs + 4 * (size_t)A.lay.runs_cap + 15) & ~(size_t)15;
   const size_t o_b = (o_a + (size_t)la + 15) & ~(size_t)15, need = o_b + (size_t)lb + 16;
@@ -492,15 +571,17 @@ int ta_align_pair(ta_ctx *ctx, const ta_params *p, const char *a, int32_t la, co
 namespace {
 
 static __device__ __align__(256) uint8_t scratch[TA_PAIR_STATIC_SCRATCH];
+static __device__ __align__(256) uint8_t scratch_planes[kPairPlanes];
 
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
-uint8_t *g_scratch[kMaxDevices] = {};
+uint8_t *g_scratch[kMaxDevices] = {}, *g_planes[kMaxDevices] = {};
 bool g_scratch_done[kMaxDevices] = {};
 
-uint8_t *scratch_of(int device) {
+uint8_t *scratch_of(int device, uint8_t **planes) {
   if (device < 0 || device >= kMaxDevices) return nullptr;
   std::lock_guard<std::mutex> g(g_scratch_mu);
+  *planes = g_planes[device];
   return g_scratch[device];
 }
 
@@ -552,14 +633,16 @@ void pair_scratch_setup(int device) {
   std::lock_guard<std::mutex> g(g_scratch_mu);
   if (g_scratch_done[device]) return;
   g_scratch_done[device] = true;
-  void *ptr = nullptr;
-  const hipError_t e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
+  void *ptr = nullptr, *pl = nullptr;
+  hipError_t e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
+  if (e == hipSuccess) e = hipGetSymbolAddress(&pl, HIP_SYMBOL(scratch_planes));
   if (e != hipSuccess) {
     (void)hipGetLastError();
     fprintf(stderr, "tweakalign: no address for the pair scratch on device %d: %s\n", device, hipGetErrorString(e));
     return;
   }
   g_scratch[device] = (uint8_t *)ptr;
+  g_planes[device] = (uint8_t *)pl;
 }
 
 int ta_align_pair_static(ta_ctx *ctx, const ta_params *p, const char *a, int32_t la, const char *b, int32_t lb,
@@ -569,7 +652,7 @@ int ta_align_pair_static(ta_ctx *ctx, const ta_params *p, const char *a, int32_t
   if ((int64_t)la + lb > TA_PAIR_STATIC_MAX) return TA_E_LIMIT;
   if (la == 0 || lb == 0) return empty_side(p, la, lb, out, cigar_buf, cap, used);
   if (!pair_path(ctx, p, la, lb)) return TA_E_LIMIT;
-  uint8_t *scr = scratch_of(ctx->device);
+  uint8_t *planes = nullptr, *scr = scratch_of(ctx->device, &planes);
   if (!scr) return TA_E_DEVICE;
   if (hipSetDevice(ctx->device) != hipSuccess) return TA_E_DEVICE;
   const StaticLayout L = static_layout(la, lb);
@@ -577,9 +660,10 @@ int ta_align_pair_static(ta_ctx *ctx, const ta_params *p, const char *a, int32_t
   if (hipMemcpyAsync(scr + L.a, a, (size_t)la, hipMemcpyHostToDevice, st) != hipSuccess ||
       hipMemcpyAsync(scr + L.b, b, (size_t)lb, hipMemcpyHostToDevice, st) != hipSuccess)
     return TA_E_DEVICE;
-  PairArgs A = pair_args(p, la, lb);
+  PairArgs A = pair_args(ctx, p, la, lb);
   A.a = (const char *)(scr + L.a);
   A.b = (const char *)(scr + L.b);
+  A.planes = planes;
   A.out = (PairOut *)scr;  // the kernel writes every field the host reads (status included)
   int rc = pair_launch(A, st);
   if (rc) return rc;

@@ -457,6 +457,7 @@ void ta_destroy(ta_ctx *c) {
   (void)hipSetDevice(c->device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   if (c->pair_stage) (void)hipHostFree(c->pair_stage);
+  device_free(c->pair_planes);
   c->seq_arena.reset();  // freed here unless a batch still holds it (none after serve_shutdown)
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;

@@ -33,6 +33,7 @@ struct ta_ctx {
   // ta_destroy.
   void *pair_stage = nullptr;
   size_t pair_stage_cap = 0;
+  void *pair_planes = nullptr;  // ta_align_pair: direction codes of pairs whose codes do not fit in LDS
   // Resident sequences (ta_seq_add): residue codes in one device arena, each
   // sequence 16-byte aligned and padded with code 0, 32 bytes of slack after
   // the last (the walkers' windows); per sequence its offset, length,
