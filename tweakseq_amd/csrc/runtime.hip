@@ -24,6 +24,7 @@
 #include "fill.h"
 #include "long.h"
 #include "runtime_internal.h"
+#include "strips.h"
 #include "traceback.h"
 
 using namespace ta;
@@ -896,6 +897,18 @@ struct ta_batch {
   // Most steps a traceback walk may take (TWEAKALIGN_WALK_GUARD lowers it so
   // that walks end flagged; otherwise above every walk's length).
   int32_t guard_cap = INT32_MAX;
+  // Batches of few pairs (strips.h).
+  bool strips = false;
+  int strips_bcode = 0;
+  std::vector<StripPair> spairs;
+  std::vector<StripItem> sitems;
+  StripPair *d_spairs = nullptr;
+  StripItem *d_sitems = nullptr;
+  int2 *d_sring = nullptr;
+  uint32_t *d_splanes = nullptr;
+  uint64_t *d_sbest = nullptr;
+  int32_t *d_sscore = nullptr;
+  uint64_t sring_n = 0, splanes_n = 0;
   // captured run
   bool graph_on = false, phases_timed = false;
   hipGraph_t graph = nullptr;
@@ -963,6 +976,8 @@ void ta_batch_destroy(ta_batch *B) {
   free_rerun(B);
   dfree(B->d_lp); dfree(B->d_litems); dfree(B->d_lring); dfree(B->d_lck); dfree(B->d_lcol); dfree(B->d_lprog);
   dfree(B->d_wring); dfree(B->d_wtb);
+  dfree(B->d_spairs); dfree(B->d_sitems); dfree(B->d_sring); dfree(B->d_splanes); dfree(B->d_sbest);
+  dfree(B->d_sscore);
   dfree(B->d_plain_tasks); dfree(B->d_prow); dfree(B->d_pcol); dfree(B->d_pring);
   dfree(B->d_ptbuf); dfree(B->d_pptb); dfree(B->d_plain_rtasks); dfree(B->d_pptb_r);
   for (auto &e : B->ev)
@@ -987,6 +1002,71 @@ static bool pair_ok(const ta_params &p, const ta_pair &q) {
   if (q.la < 0 || q.lb < 0 || q.la > 1000000 || q.lb > 1000000 || (q.la && !q.a) || (q.lb && !q.b)) return false;
   return p.mode == TA_LOCAL ||
          (int64_t)(q.la + q.lb + 2) * -p.gap_extend + 2 * (int64_t)-p.gap_open < (1ll << 28);
+}
+
+// Whether a batch's pairs all go strip by strip over the whole GPU (strips.h),
+// and their items.  Its steps are int32 and single pairs, about twice the
+// instructions per cell of the packed fill, and buy a run as long as the
+// longest pair's pipeline instead of its sweep by one or four waves.  Both
+// sides measured on related protein pairs, lengths up to L (half of it at
+// least), from run to results in place, us, task form / strips:
+//   strips per SIMD   global                           local
+//     0.9 (L 1200)    1,482 / 341                      1,635 / 393
+//     3.5 (L 600)       811 / 333                        890 / 423
+//     7   (L 1200)    2,552 / 793                      1,899 / 1,095
+//     9   (L 400)       862 / 439                        947 / 590
+//    19   (L 200)       486 / 570                        521 / 738
+// so batches of up to 8 strips per SIMD take it, except very short pairs,
+// whose whole run is launches: a pair costs it 18 ns, and three launches and
+// a status copy 25 us, which a longest pair of la + lb = 60 + pairs / 24 gains
+// back (L 30: 2 pairs 72 / 73, 2,048 95 / 117; L 120: 4,096 218 / 185,
+// 8,192 219 / 245).
+static void plan_strips(ta_ctx *ctx, ta_batch *B) {
+  if (!B->trace || getenv("TWEAKALIGN_COOP") || getenv("TWEAKALIGN_WALK_IN_FILL")) return;
+  const bool local = B->p.mode == TA_LOCAL;
+  int64_t strips = 0;
+  int max_t = 0, longest = 0;
+  std::vector<int32_t> ks;
+  for (int32_t k = 0; k < B->n; ++k) {
+    const HostPair &h = B->hp[k];
+    if (h.path != 1 && h.path != 2) continue;
+    if (h.lb > STRIPS_MAXN) return;
+    // local H and its bound in the end-cell keys
+    if (local && (int64_t)std::min(h.la, h.lb) * std::max(0, B->alph.maxS) >= 65400) return;
+    ks.push_back(k);
+    strips += ceil_div(h.la, 64 * STRIPS_PR);
+    max_t = std::max(max_t, (h.lb + 63 + 7) & ~7);
+    longest = std::max(longest, h.la + h.lb);
+    if (strips > (int64_t)ctx->cus * 4 * STRIPS_PER_SIMD) return;
+  }
+  if (ks.empty() || longest < 60 + (int)(ks.size() / 24) || strips_lds(max_t + 96) > ctx->lds_max) return;
+  B->strips = true;
+  B->strips_bcode = max_t + 96;
+  B->may_saturate = false;
+  // longest pipelines first
+  std::vector<uint64_t> key(ks.size());
+  for (size_t t = 0; t < ks.size(); ++t) {
+    const HostPair &h = B->hp[ks[t]];
+    key[t] = (1ull << 32) - (uint64_t)h.lb - 100ull * ceil_div(h.la, 64 * STRIPS_PR);
+  }
+  gather_by_key(ks, std::move(key));
+  B->spairs.reserve(ks.size());
+  B->sitems.reserve((size_t)strips);
+  for (int32_t k : ks) {
+    const HostPair &h = B->hp[k];
+    StripPair P{};
+    P.a_off = h.a_off; P.b_off = h.b_off;
+    P.pid = k; P.m = h.la; P.n = h.lb;
+    P.S = ceil_div(h.la, 64 * STRIPS_PR);
+    P.T = (h.lb + 63 + 7) & ~7;
+    P.i16 = h.path == 2;
+    P.ring = B->sring_n;
+    B->sring_n += (uint64_t)(P.S - 1) * (P.T + 8);
+    P.planes = B->splanes_n;
+    B->splanes_n += (uint64_t)P.S * (P.T / strip_spd(STRIPS_PR)) * 64;
+    for (int s = 0; s < P.S; ++s) B->sitems.push_back(StripItem{(int32_t)B->spairs.size(), s});
+    B->spairs.push_back(P);
+  }
 }
 
 int ta_batch_create(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32_t n, ta_batch **out) {
@@ -1282,6 +1362,7 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
   }
 
   tr.mark("pairs");
+  plan_strips(ctx, B);
   // Couples: local pairs pad to the longer column count; global couples
   // need equal column counts (so H(m, n) of both sits in the last column).
   Plan &pl = B->plan;
@@ -1294,7 +1375,7 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
   pl.ptb.assign(n, PairTB{0, 0, 0, 0, 0, 0, 0});
   pl.cjobs.reserve((size_t)n / 2 + NGW);
   std::vector<int> i16, i32;
-  for (int32_t k = 0; k < n; ++k) {
+  for (int32_t k = 0; k < n && !B->strips; ++k) {
     if (B->hp[k].path == 2) i16.push_back(k);
     else if (B->hp[k].path == 1) i32.push_back(k);
   }
@@ -1470,15 +1551,17 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
     for (int32_t k = 0; k < n; ++k) key[k] = 2000000 - (uint64_t)(B->hp[k].la + B->hp[k].lb);
     order = order_by_key(std::move(key));
     up.add(&B->d_order, order);
-    if (B->walk) {  // pairs without a fill task: empty and long pairs
+    if (B->walk || B->strips) {  // pairs without a fill task: empty and long pairs
       for (int32_t k : order)
-        if (pl.ptb[k].P != 1 && pl.ptb[k].P != 2) rest.push_back(k);
+        if (B->strips ? B->hp[k].path == 0 : pl.ptb[k].P != 1 && pl.ptb[k].P != 2) rest.push_back(k);
       B->n_rest = (int32_t)rest.size();
       up.add(&B->d_order_rest, rest);
     }
   }
   up.add(&B->d_lp, B->longs);
   up.add(&B->d_litems, B->litems);
+  up.add(&B->d_spairs, B->spairs);
+  up.add(&B->d_sitems, B->sitems);
   rc = rc ? rc : up.commit(st);
   rc = rc ? rc : expand_jobs(d_jobs, pl.cjobs.size(), pl.rows_n, pl.cols_n, B->d_pairs, B->d_codes, B->Kp,
                              &B->d_rowcodes, &B->d_colcodes, st);
@@ -1494,6 +1577,10 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
   rc = rc ? rc : dalloc(&B->d_lck, B->lck_elems);
   rc = rc ? rc : dalloc(&B->d_lcol, B->lcol_elems);
   rc = rc ? rc : dalloc(&B->d_lprog, (size_t)B->lprog_n);
+  rc = rc ? rc : dalloc(&B->d_sring, B->sring_n);
+  rc = rc ? rc : dalloc(&B->d_splanes, B->splanes_n);
+  rc = rc ? rc : dalloc(&B->d_sbest, B->spairs.size());
+  rc = rc ? rc : dalloc(&B->d_sscore, B->spairs.size());
   rc = rc ? rc : dalloc(&B->d_wring, B->wring_stride * B->long_wgs);
   rc = rc ? rc : dalloc(&B->d_wtb, B->wtb_stride * B->long_wgs);
   for (auto &e : B->ev)
@@ -1540,10 +1627,11 @@ int ta_batch_info(ta_batch *B, int64_t *cells, int64_t *tb_bytes, int32_t *tasks
   if (!B) return TA_E_INVALID;
   if (cells) *cells = B->cells;
   if (tb_bytes)
-    *tb_bytes = (int64_t)(B->plan.tb_bytes + B->wtb_stride * B->long_wgs + 4 * B->lck_elems + 8 * B->lcol_elems);
+    *tb_bytes = (int64_t)(B->plan.tb_bytes + B->wtb_stride * B->long_wgs + 4 * B->lck_elems + 8 * B->lcol_elems +
+                          4 * B->splanes_n);
   if (tasks)
     *tasks = (int32_t)(B->plan.tasks2[0].size() + B->plan.tasks2[1].size() + B->plan.tasks2[2].size() +
-                       B->plan.tasks1[0].size() + B->plan.tasks1[1].size() + B->litems.size());
+                       B->plan.tasks1[0].size() + B->plan.tasks1[1].size() + B->litems.size() + B->sitems.size());
   return TA_OK;
 }
 
@@ -1680,6 +1768,50 @@ int launch_long_tb(ta_ctx *ctx, ta_batch *B, int lp0, int nlp, bool clear) {
   return TA_OK;
 }
 
+StripsArgs strips_args(ta_batch *B) {
+  StripsArgs a{};
+  a.sp = B->d_spairs; a.items = B->d_sitems;
+  a.nitems = (int)B->sitems.size(); a.npairs = (int)B->spairs.size();
+  a.ctr = B->d_ctr + 11;
+  a.table = B->d_table; a.Kp = B->Kp; a.codes = B->d_codes;
+  a.ring = B->d_sring; a.planes = B->d_splanes; a.best = B->d_sbest; a.score = B->d_sscore;
+  a.open = B->p.gap_open; a.ext = B->p.gap_extend;
+  a.sat_limit = 32767 - 2 * B->alph.maxS;
+  a.spin_limit = B->spin_limit;
+  a.err = B->d_ctr + 10;
+  a.tb = tb_args(B);
+  a.bcode_bytes = B->strips_bcode;
+  return a;
+}
+
+int launch_strips(ta_ctx *ctx, ta_batch *B) {
+  if (!B->strips) return TA_OK;
+  const StripsArgs a = strips_args(B);
+  const uint64_t n16 = B->sring_n / 2;
+  (void)hipGetLastError();
+  hipLaunchKernelGGL(strips_init_kernel, dim3((unsigned)std::max<uint64_t>(1, std::min<uint64_t>(4096, (n16 + 255) / 256))),
+                     dim3(256), 0, B->stream, (uint4 *)B->d_sring, n16, B->d_sbest, a.npairs);
+  const int lds = strips_lds(a.bcode_bytes);
+  const bool local = B->p.mode == TA_LOCAL;
+  void (*k)(StripsArgs) = local ? strips_kernel<true> : strips_kernel<false>;
+  // one wave per workgroup; those that do not fit at once take items as others end
+  const int per_cu = std::max(1, std::min(16, ctx->lds_max / lds));
+  hipLaunchKernelGGL(k, dim3(std::min(a.nitems, ctx->cus * per_cu)), dim3(64), lds, B->stream, a);
+  HIPCHK(hipGetLastError());
+  return TA_OK;
+}
+
+int launch_strips_walk(ta_batch *B) {
+  if (!B->strips) return TA_OK;
+  const StripsArgs a = strips_args(B);
+  const bool local = B->p.mode == TA_LOCAL;
+  void (*k)(StripsArgs) = local ? strips_walk_kernel<true> : strips_walk_kernel<false>;
+  (void)hipGetLastError();
+  hipLaunchKernelGGL(k, dim3(a.npairs), dim3(64), 0, B->stream, a);
+  HIPCHK(hipGetLastError());
+  return TA_OK;
+}
+
 // Pairs whose int16 pass saturated go through the int32 kernel.
 int rerun_saturated(ta_ctx *ctx, ta_batch *B) {
   std::vector<FillOut> fo(B->n);
@@ -1748,15 +1880,17 @@ int launch_fills(ta_ctx *ctx, ta_batch *B) {
                           B->walk);
   if (!rc) rc = launch_fill<1>(ctx, B, B->d_tasks1, n1, B->d_rowcodes, B->d_colcodes, B->d_ring, B->d_tb,
                                B->d_ctr + 2, 0, B->walk);
+  if (!rc) rc = launch_strips(ctx, B);
   if (!rc) rc = launch_long_fwd(ctx, B, 0, (int)B->litems.size(), false);
   return rc;
 }
 
 int launch_tracebacks(ta_ctx *ctx, ta_batch *B) {
   int rc = TA_OK;
-  if (!B->walk) {
+  if (B->strips) rc = launch_strips_walk(B);
+  if (!rc && !B->walk && !B->strips) {
     rc = launch_traceback(ctx, B, B->d_pairs, B->d_ptb, B->d_tb, 0, B->n);
-  } else if (B->n_rest) {  // the fill walked every pair it filled
+  } else if (!rc && B->n_rest) {  // every pair with a fill task is walked by now
     TbArgs a = tb_args(B);
     a.npairs = B->n_rest;
     a.order = B->d_order_rest;
@@ -1838,7 +1972,7 @@ int ta_batch_wait(ta_ctx *ctx, ta_batch *B) {
     if (hipEventElapsedTime(&t, B->ev[2], B->ev[3]) == hipSuccess) B->ms[2] = t;
   }
   if (hipEventElapsedTime(&t, B->ev[0], B->ev[3]) == hipSuccess) B->ms[3] = t;
-  if (!B->longs.empty() || B->ncoop2 || B->ncoop1) {
+  if (!B->longs.empty() || B->ncoop2 || B->ncoop1 || B->strips) {
     int32_t err = 0;
     HIPCHK(hipMemcpyAsync(&err, B->d_ctr + 10, sizeof(err), hipMemcpyDeviceToHost, B->stream));
     HIPCHK(hipStreamSynchronize(B->stream));

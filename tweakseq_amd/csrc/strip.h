@@ -396,4 +396,45 @@ __device__ __forceinline__ void strip_sweep(IO &io, int s, bool last, int m, int
   }
 }
 
+// Codes in device memory ([strip][t / SPD][64 lanes]): a window of them in
+// LDS, 32 lanes' rows up from the walk's cell, for each lane WD dwords
+// around the diagonal through it.
+template <int PR>
+struct StripWindow {
+  static constexpr int SPD = strip_spd(PR), WL = 32, WD = 32 / SPD + 1;
+  const uint32_t *pl;
+  uint32_t *win;  // WL x WD
+  int T;
+  int L0, u0;     // the window's first (lowest) lane, counted over all strips, and its 0-based column
+  // first staged dword of lane L0 - q
+  __device__ __forceinline__ int first(int q) const {
+    const int t = u0 - q * PR + ((L0 - q) & 63), d = t / SPD - WD / 2, top = T / SPD - WD;
+    return d > top ? (top < 0 ? 0 : top) : (d < 0 ? 0 : d);
+  }
+  __device__ __forceinline__ int code(int i, int j) const {
+    const int L = (int)((uint32_t)(i - 1) / PR), q = L0 - L, t = j - 1 + (L & 63);
+    const int d = (int)((uint32_t)t / SPD) - first(q);
+    if (q < 0 || q >= WL || d < 0 || d >= WD) return -1;
+    return strip_code<PR>(win[q * WD + d], (uint32_t)t % SPD, (uint32_t)(i - 1) % PR);
+  }
+  __device__ __forceinline__ bool refill(int i, int j) {
+    const bool moved = (i - 1) / PR != L0 || j - 1 != u0;
+    L0 = (i - 1) / PR;
+    u0 = j - 1;
+    constexpr int N = WL * WD, U = (N + 63) / 64;
+    uint32_t v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int x = u * 64 + (int)(threadIdx.x & 63), q = x / WD, d = first(q) + x % WD, L = L0 - q;
+      v[u] = x < N && L >= 0 && d < T / SPD ? pl[((size_t)(L >> 6) * (T / SPD) + d) * 64 + (L & 63)] : 0;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int x = u * 64 + (int)(threadIdx.x & 63);
+      if (x < N) win[x] = v[u];
+    }
+    return moved;
+  }
+};
+
 }  // namespace ta
