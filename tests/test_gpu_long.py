@@ -190,3 +190,18 @@ def test_wait_limit_is_reported(eng):
         b.close()
     # the engine stays usable
     run_check(eng, pairs, "after limit", lanes=ta.LANES_LONG, **DNA_PARAMS)
+
+
+@pytest.mark.parametrize("la, lb", [(1, 700), (512, 513), (513, 512), (1024, 1025), (700, 511), (2049, 1537),
+                                    (600, 3000), (3000, 600), (5000, 64)])
+def test_region_and_checkpoint_edges(eng, la, lb):
+    # forward strips and regions of 512 rows, checkpoint columns every 512, chunks of 256 column codes; a border
+    # value above 0 (|extend| > |open|) masks the strips' first blocks; scores beyond int8 take the 16-bit slots
+    rng = random.Random(la * 7 + lb)
+    a = "".join(rng.choice("ACGT") for _ in range(la))
+    b = "".join(rng.choice("ACGT") for _ in range(lb))
+    cut = rng.randint(0, min(la, lb) // 2)
+    pairs = [(a, b), (a, (a[:cut] + b + a[cut:])[:lb] or "A"), (a, (a[cut:] + b)[:lb] or "A")]
+    for go, ge, ma, mi in ((-5, -2, 2, -3), (-2, -9, 2, -3), (0, 0, 1, -1), (-100, -60, 90, -90)):
+        run_check(eng, pairs, "regions %d %d" % (go, ge), lanes=ta.LANES_LONG, mode=ta.GLOBAL, alphabet=ta.DNA,
+                  gap_open=go, gap_extend=ge, match=ma, mismatch=mi)

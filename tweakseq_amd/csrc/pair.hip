@@ -100,66 +100,6 @@ __device__ __forceinline__ uint4 encode16(const int8_t *lmap, uint4 v, int x, in
   return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
-// A strip's surroundings in the workgroup's LDS (strip.h): the ring of the
-// strip above, its progress counter, the pair's column codes.  The ring
-// holds column x at entry x + 64.
-template <int PR, bool GP>
-struct PairIO {
-  const uint8_t *bcode;      // this lane's first column code, at step 0
-  uint32_t slot_add;
-  int32_t *pin, *pout, *status;
-  int2 *rin, *rout;          // rin: lane 0's entries (strip 0: 8 border entries), the others' 8 zero entries
-  int rin_step, need0, cols, s, spin_limit, seen = 0;
-  uint32_t *pl;              // this lane's next dword, pl_step apart (a lane past the query: one unused dword)
-  int pl_step;
-  bool lost = false;         // a wait gave up: no more waits
-
-  __device__ __forceinline__ uint64_t codes(int b) const {
-    uint64_t w;
-    __builtin_memcpy(&w, bcode + 8 * b, 8);
-    return w;
-  }
-  __device__ __forceinline__ int need(int b) const { return need0 | (8 * b + 8 < cols ? 8 * b + 8 : cols); }
-  __device__ __forceinline__ void peek() {
-    seen = __hip_atomic_load(pin, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-  }
-  __device__ __forceinline__ void await(int b) {
-    const int want = need(b);
-    int spins = 0;
-    while (!lost && __builtin_amdgcn_readfirstlane(seen) < want) {
-      if (++spins > spin_limit) {
-        if ((threadIdx.x & 63) == 0) atomicOr(status, PAIR_GAVE_UP);
-        lost = true;
-      }
-      __builtin_amdgcn_s_sleep(1);
-      peek();
-    }
-    asm volatile("" ::: "memory");  // the ring's reads stay below (a wave's LDS accesses keep their order)
-  }
-  __device__ __forceinline__ void tops(int b, int half, int (&g)[8], int (&f)[8]) const {
-    const int4 *r = (const int4 *)(rin + b * rin_step) + 2 * half;
-    const int4 v = r[0], w = r[1];
-    const int q = 4 * half;
-    g[q] = v.x; f[q] = v.y; g[q + 1] = v.z; f[q + 1] = v.w;
-    g[q + 2] = w.x; f[q + 2] = w.y; g[q + 3] = w.z; f[q + 3] = w.w;
-  }
-  __device__ __forceinline__ void bottom(int b, const int (&g)[8], const int (&f)[8]) {
-    if ((threadIdx.x & 63) == 63) {
-      int2 *r = rout + 8 * b + 1;
-#pragma unroll
-      for (int q = 0; q < 8; ++q) r[q] = make_int2(g[q], f[q]);
-      int done = 8 * b + 8 - 63;
-      done = done < 0 ? 0 : done;
-      asm volatile("" ::: "memory");  // the entries first (a wave's LDS accesses keep their order)
-      __hip_atomic_store(pout, ((s + 1) << 20) | done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    }
-  }
-  __device__ __forceinline__ void planes(uint32_t dw) {
-    *pl = dw;
-    pl += pl_step;
-  }
-};
-
 // Direction codes in LDS, all at hand: dwords [strip][t / SPD][lane], the
 // last strip as wide as it has lanes.
 template <int PR>
@@ -244,7 +184,7 @@ __global__ __launch_bounds__(64 * PAIR_WAVES) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
     for (int k = 0; k < PR; ++k) line[k] = tab + 32 * (r0 + k < m ? acode[r0 + k] : PAIR_PAD_LINE);
     strip_slot<PR>(lds + slot, line, K, LOCAL ? 0 : -A.open - A.ext, LOCAL ? PAD_SCORE : A.ext - A.open);
-    PairIO<PR, GP> io;
+    StripGroupIO io;
     io.bcode = bcode + 64 - lane;
     io.slot_add = 0x01010101u * ((uint32_t)((uint32_t)(uintptr_t)(lds_u8 *)lds + slot) >> 8);
     io.status = sy + SY_STATUS;
@@ -258,6 +198,7 @@ __global__ __launch_bounds__(64 * PAIR_WAVES) __attribute__((amdgpu_waves_per_eu
     io.cols = T - 63;
     io.s = s;
     io.spin_limit = A.spin_limit;
+    io.gave_up = PAIR_GAVE_UP;
     if constexpr (GP) {
       io.pl = (uint32_t *)A.planes + (size_t)s * (T / SPD) * 64 + lane;
       io.pl_step = 64;

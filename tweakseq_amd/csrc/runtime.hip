@@ -500,6 +500,29 @@ bool long_pair(const ta_params &p, int la, int lb) {
   return p.lanes == TA_LANES_AUTO && (int64_t)la * lb >= kLongCells;
 }
 
+// Long pairs whose bottom rows and checkpoints share memory with other groups':
+// pairs [lp0, + npairs), queue items [it0, + nitems), ring entries [0, ring_n).
+struct LongGroup {
+  int lp0, npairs, it0, nitems;
+  uint64_t ring_n;
+};
+
+// Device memory a long pair is admitted for: a checkpoint row every 4,096 rows, a
+// checkpoint column every 1,024 columns, one region's codes.  (What a batch takes
+// is limited to this, or 16 GB where that is more.)
+int64_t long_pair_estimate(int64_t la, int64_t lb) {
+  const int64_t rl = ((lb + 7) & ~7ll) + 80, S = (la + 511) / 512;
+  return (S - 1) / 8 * 8 * rl + (lb - 1) / 1024 * S * 512 * 8 + 8 * 64 * ((std::min<int64_t>(lb, 5376) + 71) / 8) * 32;
+}
+int64_t long_estimate(const std::vector<HostPair> &hp, const std::vector<int> &lk) {
+  int64_t t = 0;
+  for (int k : lk) t += long_pair_estimate(hp[k].la, hp[k].lb);
+  return t;
+}
+
+// Dwords of region codes of a long-pair traceback workgroup.
+constexpr size_t kLongPlanes = (size_t)LTW * LREG_T / strip_spd(2) * 64;
+
 // Residue codes one task's strips and columns read (expand_codes_kernel).
 struct CodeJob {
   uint64_t row_off, col_off;
@@ -825,12 +848,10 @@ int pick_gg(int mmax, int n, double mean_slot, bool few) {
 // Start of a run: work-queue counters to 0, fill outputs to their initial
 // values (empty pairs keep theirs), long-pair progress counters to 0.  A
 // kernel rather than memset / memcpy nodes, so a captured run is all kernels.
-__global__ void init_kernel(int32_t *ctr, int nctr, FillOut *fo, const FillOut *fo_init, int n, int32_t *prog,
-                            int nprog) {
+__global__ void init_kernel(int32_t *ctr, int nctr, FillOut *fo, const FillOut *fo_init, int n) {
   const int tid = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
   for (int k = tid; k < nctr; k += stride) ctr[k] = 0;
   for (int k = tid; k < n; k += stride) fo[k] = fo_init[k];
-  for (int k = tid; k < nprog; k += stride) prog[k] = 0;
 }
 
 }  // namespace
@@ -887,13 +908,13 @@ struct ta_batch {
   std::vector<LongPair> longs;
   std::vector<LongItem> litems;
   std::vector<int32_t> litem_first;  // per long pair: its first queue item
+  std::vector<LongGroup> lgroups;
   LongPair *d_lp = nullptr;
   LongItem *d_litems = nullptr;
-  int32_t *d_lring = nullptr, *d_lck = nullptr, *d_lprog = nullptr, *d_wring = nullptr;
-  int2 *d_lcol = nullptr;
-  uint8_t *d_wtb = nullptr;
-  uint64_t lring_elems = 0, lck_elems = 0, lcol_elems = 0, wring_stride = 0, wtb_stride = 0;
-  int32_t lprog_n = 0, long_wgs = 0, spin_limit = 1 << 20;  // about a second of polling
+  int2 *d_lring = nullptr, *d_lcol = nullptr;
+  uint32_t *d_wpl = nullptr;  // region codes of the traceback workgroups
+  uint64_t lring_n = 0, lcol_n = 0;
+  int32_t long_wgs = 0, spin_limit = 1 << 20;  // about a second of polling
   // Most steps a traceback walk may take (TWEAKALIGN_WALK_GUARD lowers it so
   // that walks end flagged; otherwise above every walk's length).
   int32_t guard_cap = INT32_MAX;
@@ -974,8 +995,7 @@ void ta_batch_destroy(ta_batch *B) {
   dfree(B->d_ptb); dfree(B->d_pairs); dfree(B->d_fo); dfree(B->d_res); dfree(B->d_cig);
   dfree(B->d_ctr); dfree(B->d_fo_init); dfree(B->d_order); dfree(B->d_order_rest);
   free_rerun(B);
-  dfree(B->d_lp); dfree(B->d_litems); dfree(B->d_lring); dfree(B->d_lck); dfree(B->d_lcol); dfree(B->d_lprog);
-  dfree(B->d_wring); dfree(B->d_wtb);
+  dfree(B->d_lp); dfree(B->d_litems); dfree(B->d_lring); dfree(B->d_lcol); dfree(B->d_wpl);
   dfree(B->d_spairs); dfree(B->d_sitems); dfree(B->d_sring); dfree(B->d_splanes); dfree(B->d_sbest);
   dfree(B->d_sscore);
   dfree(B->d_plain_tasks); dfree(B->d_prow); dfree(B->d_pcol); dfree(B->d_pring);
@@ -1496,33 +1516,34 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
     std::stable_sort(lk.begin(), lk.end(), [&](int x, int y) {
       return (int64_t)B->hp[x].la * B->hp[x].lb > (int64_t)B->hp[y].la * B->hp[y].lb;
     });
-    int max_rl = 0, max_n = 0;
+    // Bottom rows and column checkpoints take about 1/32 byte a cell: pairs
+    // go in groups that share the memory one after the other.
+    const uint64_t limit = (uint64_t)std::max<int64_t>((int64_t)16 << 30, long_estimate(B->hp, lk));
+    uint64_t ring = 0, col = 0;
     for (int k : lk) {
       const HostPair &h = B->hp[k];
       LongPair L{};
       L.pid = k; L.m = h.la; L.n = h.lb; L.S = ceil_div(h.la, LST);
+      L.T = (h.lb + 63 + 7) & ~7;
       L.a_off = h.a_off; L.b_off = h.b_off;
-      L.rl = ((h.lb + 7) & ~7) + 80;  // block loads / stores run up to 71 columns past n
-      L.ring_off = B->lring_elems;
-      if (L.S > 1) B->lring_elems += 4ull * L.rl;
-      L.ck_off = B->lck_elems;
-      if (p->traceback) B->lck_elems += (uint64_t)((L.S - 1) / KC) * 2 * L.rl;
-      L.colck_off = B->lcol_elems;
-      if (p->traceback) B->lcol_elems += (uint64_t)((L.n - 1) / CKX) * L.S * LST;
-      L.prog_off = B->lprog_n;
-      B->lprog_n += L.S;
+      const uint64_t nr = (uint64_t)(L.S - 1) * (L.T + 8);
+      const uint64_t nc = p->traceback ? (uint64_t)((L.n - 1) / CKX) * L.S * LST : 0;
+      if (B->lgroups.empty() || (ring + col && 8 * (ring + col + nr + nc) > limit)) {
+        ring = col = 0;
+        B->lgroups.push_back(LongGroup{(int)B->longs.size(), 0, (int)B->litems.size(), 0, 0});
+      }
+      L.ring = ring; L.colck = col;
+      ring += nr; col += nc;
+      B->lring_n = std::max(B->lring_n, ring);
+      B->lcol_n = std::max(B->lcol_n, col);
       B->litem_first.push_back((int32_t)B->litems.size());
       for (int s = 0; s < L.S; ++s) B->litems.push_back(LongItem{(int32_t)B->longs.size(), s});
       B->longs.push_back(L);
+      LongGroup &g = B->lgroups.back();
+      g.npairs += 1; g.nitems += L.S; g.ring_n = ring;
       pl.ptb[k].P = 3;
-      max_rl = std::max(max_rl, L.rl);
-      max_n = std::max(max_n, L.n);
     }
-    if (!lk.empty() && p->traceback) {
-      B->wring_stride = 4ull * max_rl;
-      B->wtb_stride = (uint64_t)KC * GWAVE * ((std::min(max_n, LREG) + GWAVE + 7) / 8) * 32;
-      B->long_wgs = std::max(1, std::min((int)lk.size(), 2 * ctx->cus));
-    }
+    if (!lk.empty() && p->traceback) B->long_wgs = std::max(1, std::min((int)lk.size(), 2 * ctx->cus));
     if (const char *e = getenv("TWEAKALIGN_SPIN_LIMIT")) B->spin_limit = std::max(1, atoi(e));
     if (const char *e = getenv("TWEAKALIGN_WALK_GUARD")) B->guard_cap = std::max(0, atoi(e));
   }
@@ -1573,16 +1594,13 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
   rc = rc ? rc : dalloc(&B->d_cig, B->cig_bytes);
   rc = rc ? rc : dalloc(&B->d_ctr, 16);
   if (!rc && hipMemsetAsync(B->d_ctr, 0, 16 * sizeof(int32_t), st) != hipSuccess) rc = TA_E_DEVICE;
-  rc = rc ? rc : dalloc(&B->d_lring, B->lring_elems);
-  rc = rc ? rc : dalloc(&B->d_lck, B->lck_elems);
-  rc = rc ? rc : dalloc(&B->d_lcol, B->lcol_elems);
-  rc = rc ? rc : dalloc(&B->d_lprog, (size_t)B->lprog_n);
+  rc = rc ? rc : dalloc(&B->d_lring, B->lring_n);
+  rc = rc ? rc : dalloc(&B->d_lcol, B->lcol_n);
   rc = rc ? rc : dalloc(&B->d_sring, B->sring_n);
   rc = rc ? rc : dalloc(&B->d_splanes, B->splanes_n);
   rc = rc ? rc : dalloc(&B->d_sbest, B->spairs.size());
   rc = rc ? rc : dalloc(&B->d_sscore, B->spairs.size());
-  rc = rc ? rc : dalloc(&B->d_wring, B->wring_stride * B->long_wgs);
-  rc = rc ? rc : dalloc(&B->d_wtb, B->wtb_stride * B->long_wgs);
+  rc = rc ? rc : dalloc(&B->d_wpl, kLongPlanes * B->long_wgs);
   for (auto &e : B->ev)
     if (!rc && hipEventCreate(&e) != hipSuccess) rc = TA_E_DEVICE;
   tr.mark("allocations");
@@ -1612,10 +1630,8 @@ int64_t batch_tb_estimate(const ta_params *p, const ta_pair *pairs, int32_t n) {
   for (int32_t k = 0; k < n; ++k) {
     const int la = pairs[k].la, lb = pairs[k].lb;
     if (la <= 0 || lb <= 0) continue;
-    if (long_pair(*p, la, lb)) {  // row + column checkpoints, one traceback workgroup's planes
-      const int64_t rl = ((lb + 7) & ~7) + 80, S = ceil_div(la, LST);
-      t += (S - 1) / KC * 8 * rl + (int64_t)((lb - 1) / CKX) * S * LST * 8 +
-           (int64_t)KC * GWAVE * ((std::min(lb, LREG) + GWAVE + 7) / 8) * 32;
+    if (long_pair(*p, la, lb)) {
+      t += long_pair_estimate(la, lb);
     } else {
       t += (int64_t)ceil_div(la, STRIP) * ceil_div(lb + G, 8) * (G * R * 4);
     }
@@ -1627,8 +1643,7 @@ int ta_batch_info(ta_batch *B, int64_t *cells, int64_t *tb_bytes, int32_t *tasks
   if (!B) return TA_E_INVALID;
   if (cells) *cells = B->cells;
   if (tb_bytes)
-    *tb_bytes = (int64_t)(B->plan.tb_bytes + B->wtb_stride * B->long_wgs + 4 * B->lck_elems + 8 * B->lcol_elems +
-                          4 * B->splanes_n);
+    *tb_bytes = (int64_t)(B->plan.tb_bytes + 4 * kLongPlanes * B->long_wgs + 8 * B->lcol_n + 4 * B->splanes_n);
   if (tasks)
     *tasks = (int32_t)(B->plan.tasks2[0].size() + B->plan.tasks2[1].size() + B->plan.tasks2[2].size() +
                        B->plan.tasks1[0].size() + B->plan.tasks1[1].size() + B->litems.size() + B->sitems.size());
@@ -1725,9 +1740,7 @@ LongArgs long_args(ta_batch *B, int it0, int nit, int lp0, int nlp) {
   a.items = B->d_litems + it0; a.nitems = nit;
   a.ctr = B->d_ctr + 8;
   a.table = B->d_table; a.Kp = B->Kp; a.codes = B->d_codes;
-  a.ring = B->d_lring; a.ckpt = B->d_lck; a.prog = B->d_lprog; a.colck = B->d_lcol;
-  a.wring = B->d_wring; a.wring_stride = B->wring_stride;
-  a.wtb = B->d_wtb; a.wtb_stride = B->wtb_stride;
+  a.ring = B->d_lring; a.colck = B->d_lcol; a.wpl = B->d_wpl;
   a.pd = B->d_pairs; a.fo = B->d_fo; a.res = B->d_res; a.cig = B->d_cig;
   a.open = B->p.gap_open; a.ext = B->p.gap_extend;
   a.ckpt_on = B->p.traceback;
@@ -1736,34 +1749,38 @@ LongArgs long_args(ta_batch *B, int it0, int nit, int lp0, int nlp) {
   return a;
 }
 
-// Forward pass of long pairs: counters cleared, then one wave per workgroup
-// pulling strips.  Items index pairs relative to lp0 = 0, so a subset of
-// items must keep the full pair array.
-int launch_long_fwd(ta_ctx *ctx, ta_batch *B, int it0, int nit, bool clear) {
+// Forward pass of queue items [it0, it0 + nit), whose pairs' bottom rows lie in
+// entries [ring0, ring0 + ring_n): entries emptied and counters cleared, then
+// one wave per workgroup pulling strips.  Items name pairs from 0.
+int launch_long_fwd(ta_ctx *ctx, ta_batch *B, int it0, int nit, uint64_t ring0, uint64_t ring_n) {
   if (nit <= 0) return TA_OK;
-  if (clear) {  // the per-pair (plain) form; a batch run starts with init_kernel
-    HIPCHK(hipMemsetAsync(B->d_ctr + 8, 0, 3 * sizeof(int32_t), B->stream));
-    HIPCHK(hipMemsetAsync(B->d_lprog, 0, sizeof(int32_t) * B->lprog_n, B->stream));
-  }
-  LongArgs a = long_args(B, it0, nit, 0, (int)B->longs.size());
-  const int lds = long_fwd_lds(B->Kp);
-  const int per_cu = std::max(1, std::min(16, (160 * 1024) / lds));  // 4 waves per SIMD (117 VGPRs)
-  const int grid = std::max(1, std::min(nit, ctx->cus * per_cu));
+  const uint64_t n16 = ring_n / 2;
   (void)hipGetLastError();
-  hipLaunchKernelGGL(long_fwd_kernel, dim3(grid), dim3(64), lds, B->stream, a);
+  hipLaunchKernelGGL(long_init_kernel<0>, dim3((unsigned)std::max<uint64_t>(1, std::min<uint64_t>(4096, (n16 + 255) / 256))),
+                     dim3(256), 0, B->stream, (uint4 *)(B->d_lring + ring0), n16, B->d_ctr + 8);
+  const LongArgs a = long_args(B, it0, nit, 0, (int)B->longs.size());
+  const bool dna = B->Kp <= STRIP_NC_DNA;
+  const int gaps = -a.open - a.ext, pad = a.ext - a.open;  // scores are kept plus gaps, the pad's as it is
+  const bool bytes = B->alph.minS + gaps >= -128 && B->alph.maxS + gaps <= 127 && PAD_SCORE + gaps <= 127 &&
+                     pad >= -128 && pad <= 127;
+  constexpr int D = STRIP_NC_DNA, P = STRIP_NC;
+  const int lds = dna ? (bytes ? long_fwd_lds<D, true> : long_fwd_lds<D, false>)
+                      : (bytes ? long_fwd_lds<P, true> : long_fwd_lds<P, false>);
+  void (*k)(LongArgs) = dna ? (bytes ? long_fwd_kernel<D, true> : long_fwd_kernel<D, false>)
+                            : (bytes ? long_fwd_kernel<P, true> : long_fwd_kernel<P, false>);
+  const int per_cu = std::max(1, std::min(LONG_WAVES, ctx->lds_max / lds));
+  hipLaunchKernelGGL(k, dim3(std::max(1, std::min(nit, ctx->cus * per_cu))), dim3(64), lds, B->stream, a);
   HIPCHK(hipGetLastError());
   return TA_OK;
 }
 
-// Traceback of long pairs [lp0, lp0 + nlp): one workgroup of LW waves per pair.
-int launch_long_tb(ta_ctx *ctx, ta_batch *B, int lp0, int nlp, bool clear) {
+// Traceback of long pairs [lp0, lp0 + nlp): one workgroup per pair.
+int launch_long_tb(ta_ctx *ctx, ta_batch *B, int lp0, int nlp) {
   if (nlp <= 0 || !B->p.traceback) return TA_OK;
-  if (clear) HIPCHK(hipMemsetAsync(B->d_ctr + 9, 0, sizeof(int32_t), B->stream));
-  LongArgs a = long_args(B, 0, 0, lp0, nlp);
-  const int lds = long_tb_lds(B->Kp);
-  const int grid = std::max(1, std::min(nlp, B->long_wgs));
+  const LongArgs a = long_args(B, 0, 0, lp0, nlp);
   (void)hipGetLastError();
-  hipLaunchKernelGGL(long_tb_kernel, dim3(grid), dim3(64 * LW), lds, B->stream, a);
+  hipLaunchKernelGGL(long_tb_kernel<0>, dim3(std::max(1, std::min(nlp, B->long_wgs))), dim3(64 * LTW), LONG_TB_LDS,
+                     B->stream, a);
   HIPCHK(hipGetLastError());
   return TA_OK;
 }
@@ -1867,7 +1884,7 @@ namespace {
 int launch_init(ta_batch *B) {
   (void)hipGetLastError();
   hipLaunchKernelGGL(init_kernel, dim3(std::max(1, std::min(1024, (B->n + 255) / 256))), dim3(256), 0, B->stream,
-                     B->d_ctr, 16, B->d_fo, B->d_fo_init, B->n, B->d_lprog, B->lprog_n);
+                     B->d_ctr, 16, B->d_fo, B->d_fo_init, B->n);
   HIPCHK(hipGetLastError());
   return TA_OK;
 }
@@ -1881,7 +1898,12 @@ int launch_fills(ta_ctx *ctx, ta_batch *B) {
   if (!rc) rc = launch_fill<1>(ctx, B, B->d_tasks1, n1, B->d_rowcodes, B->d_colcodes, B->d_ring, B->d_tb,
                                B->d_ctr + 2, 0, B->walk);
   if (!rc) rc = launch_strips(ctx, B);
-  if (!rc) rc = launch_long_fwd(ctx, B, 0, (int)B->litems.size(), false);
+  // Long pairs, group by group; the last group's traceback is launch_tracebacks'.
+  for (size_t g = 0; !rc && g < B->lgroups.size(); ++g) {
+    const LongGroup &L = B->lgroups[g];
+    rc = launch_long_fwd(ctx, B, L.it0, L.nitems, 0, L.ring_n);
+    if (!rc && g + 1 < B->lgroups.size()) rc = launch_long_tb(ctx, B, L.lp0, L.npairs);
+  }
   return rc;
 }
 
@@ -1899,7 +1921,7 @@ int launch_tracebacks(ta_ctx *ctx, ta_batch *B) {
                        B->stream, a);
     HIPCHK(hipGetLastError());
   }
-  if (!rc) rc = launch_long_tb(ctx, B, 0, (int)B->longs.size(), false);
+  if (!rc && !B->lgroups.empty()) rc = launch_long_tb(ctx, B, B->lgroups.back().lp0, B->lgroups.back().npairs);
   return rc;
 }
 
@@ -2385,9 +2407,10 @@ int ta_batch_run_plain(ta_ctx *ctx, ta_batch *B, int32_t first, int32_t count) {
     const HostPair &h = B->hp[k];
     if (h.path == 3) {
       const int q = lp_of[k];
-      int rc = launch_long_fwd(ctx, B, B->litem_first[q], B->longs[q].S, true);
+      const LongPair &L = B->longs[q];
+      int rc = launch_long_fwd(ctx, B, B->litem_first[q], L.S, L.ring, (uint64_t)(L.S - 1) * (L.T + 8));
       if (!rc) rc = launch_traceback(ctx, B, B->d_pairs, B->d_pptb, B->d_ptbuf, k, 1);
-      if (!rc) rc = launch_long_tb(ctx, B, q, 1, true);
+      if (!rc) rc = launch_long_tb(ctx, B, q, 1);
       if (rc) return rc;
       continue;
     }

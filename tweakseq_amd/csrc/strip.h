@@ -43,15 +43,20 @@ template <int PR>
 __device__ __forceinline__ int strip_code(uint32_t dw, int q, int k) { return (int)(dw >> (28 - 4 * (q * PR + k))) & 15; }
 
 // Score slots: a row of 64 entries per code; an entry holds a lane's rows, int32 for
-// one row, int16 pairs for two, two tables of such pairs for four.
+// one row, int16 pairs for two, PR / 2 tables of such pairs for more (NC rows apart),
+// or int8 quadruples in PR / 4 tables (BYTES; where every score fits).
 constexpr int STRIP_NC = 24;                  // codes (23 residues and a pad)
+constexpr int STRIP_NC_DNA = 8;               // 4 and a pad
 constexpr int STRIP_ROW = 256;                // bytes per code
-__host__ __device__ constexpr int strip_slot_bytes(int PR) { return (PR == 4 ? 2 : 1) * STRIP_NC * STRIP_ROW; }
+__host__ __device__ constexpr int strip_slot_tables(int PR, bool BYTES) { return PR <= 2 ? 1 : PR / (BYTES ? 4 : 2); }
+__host__ __device__ constexpr int strip_slot_bytes(int PR, int NC = STRIP_NC, bool BYTES = false) {
+  return strip_slot_tables(PR, BYTES) * NC * STRIP_ROW;
+}
 
 // Fills the calling lane's slot entries at LDS byte `slot` + 4 lane: row k's score
 // against code c < nc is line[k][c] + bias (line: 32-byte table lines in LDS); code
 // nc, the pad outside the columns, scores `pad`.
-template <int PR>
+template <int PR, int NC = STRIP_NC, bool BYTES = false>
 __device__ __forceinline__ void strip_slot(uint8_t *slot, const uint8_t *const (&line)[PR], int nc, int bias, int pad) {
   const int lane = threadIdx.x & 63;
   for (int c4 = 0; c4 <= nc; c4 += 4) {
@@ -66,10 +71,15 @@ __device__ __forceinline__ void strip_slot(uint8_t *slot, const uint8_t *const (
       for (int k = 0; k < PR; ++k) v[k] = c4 + b == nc ? pad : (int)(int8_t)(w[k] >> (8 * b)) + bias;
       if constexpr (PR == 1) {
         d[0] = (uint32_t)v[0];
+      } else if constexpr (BYTES) {
+#pragma unroll
+        for (int k = 0; k < PR; k += 4)
+          d[(k / 4) * NC * STRIP_ROW / 4] = ((uint32_t)v[k] & 0xffu) | (((uint32_t)v[k + 1] & 0xffu) << 8) |
+                                            (((uint32_t)v[k + 2] & 0xffu) << 16) | ((uint32_t)v[k + 3] << 24);
       } else {
 #pragma unroll
         for (int k = 0; k < PR; k += 2)
-          d[(k / 2) * STRIP_NC * STRIP_ROW / 4] = ((uint32_t)v[k] & 0xffffu) | ((uint32_t)v[k + 1] << 16);
+          d[(k / 2) * NC * STRIP_ROW / 4] = ((uint32_t)v[k] & 0xffffu) | ((uint32_t)v[k + 1] << 16);
       }
     }
   }
@@ -91,6 +101,17 @@ __device__ __forceinline__ bool strip_better(int h, int i, int j, int bh, int bi
   return h > bh || (h == bh && (i < bi || (i == bi && j < bj)));
 }
 
+// What most strips' surroundings have in common: direction codes kept, the
+// matrix's own left border, no columns kept.
+struct StripIODefaults {
+  static constexpr bool TB = true, KEEP = false, BYTES = false;
+  static constexpr int NC = STRIP_NC;
+  static constexpr const int2 *left = nullptr;
+  __device__ __forceinline__ bool keeps(int) const { return false; }
+  template <int PR>
+  __device__ __forceinline__ void column(int, const int (&)[PR], const int (&)[PR]) const {}
+};
+
 // Strip s (0-based) of an m x n pair over T = n + 63 steps (rounded up to 8).
 // IO is the strip's surroundings:
 //   uint64_t codes(b)            the codes of this lane's 8 columns of block b <= T / 8 (pads outside the columns)
@@ -101,7 +122,10 @@ __device__ __forceinline__ bool strip_better(int h, int i, int j, int bh, int bi
 //                                first strip every value is the border's (0, or 2 (open - ext)), and local
 //                                columns from T - 63 on are 0
 //   void bottom(b, g, f)         this strip's bottom row after block b, in lane 63 (columns 8 b - 63 ..)
-//   void planes(dw)              the next dword of direction codes (SPD steps)
+//   void planes(dw)              the next dword of direction codes (SPD steps; IO::TB only)
+//   bool keeps(b)                IO::KEEP: whether block b calls column(c, G, E) after each step, c the lane's column
+//   const int2 *left             (G, E) of the lane's rows in the column left of the strip's first, null at the
+//                                matrix border; the rows above it precede it
 // Local columns and H stay below 2^16 - 128 (the end-cell keys).
 //
 // Lanes left or right of the columns run along on pads: left of column 0 the
@@ -109,10 +133,12 @@ __device__ __forceinline__ bool strip_better(int h, int i, int j, int bh, int bi
 // which needs |open| >= |ext|; else those blocks are masked by column; local:
 // 0), right of the last column the values go nowhere.  So no step tests its
 // column but the last ones of the strip that holds row m, which keep H(m, n).
+// Strips that start inside the matrix (io.left) mask their first blocks too.
 template <int PR, bool LOCAL, class IO>
 __device__ __forceinline__ void strip_sweep(IO &io, int s, bool last, int m, int n, int T, int open, int ext,
                                             StripEnd &end) {
-  constexpr int SPD = strip_spd(PR), NS = PR == 4 ? 2 : 1;
+  constexpr bool TB = IO::TB;
+  constexpr int SPD = TB ? strip_spd(PR) : 1, NS = strip_slot_tables(PR, IO::BYTES);
   const int lane = threadIdx.x & 63;
   const int r0 = (s * 64 + lane) * PR;  // 0-based first row of the lane
   const int c = open - ext, go = -open, ge = -ext;
@@ -122,6 +148,16 @@ __device__ __forceinline__ void strip_sweep(IO &io, int s, bool last, int m, int
 #pragma unroll
   for (int k = 0; k < PR; ++k) { G[k] = edge; E[k] = edge; X[k] = 0; key[k] = 0; cap[k] = 0; }
   int hd = (!LOCAL && r0 == 0) ? c : edge;  // the row above at the previous column
+  const bool inner = !LOCAL && io.left != nullptr;
+  if (inner) {
+#pragma unroll
+    for (int k = 0; k < PR; ++k) {
+      const int2 v = io.left[k];
+      G[k] = v.x;
+      E[k] = v.y;
+    }
+    hd = r0 == 0 ? edge : io.left[-1].x;
+  }
   int Gb = edge, Fb = edge;                 // handed to the lane below
   int tg[8], tf[8];                         // lane 0's top inputs, each half read once its last values are used
   io.peek();
@@ -136,12 +172,13 @@ __device__ __forceinline__ void strip_sweep(IO &io, int s, bool last, int m, int
     for (int q = 0; q < 4; ++q) {
       // byte 1 = code q's slot row, byte 0 = 4 lane
       const uint32_t a = __builtin_amdgcn_perm(w, lbase, 0x0c0c0000u | ((uint32_t)(4 + q) << 8));
-      sc.v[q][0] = *(lds_cu32 *)(uintptr_t)a;
-      if constexpr (PR == 4) sc.v[q][1] = *(lds_cu32 *)(uintptr_t)(a + STRIP_NC * STRIP_ROW);
+#pragma unroll
+      for (int x = 0; x < NS; ++x) sc.v[q][x] = *(lds_cu32 *)(uintptr_t)(a + x * IO::NC * STRIP_ROW);
     }
   };
   auto score = [](const Sc &sc, int q, int k) {
-    const uint32_t w = sc.v[q][PR == 4 ? k >> 1 : 0];
+    if constexpr (IO::BYTES) return (int)(int8_t)(sc.v[q][k >> 2] >> (8 * (k & 3)));
+    const uint32_t w = sc.v[q][PR > 2 && !IO::BYTES ? k >> 1 : 0];
     return PR == 1 ? (int)w : (k & 1) ? (int)w >> 16 : (int)(int16_t)w;
   };
   uint64_t cw = io.codes(0);
@@ -168,15 +205,18 @@ __device__ __forceinline__ void strip_sweep(IO &io, int s, bool last, int m, int
         const int Gu0 = __builtin_amdgcn_update_dpp(0, Gb, 0x138, 0xf, 0xf, true) + tg[q];
         const int Fu0 = __builtin_amdgcn_update_dpp(0, Fb, 0x138, 0xf, 0xf, true) + tf[q];
         uint32_t nib = 0;
-        if (tb + q >= lane) {
+        const int c0 = tb + q - lane;
+        if (c0 >= 0) {
           int upk = Gu0, Fk = Fu0, d = hd;
 #pragma unroll
           for (int k = 0; k < PR; ++k) {
             const int Dk = d + score(Q0 ? sb : sa, q - Q0, k), Ek = max(E[k], G[k]), H = max(Dk, max(Ek, Fk));
-            nib = __builtin_amdgcn_alignbit(nib, (uint32_t)(Ek - Fk), 31);
-            nib = __builtin_amdgcn_alignbit(nib, (uint32_t)(Dk - H), 31);
-            nib = __builtin_amdgcn_alignbit(nib, (uint32_t)(upk - Fk), 31);
-            nib = __builtin_amdgcn_alignbit(nib, (uint32_t)(G[k] - Ek), 31);
+            if constexpr (TB) {
+              nib = __builtin_amdgcn_alignbit(nib, (uint32_t)(Ek - Fk), 31);
+              nib = __builtin_amdgcn_alignbit(nib, (uint32_t)(Dk - H), 31);
+              nib = __builtin_amdgcn_alignbit(nib, (uint32_t)(upk - Fk), 31);
+              nib = __builtin_amdgcn_alignbit(nib, (uint32_t)(G[k] - Ek), 31);
+            }
             d = G[k];
             E[k] = Ek;
             upk = G[k] = H + c;
@@ -186,12 +226,15 @@ __device__ __forceinline__ void strip_sweep(IO &io, int s, bool last, int m, int
           Fb = Fk;
           hd = Gu0;
         }
-        acc = (acc << (4 * PR)) | nib;
-        if ((q + 1) % SPD == 0) io.planes(acc);
+        if constexpr (TB) {
+          acc = ((PR == 8 ? 0u : acc << (4 * (PR & 7))) | nib);
+          if ((q + 1) % SPD == 0) io.planes(acc);
+        }
         rg[q] = Gb;
         rf[q] = Fb;
 #pragma unroll
-        for (int k = 0; k < PR; ++k) cap[k] = tb + q == n - 1 + lane ? G[k] : cap[k];
+        for (int k = 0; k < PR; ++k) cap[k] = c0 == n - 1 ? G[k] : cap[k];
+        if constexpr (IO::KEEP) io.column(c0, G, E);
       }
     };
     // Four steps.  The order is pinned: each operation of a row's recurrence
@@ -228,14 +271,14 @@ __device__ __forceinline__ void strip_sweep(IO &io, int s, bool last, int m, int
     };
 #define STRIP_PEND(i) \
   if (have) pend(std::integral_constant<int, i>{}, row)
-    auto steps = [&](auto cap_tag, auto q0_tag) {
-      constexpr bool CAP = decltype(cap_tag)::value;
+    auto steps = [&](auto cap_tag, auto keep_tag, auto q0_tag) {
+      constexpr bool CAP = decltype(cap_tag)::value, KEEP = decltype(keep_tag)::value;
       constexpr int Q0 = decltype(q0_tag)::value;
 #pragma unroll
       for (int q = Q0; q < Q0 + 4; ++q) {
 #pragma unroll
         for (int k = 0; k < PR; ++k) {
-          const bool have = q > 0 || k > 0;  // a row is pending (a block starts without)
+          const bool have = TB && (q > 0 || k > 0);  // a row is pending (a block starts without)
           const bool lastrow = k == PR - 1;
           int row = (k + PR - 1) % PR;       // its row of the lane
           if (k == 0 && q == 0) {  // the block's first row: nothing to pair with
@@ -314,7 +357,7 @@ __device__ __forceinline__ void strip_sweep(IO &io, int s, bool last, int m, int
           } else {
             STRIP_PEND(7);
           }
-          if (k == 0 && q % SPD == 0 && q > 0) io.planes(acc);  // the step before is complete
+          if (TB && k == 0 && q % SPD == 0 && q > 0) io.planes(acc);  // the step before is complete
           pd.En = En; pd.F = F; pd.D = D; pd.H = H; pd.up = up; pd.oe = oe;
           pd.kc = (uint32_t)(0xFFBF - (tb + q - lane));
           if (lastrow) {
@@ -328,6 +371,7 @@ __device__ __forceinline__ void strip_sweep(IO &io, int s, bool last, int m, int
 #pragma unroll
               for (int x = 0; x < PR; ++x) cap[x] = here ? G[x] : cap[x];
             }
+            if constexpr (KEEP) io.column(tb + q - lane, G, E);
           }
           if (next) {
             En = En1; D = D1;
@@ -340,7 +384,7 @@ __device__ __forceinline__ void strip_sweep(IO &io, int s, bool last, int m, int
               up = Gn;
               F = Fn;
             }
-          } else {  // the block's last row: its bits, and its dword
+          } else if constexpr (TB) {  // the block's last row: its bits, and its dword
             const bool have = true;
             row = PR - 1;
             STRIP_PEND(0); STRIP_PEND(1); STRIP_PEND(2); STRIP_PEND(3);
@@ -355,7 +399,7 @@ __device__ __forceinline__ void strip_sweep(IO &io, int s, bool last, int m, int
     };
     auto half = [&](auto q0_tag) {
       if constexpr (MODE == 0) masked_steps(q0_tag);
-      else steps(std::integral_constant<bool, MODE == 2>{}, q0_tag);
+      else steps(std::integral_constant<bool, MODE == 2>{}, std::integral_constant<bool, IO::KEEP && MODE >= 2>{}, q0_tag);
     };
     const uint64_t nw = io.codes(b + 1);
     io.tops(b, 1, tg, tf);
@@ -374,9 +418,17 @@ __device__ __forceinline__ void strip_sweep(IO &io, int s, bool last, int m, int
   };
   int b = 0;
   if constexpr (!LOCAL) {
-    if (c > 0)
-      for (; b < 8; ++b) block(b, std::integral_constant<int, 0>{});
-    for (const int kb = last ? (n - 1) / 8 : NB; b < kb; ++b) block(b, std::integral_constant<int, 1>{});
+    if (c > 0 || inner)
+      for (; b < 8 && b < NB; ++b) block(b, std::integral_constant<int, 0>{});
+    for (const int kb = last && n > 0 ? (n - 1) / 8 : NB; b < kb; ++b) {
+      if constexpr (IO::KEEP) {
+        if (io.keeps(b)) {
+          block(b, std::integral_constant<int, 3>{});
+          continue;
+        }
+      }
+      block(b, std::integral_constant<int, 1>{});
+    }
     for (; b < NB; ++b) block(b, std::integral_constant<int, 2>{});
   } else {
     for (; b < NB; ++b) block(b, std::integral_constant<int, 1>{});
@@ -395,6 +447,65 @@ __device__ __forceinline__ void strip_sweep(IO &io, int s, bool last, int m, int
       if (r0 + k + 1 == m) { end.h = cap[k] - c + ext * (m + n); end.has = true; }
   }
 }
+
+// A strip whose neighbours are in its workgroup: their bottom rows in LDS rings
+// (column x at entry x + 64), a progress counter each.
+struct StripGroupIO : StripIODefaults {
+  const uint8_t *bcode;      // this lane's first column code, at step 0
+  uint32_t slot_add;
+  int32_t *pin, *pout, *status;
+  int2 *rin, *rout;          // rin: lane 0's entries (strip 0: 8 border entries), the others' 8 zero entries
+  int rin_step, need0, cols, s, spin_limit, seen = 0;
+  uint32_t *pl;              // this lane's next dword, pl_step apart (a lane past the query: one unused dword)
+  int pl_step;
+  int gave_up;               // OR-ed into *status when a wait gives up
+  bool lost = false;         // a wait gave up: no more waits
+
+  __device__ __forceinline__ uint64_t codes(int b) const {
+    uint64_t w;
+    __builtin_memcpy(&w, bcode + 8 * b, 8);
+    return w;
+  }
+  __device__ __forceinline__ int need(int b) const { return need0 | (8 * b + 8 < cols ? 8 * b + 8 : cols); }
+  __device__ __forceinline__ void peek() {
+    seen = __hip_atomic_load(pin, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+  __device__ __forceinline__ void await(int b) {
+    const int want = need(b);
+    int spins = 0;
+    while (!lost && __builtin_amdgcn_readfirstlane(seen) < want) {
+      if (++spins > spin_limit) {
+        if ((threadIdx.x & 63) == 0) atomicOr(status, gave_up);
+        lost = true;
+      }
+      __builtin_amdgcn_s_sleep(1);
+      peek();
+    }
+    asm volatile("" ::: "memory");  // the ring's reads stay below (a wave's LDS accesses keep their order)
+  }
+  __device__ __forceinline__ void tops(int b, int half, int (&g)[8], int (&f)[8]) const {
+    const int4 *r = (const int4 *)(rin + b * rin_step) + 2 * half;
+    const int4 v = r[0], w = r[1];
+    const int q = 4 * half;
+    g[q] = v.x; f[q] = v.y; g[q + 1] = v.z; f[q + 1] = v.w;
+    g[q + 2] = w.x; f[q + 2] = w.y; g[q + 3] = w.z; f[q + 3] = w.w;
+  }
+  __device__ __forceinline__ void bottom(int b, const int (&g)[8], const int (&f)[8]) {
+    if ((threadIdx.x & 63) == 63) {
+      int2 *r = rout + 8 * b + 1;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) r[q] = make_int2(g[q], f[q]);
+      int done = 8 * b + 8 - 63;
+      done = done < 0 ? 0 : done;
+      asm volatile("" ::: "memory");  // the entries first (a wave's LDS accesses keep their order)
+      __hip_atomic_store(pout, ((s + 1) << 20) | done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+  }
+  __device__ __forceinline__ void planes(uint32_t dw) {
+    *pl = dw;
+    pl += pl_step;
+  }
+};
 
 // Codes in device memory ([strip][t / SPD][64 lanes]): a window of them in
 // LDS, 32 lanes' rows up from the walk's cell, for each lane WD dwords

@@ -81,26 +81,19 @@ __host__ __device__ constexpr int strips_lds(int bcode_bytes) {
   return SL_SLOT + strip_slot_bytes(STRIPS_PR) + bcode_bytes;
 }
 
-struct StripsIO {
-  const uint8_t *bcode;
-  uint32_t slot_add;
+// A strip whose neighbours are anywhere on the GPU: bottom rows in device
+// memory, entries that are their own flags, and a window of the row above in LDS.
+struct StripRingIO : StripIODefaults {
   uint8_t *lds;
   const int2 *rin;          // the strip above's entries, column 0 on; null above the first strip
   int2 *rout;               // this strip's
-  __amdgpu_buffer_rsrc_t pl;
-  uint32_t pl_at = 0;
-  int T, cols, spin_limit;  // cols: columns the strip above stores
+  int cols, spin_limit;     // cols: columns the strip above stores
   int32_t *err;
   int avail = 0;            // columns in the LDS window
   int2 ahead;               // the 64 entries from `avail` on, as of the last look
   int age = 0;
   bool lost = false;
 
-  __device__ __forceinline__ uint64_t codes(int b) const {
-    uint64_t w;
-    __builtin_memcpy(&w, bcode + 8 * b, 8);
-    return w;
-  }
   __device__ __forceinline__ void look() {
     const int col = avail + (int)(threadIdx.x & 63);
     ahead = make_int2(0, 0);  // past the last stored column: zeros
@@ -134,6 +127,8 @@ struct StripsIO {
           lost = true;
           break;
         }
+        // a strip that has not begun may wait for long, beside hundreds like it
+        if (avail < want && b == 0) __builtin_amdgcn_s_sleep(32);
       }
       look();
     }
@@ -159,6 +154,19 @@ struct StripsIO {
         put(7);
       }
     }
+  }
+};
+
+struct StripsIO : StripRingIO {
+  const uint8_t *bcode;
+  uint32_t slot_add;
+  __amdgpu_buffer_rsrc_t pl;
+  uint32_t pl_at = 0;
+
+  __device__ __forceinline__ uint64_t codes(int b) const {
+    uint64_t w;
+    __builtin_memcpy(&w, bcode + 8 * b, 8);
+    return w;
   }
   __device__ __forceinline__ void planes(uint32_t dw) {
     __builtin_amdgcn_raw_buffer_store_b32(dw, pl, 4u * (threadIdx.x & 63), pl_at, 0);
@@ -216,7 +224,6 @@ __global__ __launch_bounds__(64) void strips_kernel(StripsArgs A) {
     io.rout = A.ring + P.ring + (uint64_t)s * (T + 8);
     io.pl = __builtin_amdgcn_make_buffer_rsrc(A.planes + P.planes + (uint64_t)s * (T / SPD) * 64, 0, (T / SPD) * 256,
                                               0x00020000);
-    io.T = T;
     io.cols = T - 63;
     io.spin_limit = A.spin_limit;
     io.err = A.err;
