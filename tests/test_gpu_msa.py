@@ -93,6 +93,34 @@ def test_long_profiles_in_strips(eng, alphabet):
     assert joins == wjoins and rows == want
 
 
+@pytest.mark.parametrize("lens", [(1, 1, 2), (8, 9, 64, 65), (127, 128, 129, 130), (150,) * 8, (2047, 2049, 260, 1)])
+@pytest.mark.parametrize("go,ge", [(-10, -1), (-1, -5), (0, 0), (-1000, -1000)])
+def test_join_edges(eng, lens, go, ge):
+    """Edges of a strip's rows, blocks and waves; gaps that open cheaper than
+    they extend, that cost nothing, and the largest."""
+    rng = random.Random(sum(lens) + go)
+    base = "".join(rng.choice(AA) for _ in range(max(lens)))
+    seqs = []
+    for n in lens:
+        at = rng.randint(0, max(lens) - n)
+        seqs.append("".join(rng.choice(AA) if rng.random() < 0.2 else c for c in base[at:at + n]))
+    p = ta.engine.make_params(mode=ta.GLOBAL, gap_open=go, gap_extend=ge)
+    rows, joins = eng.msa(seqs, p)
+    want, wjoins = oracle_rows(seqs, go=go, ge=ge)
+    assert joins == wjoins and rows == want
+
+
+@pytest.mark.parametrize("go,ge", [(-1000, -1000), (-1, -1000)])
+def test_join_sums_past_32_bits(eng, go, ge):
+    """Two families of 50: the last join scales its gap costs by 2,500."""
+    rng = random.Random(-go)
+    seqs = family(rng, 50, 360) + family(rng, 50, 330)
+    p = ta.engine.make_params(mode=ta.GLOBAL, gap_open=go, gap_extend=ge)
+    rows, joins = eng.msa(seqs, p)
+    want, wjoins = oracle_rows(seqs, go=go, ge=ge)
+    assert joins == wjoins and rows == want
+
+
 def test_two_sequences_are_the_pairwise_alignment(eng):
     rng = random.Random(11)
     a, b = family(rng, 2, 200)

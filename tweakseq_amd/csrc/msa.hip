@@ -15,26 +15,32 @@
 //     cluster's profile (DP rows) with the higher one's (DP columns) by
 //     global Gotoh -- match score M(i,j) = cntA[i] . PB[j] with
 //     PB[j][x] = sum_y S(x,y) cntB[j][y], gap costs times nA * nB, the
-//     pairwise ties (diag > E > F, E / F prefer opening) -- then walks the
-//     direction bytes back from (la, lb) to ops; the host applies the ops to
-//     the profiles' rows.
+//     pairwise ties (diag > E > F, E / F prefer opening) -- and walks the
+//     direction codes back from (la, lb) to runs.
+//
+// Profiles stay on the device: a cluster's column is a row of 24 residue
+// counts and 24 PB entries.  Both are sums over its sequences, so a join's
+// workgroup makes the merged columns by adding the rows its runs bring
+// together, and records for each column of either side the merged column it
+// went to; in the end a thread per residue follows those maps to the root.
+// The host sees each join's length only, which sizes the next level.  (A
+// sequence's own columns are rows of a table of K, picked by its codes.)
 //
 // Each level first scores every column pair of every join over the whole GPU
-// (msa_scores_kernel, 64 x 64-cell tiles; int32: nA * nB is bounded so that
-// 24 codes x 11 x nA * nB fits), in the order the sweeps read them.  Then a
-// join's workgroup sweeps the DP in the register-strip form of the pairwise
-// fill: a strip is
-// 64 lanes x JR rows, lane l holds its JR rows' H and E in registers and
-// works on column t - l + 1 at step t; the bottom row (H, F) reaches the
-// next lane one step later through a wave_shr:1 DPP move, so a wave needs
-// no barrier at all.  The workgroup's four waves take strips s, s + 4, ...;
-// strip s + 1 reads strip s's last row from an LDS ring once strip s has
-// published (an LDS progress counter per strip slot, workgroup scope,
-// bounded waits) that it stored the columns it needs.  Values are int32
-// where the join's bound allows (most joins), else int64.  Direction bytes
-// go out per lane and step, [strip][8-step block][lane][step][row].  The walk
-// back runs on thread 0 over 64 x 64 tiles of direction bytes that the
-// workgroup stages in LDS, one barrier pair per tile.
+// (msa_scores_kernel; int32: nA * nB is bounded so that 24 codes x 11 x
+// nA * nB fits), in the order the sweeps read them, pads included.  A join's
+// workgroup then sweeps strips of 128 rows (strip.h, 2 rows a lane), a wave
+// each, up to 16 waves; each trails the one above through a ring of bottom
+// rows in LDS.  Its values G = H - ext (i + j) + (open - ext) stay between
+// 3 (open - ext) nA nB and min(la, lb) (max S + 2 |ext|) nA nB; joins where
+// that could leave int32 take the plain recurrence in int64.
+//
+// Bound by the dependent steps of the largest join of a level: lb + 63 + 72
+// a strip of 128 rows, each as long as a wave takes to issue it.  512
+// sequences of 100 to 600 (17 levels): with a plain recurrence that passed
+// direction bytes to a walk by one thread, and counts made by the host from
+// row-by-row profiles, a level took 420 us of join kernel and 800 us in all;
+// now 161 us and 240 us; the call 32.6 -> 20.0 ms.
 
 #include <hip/hip_runtime.h>
 
@@ -45,246 +51,215 @@
 #include <vector>
 
 #include "runtime_internal.h"
+#include "strip.h"
+#include "walk.h"
 
 namespace {
 
-constexpr int JT = 256;                  // threads per join: 4 waves
-constexpr int JW = JT / 64;              // waves per join
-constexpr int JRMAX = 8;                 // DP rows per lane at most (a strip: 64 * JR rows)
-constexpr int TW = 64;                   // walk tile: TW x TW direction bytes in LDS
-constexpr int KS = 24;                   // row stride of counts and PB (codes padded with zeros)
+using namespace ta;
+
+constexpr int JWMAX = 16;                // waves per join at most
+constexpr int JR = 2;                    // DP rows per lane
+constexpr int JRS = 64 * JR;             // DP rows per strip
+constexpr int KS = 24;                   // codes of a column, padded with zeros
+constexpr int CI = 2 * KS / 4;           // int4s of a column: its KS counts, then its KS PB entries
 constexpr int64_t WMAX = 8000000;        // nA * nB bound: 24 codes x 11 x nA * nB fits int32
 
+// One side of a join: len columns, of a sequence (codes) or of a joined cluster (rows).
+struct JoinSide {
+  const uint8_t *code;  // a sequence: its residue codes
+  const int4 *rows;     // a cluster: CI int4s per column
+  int32_t *map;         // the merged column of each of its columns
+  int32_t len;
+};
+
 struct JoinJob {
-  int32_t la, lb;
+  JoinSide a, b;
   int64_t w;        // nA * nB: gap costs scale
-  int64_t cnt_off;  // la x KS: residues of each code in A's columns
-  int64_t pb_off;   // lb x KS: PB[j][x] = sum_y S(x, y) cntB[j][y]
-  int64_t m_off;    // match scores M(i, j) in the sweep's order: [strip][step][lane][row]
-  int64_t tb_off;   // direction bytes src | e << 2 | f << 3, [strip][block][lane][step][row]
-  int64_t ops_off;  // la + lb ops, walk order (last column first)
+  int64_t m_off;    // match scores in the sweep's order: [strip][step][lane][row]
+  int64_t tb_off;   // direction codes, dwords of 4 steps x 2 rows: [strip][step / 4][lane]
+  int64_t run_off;  // la + lb + 2 runs
+  int64_t src_off;  // la + lb merged columns: (A's column or -1, B's column or -1)
+  int4 *out;        // the merged columns' rows (null: not needed)
 };
 
 struct JoinArgs {
   const JoinJob *jobs;
-  const int32_t *cnt, *pb;
+  const int4 *leaf;   // rows of the K single residues
   int32_t *mbuf;
-  uint8_t *tb;
-  uint8_t *ops;
+  uint32_t *tb, *runs;
+  int2 *src;
   int32_t *nops;
-  int32_t *err;     // | 1: a wait on another wave's progress gave up
-  int32_t K, open, ext, spin_limit;
+  int32_t *err;       // | 1: a wait on another wave's progress gave up; | 2: a walk did
+  int32_t open, ext, spin_limit;
 };
 
-// 8-step blocks of a strip of a join with lb columns (lane 63 trails lane 0).
-__host__ __device__ inline int join_blocks(int lb) { return (lb + 63 + 7) / 8; }
+// Steps of a strip of a join with lb columns (lane 63 trails lane 0), in whole blocks of 8.
+__host__ __device__ inline int join_steps(int lb) { return (lb + 63 + 7) & ~7; }
+__host__ __device__ inline int join_strips(int la) { return (la + JRS - 1) / JRS; }
+// LDS of the int32 ring: a column's bottom row at entry column + 64.
+__host__ __device__ inline int join_ring(int lb) { return join_steps(lb) + 80; }
 
-// Direction byte of cell (i, j), 1-based, in a join's layout.
-__device__ __forceinline__ int64_t join_tb_at(int i, int j, int JR, int NB) {
-  const int RS = 64 * JR, r = (i - 1) % RS, l = r / JR, t = j - 1 + l;
-  return (((((int64_t)((i - 1) / RS) * NB + (t >> 3)) * 64 + l) * 8 + (t & 7)) * JR + (r % JR));
+__device__ __forceinline__ const int4 *join_row(const JoinSide &s, const int4 *leaf, int c) {
+  return s.code ? leaf + s.code[c] * CI : s.rows + (int64_t)c * CI;
 }
 
-// wave_shr:1 (lane l takes lane l - 1's value, lane 0 keeps `old`), for the
-// 32- and 64-bit value types.
-__device__ __forceinline__ int32_t shr_lane(int32_t old, int32_t v) {
-  return __builtin_amdgcn_update_dpp(old, v, 0x138, 0xf, 0xf, false);
+// Every join's match scores M(i, j) = cntA[i] . PB[j] + bias w, over the
+// whole GPU.  A tile is a strip of 128 rows and 64 of its steps: its 127
+// columns' PB rows in LDS (28 dwords apart: lanes read consecutive columns
+// without bank conflicts), a lane's two rows of counts in registers; a
+// sequence's row picks one entry.  Columns outside the pair score `pad` w.
+// M24: every count and PB entry fits 24 bits (one multiply-add a code).
+// blockIdx.x is the join, its tiles dealt over blockIdx.y.
+template <bool M24>
+__global__ __launch_bounds__(256) void msa_scores_kernel(JoinArgs A, int bias, int pad) {
+  constexpr int PS = 28;
+  __shared__ __align__(16) int32_t pbs[127 * PS];
+  const JoinJob &J = A.jobs[blockIdx.x];
+  const int la = J.a.len, lb = J.b.len, T = join_steps(lb), NC = (T + 63) / 64;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int wbias = (int)(bias * J.w), wpad = (int)(pad * J.w);
+  for (int tile = blockIdx.y; tile < join_strips(la) * NC; tile += gridDim.y) {
+    const int s = tile / NC, t0 = (tile % NC) * 64;
+    for (int x = threadIdx.x; x < 127 * 6; x += 256) {
+      const int c = t0 - 63 + x / 6;
+      if (c >= 0 && c < lb) *(int4 *)(pbs + x / 6 * PS + x % 6 * 4) = join_row(J.b, A.leaf, c)[6 + x % 6];
+    }
+    const int i0 = s * JRS + lane * JR;
+    int a[JR][KS], ac[JR];
+#pragma unroll
+    for (int k = 0; k < JR; ++k) {
+      const bool in = i0 + k < la;
+      if (J.a.code) {
+        ac[k] = in ? J.a.code[i0 + k] : 0;
+      } else {
+#pragma unroll
+        for (int x = 0; x < KS / 4; ++x) {
+          const int4 v = in ? J.a.rows[(int64_t)(i0 + k) * CI + x] : make_int4(0, 0, 0, 0);
+          a[k][4 * x] = v.x; a[k][4 * x + 1] = v.y; a[k][4 * x + 2] = v.z; a[k][4 * x + 3] = v.w;
+        }
+      }
+    }
+    __syncthreads();
+    int2 *mm = (int2 *)(A.mbuf + J.m_off) + ((int64_t)s * T + t0) * 64 + lane;
+    for (int q = wave; q < 64 && t0 + q < T; q += 4) {
+      const int c = t0 + q - lane;
+      const int32_t *pb = pbs + (q - lane + 63) * PS;
+      int2 m = make_int2(wpad, wpad);
+      if (c >= 0 && c < lb) {
+        m = make_int2(wbias, wbias);
+        if (J.a.code) {
+          m.x += pb[ac[0]];
+          m.y += pb[ac[1]];
+        } else {
+#pragma unroll
+          for (int x = 0; x < KS; x += 4) {
+            const int4 v = *(const int4 *)(pb + x);
+            const int p[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int y = 0; y < 4; ++y) {
+              m.x += M24 ? __mul24(a[0][x + y], p[y]) : a[0][x + y] * p[y];
+              m.y += M24 ? __mul24(a[1][x + y], p[y]) : a[1][x + y] * p[y];
+            }
+          }
+        }
+      }
+      mm[(int64_t)q * 64] = m;
+    }
+    __syncthreads();
+  }
 }
+
+// wave_shr:1 (lane l takes lane l - 1's value, lane 0 keeps `old`).
 __device__ __forceinline__ int64_t shr_lane(int64_t old, int64_t v) {
   const int32_t lo = __builtin_amdgcn_update_dpp((int32_t)old, (int32_t)v, 0x138, 0xf, 0xf, false);
   const int32_t hi = __builtin_amdgcn_update_dpp((int32_t)(old >> 32), (int32_t)(v >> 32), 0x138, 0xf, 0xf, false);
   return ((int64_t)hi << 32) | (uint32_t)lo;
 }
 
-template <typename T>
-struct JoinNeg;
-template <>
-struct JoinNeg<int32_t> { static constexpr int32_t v = -(1 << 29); };
-template <>
-struct JoinNeg<int64_t> { static constexpr int64_t v = INT64_MIN / 4; };
+// A strip of a join: scores from memory, read a block ahead.
+struct JoinIO : StripGroupIO {
+  static constexpr bool SLOTS = false;
+  const int2 *ms;   // this lane's, 64 a step
+  int blocks;
+  int2 pre[2][4];   // the next block's halves
 
-// Index of the match score of cell (i + 1, j + 1) (0-based i, j) in the order
-// a join's sweep reads them: [strip][step][lane][row], step t = j + lane.
-__device__ __forceinline__ int64_t join_m_at(int i, int j, int JR, int NST) {
-  const int RS = 64 * JR, l = (i % RS) / JR;
-  return (((int64_t)(i / RS) * NST + j + l) * 64 + l) * JR + (i % JR);
-}
-
-// PB of B's columns from their residue counts, in place, a thread per
-// column: PB[j][x] = sum_y S(x, y) cntB[j][y] (K x K per column, which the
-// host used to spend most of a level's preparation on).
-__global__ __launch_bounds__(256) void msa_pb_kernel(int32_t *pb, int64_t rows, const int8_t *S, int K) {
-  __shared__ int32_t st[KS * KS];  // S(x, y) at [x][y], zero beyond K
-  for (int e = threadIdx.x; e < KS * KS; e += blockDim.x) {
-    const int x = e / KS, y = e % KS;
-    st[e] = (x < K && y < K) ? (int32_t)S[x * K + y] : 0;
-  }
-  __syncthreads();
-  const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= rows) return;
-  int32_t *row = pb + j * KS;
-  int32_t c[KS];
+  __device__ __forceinline__ void load(int b, int half) {
+    const int2 *p = ms + (int64_t)(8 * (b < blocks ? b : blocks - 1) + 4 * half) * 64;
 #pragma unroll
-  for (int y = 0; y < KS; ++y) c[y] = y < K ? row[y] : 0;
-  for (int x = 0; x < K; ++x) {
-    int32_t v = 0;
-#pragma unroll
-    for (int y = 0; y < KS; ++y) v += c[y] * st[x * KS + y];
-    row[x] = v;
+    for (int q = 0; q < 4; ++q) pre[half][q] = p[q * 64];
   }
-}
-
-// Every join's match scores M(i, j) = cntA[i] . PB[j], tile by tile over
-// the whole GPU (a join's own workgroup would compute them on one CU): a
-// workgroup takes 64 rows x 64 columns of one join, stages their counts and
-// PB rows in LDS, and each thread scores 16 cells.  Tiles: (join, tile index).
-__global__ __launch_bounds__(256) void msa_scores_kernel(const JoinJob *jobs, const int2 *tiles, const int32_t *cnt,
-                                                         const int32_t *pb, int32_t *mbuf, int JR) {
-  __shared__ int32_t ca[64 * KS], pbs[64 * KS];
-  const int2 tl = tiles[blockIdx.x];
-  const JoinJob J = jobs[tl.x];
-  const int ncb = (J.lb + 63) / 64, i0 = (tl.y / ncb) * 64, j0 = (tl.y % ncb) * 64;
-  const int ni = J.la - i0 < 64 ? J.la - i0 : 64, nj = J.lb - j0 < 64 ? J.lb - j0 : 64;
-  for (int x = threadIdx.x; x < 64 * KS; x += 256) {
-    ca[x] = x < ni * KS ? cnt[J.cnt_off + (int64_t)i0 * KS + x] : 0;
-    pbs[x] = x < nj * KS ? pb[J.pb_off + (int64_t)j0 * KS + x] : 0;
-  }
-  __syncthreads();
-  const int r = threadIdx.x & 63, NST = 8 * join_blocks(J.lb);
-  if (r >= ni) return;
-  int32_t a[KS];
+  __device__ __forceinline__ void scores(int b, int half, int (&v)[4][JR]) {
 #pragma unroll
-  for (int x = 0; x < KS; ++x) a[x] = ca[r * KS + x];
-  int32_t *mm = mbuf + J.m_off;
-  for (int c = threadIdx.x >> 6; c < nj; c += 4) {
-    const int32_t *pj = pbs + c * KS;
-    int32_t m = 0;
-#pragma unroll
-    for (int x = 0; x < KS; ++x) m += a[x] * pj[x];
-    mm[join_m_at(i0 + r, j0 + c, JR, NST)] = m;
+    for (int q = 0; q < 4; ++q) {
+      v[q][0] = pre[half][q].x;
+      v[q][1] = pre[half][q].y;
+    }
+    load(b + 1, half);
   }
-}
+};
 
-// JR: DP rows per lane, the fewest that cover the level's longest row
-// profile in one strip per wave where possible; T: int32_t when every join of
-// the level keeps its values within +-2^28, else int64_t.
-template <int JR, typename T>
-__global__ __launch_bounds__(JT) void msa_join_kernel(JoinArgs A) {
-  extern __shared__ __align__(16) uint8_t jlds[];  // ring H[lb + 2], F[lb + 2] (T)
-  __shared__ uint8_t tile[TW * TW];
-  __shared__ int32_t walk[4];                      // i, j, state, finished
-  __shared__ int32_t prog[8];                      // strip s publishes ((s + 1) << 20) | columns stored
-  constexpr T NEG = JoinNeg<T>::v;
-  const JoinJob J = A.jobs[blockIdx.x];
-  const int la = J.la, lb = J.lb, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const T go = (T)((int64_t)A.open * J.w), ge = (T)((int64_t)A.ext * J.w);
-  constexpr int RS = 64 * JR;  // DP rows per strip
-  const int S = (la + RS - 1) / RS, NB = join_blocks(lb);
-  T *ringH = (T *)jlds, *ringF = ringH + (lb + 2);
-  const int32_t *mm = A.mbuf + J.m_off;
-  uint8_t *tb = A.tb + J.tb_off;
-  if (tid < 8) prog[tid] = 0;
+// LDS words of the sync area: a progress counter per wave, then as in StripGroupIO.
+enum { JS_PROG = 0, JS_STATUS = 16, JS_READY = 17, JS_RUNS = 18, JS_ZERO = 32, JS_EDGE = 48, JS_WORDS = 64 };
 
-  // (the match scores were written by msa_scores_kernel, launched before)
-  const int NST = 8 * NB;  // steps per strip
-  __syncthreads();         // prog
-
-  // ---- the DP, strip by strip on each wave.
-  for (int s = wave; s < S; s += JW) {
-    const int i0 = s * RS + lane * JR + 1;  // this lane's first row
-    T Hl[JR], El[JR];                       // H(i, j - 1), E(i, j - 1)
+// The strips of a join in int64, plain recurrence: H, E, F with a column test
+// a step; direction codes as strip.h's.
+__device__ __forceinline__ void join_sweep_wide(const JoinArgs &A, const JoinJob &J, int64_t *ringH, int32_t *sy,
+                                                int W) {
+  constexpr int64_t NEG = INT64_MIN / 4;
+  const int la = J.a.len, lb = J.b.len, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t go = A.open * J.w, ge = A.ext * J.w;
+  const int S = join_strips(la), NST = join_steps(lb);
+  int64_t *ringF = ringH + (lb + 2);
+  for (int s = wave; s < S; s += W) {
+    const int i0 = s * JRS + lane * JR + 1;  // this lane's first row
+    int64_t Hl[JR], El[JR];                  // H(i, j - 1), E(i, j - 1)
 #pragma unroll
     for (int k = 0; k < JR; ++k) {
-      Hl[k] = go + (T)(i0 + k - 1) * ge;  // H(i, 0)
+      Hl[k] = go + (i0 + k - 1) * ge;  // H(i, 0)
       El[k] = NEG;
     }
-    T hd0 = i0 == 1 ? (T)0 : go + (T)(i0 - 2) * ge;  // H(i0 - 1, j - 1) for the next column: H(i0 - 1, 0)
-    T Hbot = 0, Fbot = NEG;                           // this lane's last row at its last column
-    const bool writer = lane == 63 && s + 1 < S;       // stores the strip's last row for strip s + 1
-    // match scores, MD steps ahead (one step ahead left every step waiting
-    // on its load); cells outside the pair read slots nobody wrote, and
-    // those steps are masked
-    constexpr int MD = 4;
-    int32_t mring[MD][JR];
-    const int32_t *ms = mm + ((int64_t)s * NST * 64 + lane) * JR;
-    auto load_m = [&](int t, int32_t (&m)[JR]) {
-      const int tt = t < NST ? t : NST - 1;
-      const int32_t *src = ms + (int64_t)tt * 64 * JR;
-      if constexpr (JR == 2) {
-        const int2 v = *(const int2 *)src;
-        m[0] = v.x; m[1] = v.y;
-      } else {
-#pragma unroll
-        for (int k = 0; k < JR; k += 4) {
-          const int4 v = *(const int4 *)(src + k);
-          m[k] = v.x; m[k + 1] = v.y; m[k + 2] = v.z; m[k + 3] = v.w;
-        }
-      }
-    };
-#pragma unroll
-    for (int d = 0; d < MD; ++d) load_m(d, mring[d]);
-    for (int b = 0; b < NB; ++b) {
-      // strip s - 1 must have stored the ring up to this block's last column
-      if (s > 0) {
-        const int need = (s << 20) | min(8 * b + 8, lb);
+    int64_t hd0 = i0 == 1 ? 0 : go + (i0 - 2) * ge;  // H(i0 - 1, j - 1) for the next column: H(i0 - 1, 0)
+    int64_t Hbot = 0, Fbot = NEG;                    // this lane's last row at its last column
+    const bool writer = lane == 63 && s + 1 < S;     // stores the strip's last row for strip s + 1
+    const int2 *ms = (const int2 *)(A.mbuf + J.m_off) + (int64_t)s * NST * 64 + lane;
+    uint32_t *tb = A.tb + J.tb_off + (int64_t)s * (NST / 4) * 64 + lane;
+    for (int b = 0; b < NST / 8; ++b) {
+      if (s > 0) {  // strip s - 1 must have stored the ring up to this block's last column
+        const int need = ((s - 1) / W + 1) << 20 | min(8 * b + 8, lb);
         int spins = 0;
-        while (__hip_atomic_load(&prog[(s - 1) & 7], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < need) {
+        while (__hip_atomic_load(&sy[JS_PROG + (s - 1) % W], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < need) {
           if (++spins > A.spin_limit) {
-            if (lane == 0) atomicOr(A.err, 1);
+            if (lane == 0) atomicOr(&sy[JS_STATUS], 1);
             break;
           }
           __builtin_amdgcn_s_sleep(1);
         }
       }
-      // lane 0's top inputs of the block's 8 steps: row 0 or the ring, read
-      // once the progress allows (not a dependent LDS read per step)
-      T tops[8], topfs[8];
-#pragma unroll
+      uint32_t acc = 0;
       for (int q = 0; q < 8; ++q) {
-        const int c = 8 * b + q + 1;  // lane 0's column at step 8b + q
-        if (s == 0) {
-          tops[q] = go + (T)(c - 1) * ge;  // H(0, c)
-          topfs[q] = NEG;
-        } else {
-          tops[q] = c <= lb ? ringH[c] : (T)0;
-          topfs[q] = c <= lb ? ringF[c] : NEG;
+        const int t = 8 * b + q, j = t - lane + 1, c = t + 1;  // c: lane 0's column
+        int64_t top = go + (c - 1) * ge, topf = NEG;           // row 0, or the ring
+        if (s > 0) {
+          top = c <= lb ? ringH[c] : 0;
+          topf = c <= lb ? ringF[c] : NEG;
         }
-      }
-      uint32_t codes[8][JR / 4 > 0 ? JR / 4 : 1];  // direction bytes of the block's steps, packed
-#pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const int t = 8 * b + q, j = t - lane + 1;
-        int32_t mcur[JR];
-#pragma unroll
-        for (int k = 0; k < JR; ++k) mcur[k] = mring[q % MD][k];
-        load_m(t + MD, mring[q % MD]);
-        // lane 0's top: row 0 or the ring; the others: the lane above's bottom row
-        const T Hup0 = shr_lane(tops[q], Hbot), Fup0 = shr_lane(topfs[q], Fbot);
-        uint32_t bytes = 0;
+        const int64_t Hup0 = shr_lane(top, Hbot), Fup0 = shr_lane(topf, Fbot);
+        const int2 m2 = ms[(int64_t)t * 64];
+        uint32_t nib = 0;
         if (j >= 1 && j <= lb) {
-          T hup = Hup0, fup = Fup0, hd = hd0;
+          int64_t hup = Hup0, fup = Fup0, hd = hd0;
 #pragma unroll
           for (int k = 0; k < JR; ++k) {
-            const T eo = Hl[k] + go, ee = El[k] + ge;
-            const bool eb = ee > eo;
-            const T E = eb ? ee : eo;
-            const T fo = hup + go, fe = fup + ge;
-            const bool fb = fe > fo;
-            const T F = fb ? fe : fo;
-            T h = hd + (T)mcur[k];
-            int src = 0;
-            if (E > h) { h = E; src = 1; }
-            if (F > h) { h = F; src = 2; }
+            const int64_t eo = Hl[k] + go, ee = El[k] + ge, fo = hup + go, fe = fup + ge;
+            const int64_t E = ee > eo ? ee : eo, F = fe > fo ? fe : fo, d = hd + (k ? m2.y : m2.x);
+            const int64_t h = max(d, max(E, F));
+            nib = nib << 4 | (uint32_t)((ee > eo) | (fe > fo) << 1 | (d < h) << 2 | (E < F) << 3);
             hd = Hl[k];
             Hl[k] = h;
             El[k] = E;
             hup = h;
             fup = F;
-            bytes |= (uint32_t)(src | ((int)eb << 2) | ((int)fb << 3)) << (8 * (k & 3));
-            if ((k & 3) == 3 || k == JR - 1) {
-              codes[q][k >> 2] = bytes;
-              bytes = 0;
-            }
           }
           Hbot = hup;
           Fbot = fup;
@@ -293,85 +268,152 @@ __global__ __launch_bounds__(JT) void msa_join_kernel(JoinArgs A) {
             ringH[j] = hup;
             ringF[j] = fup;
           }
-        } else {
-#pragma unroll
-          for (int k = 0; k < (JR / 4 > 0 ? JR / 4 : 1); ++k) codes[q][k] = 0;
         }
-      }
-      // the block's direction bytes: 8 steps x JR rows, contiguous per lane
-      uint8_t *dst = tb + ((((int64_t)s * NB + b) * 64 + lane) * 8) * JR;
-      if constexpr (JR >= 4) {
-#pragma unroll
-        for (int q = 0; q < 8; ++q)
-#pragma unroll
-          for (int k = 0; k < JR / 4; ++k) ((uint32_t *)dst)[q * (JR / 4) + k] = codes[q][k];
-      } else {
-#pragma unroll
-        for (int q = 0; q < 8; ++q) ((uint16_t *)dst)[q] = (uint16_t)codes[q][0];
+        acc = acc << 8 | nib;
+        if ((q & 3) == 3) tb[(int64_t)(t / 4) * 64] = acc;
       }
       // publish the ring columns stored so far (the writer lane's column)
       if (s + 1 < S) {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         const int done = min(max(8 * b + 8 - 63, 0), lb);
-        if (lane == 63) __hip_atomic_store(&prog[s & 7], ((s + 1) << 20) | done, __ATOMIC_RELEASE,
+        if (lane == 63) __hip_atomic_store(&sy[JS_PROG + wave], (s / W + 1) << 20 | done, __ATOMIC_RELEASE,
                                            __HIP_MEMORY_SCOPE_WORKGROUP);
       }
     }
   }
-  __syncthreads();
-
-  // ---- walk back from (la, lb): the pairwise state machine (H, E 'D',
-  // F 'I').  The workgroup stages the TW x TW tile of direction bytes ending
-  // at the walk's cell in LDS; thread 0 walks it until the walk leaves it.
-  uint8_t *ops = A.ops + J.ops_off;
-  if (tid == 0) { walk[0] = la; walk[1] = lb; walk[2] = 0; walk[3] = 0; }
-  int k = 0;  // ops written (thread 0)
-  __syncthreads();
-  for (;;) {
-    const int wi = walk[0], wj = walk[1];
-    if (walk[3]) break;
-    const int i0 = wi - (TW - 1) > 1 ? wi - (TW - 1) : 1, j0 = wj - (TW - 1) > 1 ? wj - (TW - 1) : 1;
-    const int ni = wi - i0 + 1, nj = wj - j0 + 1;
-    if (wi >= 1 && wj >= 1)
-      for (int c = tid; c < ni * nj; c += JT) {
-        const int r = c / nj, q = c - r * nj;
-        tile[r * TW + q] = tb[join_tb_at(i0 + r, j0 + q, JR, NB)];
-      }
-    __syncthreads();
-    if (tid == 0) {
-      int i = wi, j = wj, state = walk[2];
-      bool fin = false;
-      for (;;) {
-        if (i == 0) { while (j-- > 0) ops[k++] = 'D'; fin = true; break; }
-        if (j == 0) { while (i-- > 0) ops[k++] = 'I'; fin = true; break; }
-        if (i < i0 || j < j0) break;  // left the tile
-        const int code = tile[(i - i0) * TW + (j - j0)];
-        if (state == 0) {
-          const int s = code & 3;
-          if (s == 0) { ops[k++] = 'M'; --i; --j; }
-          else state = s;
-        } else if (state == 1) {
-          ops[k++] = 'D';
-          if (!(code & 4)) state = 0;
-          --j;
-        } else {
-          ops[k++] = 'I';
-          if (!(code & 8)) state = 0;
-          --i;
-        }
-      }
-      walk[0] = i; walk[1] = j; walk[2] = state; walk[3] = fin;
-    }
-    __syncthreads();
-  }
-  if (tid == 0) A.nops[blockIdx.x] = k;
 }
 
-struct Profile {
-  std::vector<int32_t> rows;  // sequence ids
-  int32_t len = 0;
-  std::vector<int16_t> cell;  // rows x len: code, or -1 for a gap
+// A join: the DP, the walk back, the merged columns.  WIDE: values in int64.
+template <bool WIDE>
+__global__ __launch_bounds__(64 * JWMAX) void msa_join_kernel(JoinArgs A) {
+  extern __shared__ __align__(16) uint8_t jlds[];  // the strips' ring of bottom rows
+  __shared__ __align__(16) int32_t sy[JS_WORDS];
+  __shared__ uint32_t win[StripWindow<JR>::WL * StripWindow<JR>::WD];
+  const JoinJob &J = A.jobs[blockIdx.x];
+  const int la = J.a.len, lb = J.b.len, tid = threadIdx.x, lane = tid & 63, nthr = blockDim.x, W = nthr >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int S = join_strips(la), T = join_steps(lb);
+  const int go = (int)(A.open * J.w), ge = (int)(A.ext * J.w);  // (not WIDE: they fit)
+  uint32_t *tb = A.tb + J.tb_off;
+  if (tid < JS_WORDS) sy[tid] = tid == JS_READY ? 0x7fffffff : tid >= JS_EDGE ? 2 * (go - ge) : 0;
+  __syncthreads();
+
+  // ---- the DP: strip s on wave s % W; every strip stores its bottom row over
+  // the one it read, 63 columns behind
+  if constexpr (WIDE) {
+    join_sweep_wide(A, J, (int64_t *)jlds, sy, W);
+  } else {
+    int2 *const ring = (int2 *)jlds;
+    for (int s = wave; s < S; s += W) {
+      JoinIO io;
+      io.ms = (const int2 *)(A.mbuf + J.m_off) + (int64_t)s * T * 64 + lane;
+      io.blocks = T / 8;
+      io.load(0, 0);
+      io.load(0, 1);
+      io.status = sy + JS_STATUS;
+      io.pin = sy + (s ? JS_PROG + (s - 1) % W : JS_READY);
+      io.pout = sy + JS_PROG + wave;
+      io.rin = lane ? (int2 *)(sy + JS_ZERO) : s ? ring + 64 : (int2 *)(sy + JS_EDGE);
+      io.rin_step = lane == 0 && s ? 8 : 0;
+      io.rout = ring;
+      io.need0 = s ? ((s - 1) / W + 1) << 20 : 0;
+      io.s = s / W;
+      io.cols = T - 63;
+      io.spin_limit = A.spin_limit;
+      io.gave_up = 1;
+      io.pl = tb + (int64_t)s * (T / 4) * 64 + lane;
+      io.pl_step = 64;
+      StripEnd end;
+      strip_sweep<JR, false>(io, s, s + 1 == S, la, lb, T, go, ge, end);
+    }
+  }
+  __syncthreads();  // every code of the workgroup is visible to it
+
+  // ---- walk back from (la, lb), a run at a time (wave 0)
+  const int cap = la + lb + 2;
+  uint32_t *const rend = A.runs + J.run_off + cap;
+  if (wave == 0) {
+    WaveRuns rw;
+    rw.end = rend;
+    rw.cap = cap;
+    StripWindow<JR> src{tb, win, T, -1, -1};
+    int i = la, j = lb, state = 0, h = 0, steps = 0;
+    src.refill(i, j);
+    const int how = wave_walk<WALK_GLOBAL>(src, rw, i, j, state, h, go, ge, la + lb, steps);
+    if (how != WALK_GAVE_UP) {
+      if (i == 0 && j > 0) rw.emit(1, j);
+      if (j == 0 && i > 0) rw.emit(2, i);
+    }
+    const bool ok = rw.finish() && how != WALK_GAVE_UP;
+    if (lane == 0) {
+      sy[JS_RUNS] = ok ? rw.n : 0;
+      if (!ok) atomicOr(&sy[JS_STATUS], 2);
+    }
+  }
+  __syncthreads();
+
+  // ---- the merged columns' sources and both sides' maps, a run to a wave
+  const int nr = sy[JS_RUNS];
+  const uint32_t *runs = rend - nr;
+  int2 *const src = A.src + J.src_off;
+  int x0 = 0, a0 = 0, b0 = 0;  // columns before run `base`
+  for (int base = 0; base < nr; base += 64) {
+    const uint32_t v = base + lane < nr ? runs[base + lane] : 0;
+    const int op = v & 3, len = (int)(v >> 2);
+    int na = op == 1 ? 0 : len, nb = op == 2 ? 0 : len, nx = len;  // inclusive sums over the lanes
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int oa = __shfl_up(na, d, 64), ob = __shfl_up(nb, d, 64), ox = __shfl_up(nx, d, 64);
+      if (lane >= d) { na += oa; nb += ob; nx += ox; }
+    }
+    for (int k = wave; k < min(64, nr - base); k += W) {
+      const int o = __builtin_amdgcn_readlane(op, k), l = __builtin_amdgcn_readlane(len, k);
+      const int x = x0 + __builtin_amdgcn_readlane(nx, k) - l;
+      const int ia = a0 + __builtin_amdgcn_readlane(na, k) - (o == 1 ? 0 : l);
+      const int ib = b0 + __builtin_amdgcn_readlane(nb, k) - (o == 2 ? 0 : l);
+      for (int e = lane; e < l; e += 64) {
+        src[x + e] = make_int2(o == 1 ? -1 : ia + e, o == 2 ? -1 : ib + e);
+        if (o != 1) J.a.map[ia + e] = x + e;
+        if (o != 2) J.b.map[ib + e] = x + e;
+      }
+    }
+    x0 += __builtin_amdgcn_readlane(nx, 63);
+    a0 += __builtin_amdgcn_readlane(na, 63);
+    b0 += __builtin_amdgcn_readlane(nb, 63);
+  }
+  if (tid == 0) {
+    A.nops[blockIdx.x] = x0;
+    if (sy[JS_STATUS]) atomicOr(A.err, sy[JS_STATUS]);
+  }
+  if (!J.out) return;
+  __syncthreads();
+  for (int64_t e = tid; e < (int64_t)x0 * CI; e += nthr) {
+    const int x = (int)(e / CI), y = (int)(e % CI);
+    const int2 s = src[x];
+    int4 v = make_int4(0, 0, 0, 0);
+    if (s.x >= 0) v = join_row(J.a, A.leaf, s.x)[y];
+    if (s.y >= 0) {
+      const int4 u = join_row(J.b, A.leaf, s.y)[y];
+      v.x += u.x; v.y += u.y; v.z += u.z; v.w += u.w;
+    }
+    J.out[e] = v;
+  }
+}
+
+// Every residue's column in the root: up the tree through the joins' maps.
+struct MsaNode {
+  const int32_t *map;  // the node's columns in its parent's
+  int32_t parent;      // -1: the root
 };
+__global__ __launch_bounds__(256) void msa_columns_kernel(const MsaNode *nodes, const int64_t *off, int32_t *cols,
+                                                          int chunks) {
+  const int s = blockIdx.x / chunks;
+  const int64_t k = (int64_t)(blockIdx.x % chunks) * 256 + threadIdx.x;
+  if (k >= off[s + 1] - off[s]) return;
+  int c = (int)k;
+  for (int v = s; nodes[v].parent >= 0; v = nodes[v].parent) c = nodes[v].map[c];
+  cols[off[s] + k] = c;
+}
 
 }  // namespace
 
@@ -474,192 +516,165 @@ int ta_msa(ta_ctx *ctx, const ta_params *p, const char *const *seqs, const int32
 
   tr.mark("upgma");
   // 3. joins level by level
-  std::vector<Profile> prof(nc);
-  for (int32_t s = 0; s < nseq; ++s) {
-    prof[s].rows = {s};
-    prof[s].len = lens[s];
-    prof[s].cell.assign(codes.begin() + off[s], codes.begin() + off[s + 1]);
-  }
   hipStream_t st = ctx->stream;
-  // The substitution table on the device (the PB kernel reads it).
-  int8_t *d_S = (int8_t *)device_alloc((size_t)K * K);
-  if (!d_S || hipMemcpy(d_S, S, (size_t)K * K, hipMemcpyHostToDevice) != hipSuccess) {
-    device_free(d_S);
-    return TA_E_DEVICE;
+  std::vector<void *> held;  // device blocks of the whole call
+  auto hold = [&](size_t bytes) {
+    void *d = device_alloc(std::max<size_t>(1, bytes));
+    if (d) held.push_back(d);
+    return d;
+  };
+  // A level's merged columns, given back once every cluster in it is joined.
+  struct Level {
+    void *p;
+    int32_t live;
+  };
+  std::vector<Level> levels;
+  struct Free {
+    std::vector<void *> &held;
+    std::vector<Level> &levels;
+    ~Free() {
+      for (void *d : held) device_free(d);
+      for (const Level &l : levels) device_free(l.p);
+    }
+  } free_all{held, levels};
+  // Rows of single residues, and the sequences' codes.
+  std::vector<int32_t> hleaf((size_t)K * 2 * KS, 0);
+  for (int32_t x = 0; x < K; ++x) {
+    hleaf[(size_t)x * 2 * KS + x] = 1;
+    for (int32_t y = 0; y < K; ++y) hleaf[(size_t)x * 2 * KS + KS + y] = S[y * K + x];
   }
-  struct FreeS {
-    int8_t *p;
-    ~FreeS() { device_free(p); }
-  } free_s{d_S};
-  // The levels' count tables, kept by the calling thread between levels and
-  // calls: fresh multi-MB vectors pay a page fault per 4 KB.
-  static thread_local std::vector<int32_t> tl_cnt, tl_pb;
-  std::vector<int32_t> &hcnt = tl_cnt, &hpb = tl_pb;
+  int4 *d_leaf = (int4 *)hold(hleaf.size() * sizeof(int32_t));
+  uint8_t *d_codes = (uint8_t *)hold((size_t)off[nseq]);
+  int32_t *d_err = (int32_t *)hold(sizeof(int32_t));
+  if (!d_leaf || !d_codes || !d_err) return TA_E_NOMEM;
+  if (hipMemsetAsync(d_err, 0, sizeof(int32_t), st) ||
+      hipMemcpyAsync(d_leaf, hleaf.data(), hleaf.size() * sizeof(int32_t), hipMemcpyHostToDevice, st) ||
+      hipMemcpyAsync(d_codes, codes.data(), (size_t)off[nseq], hipMemcpyHostToDevice, st) || hipStreamSynchronize(st))
+    return TA_E_DEVICE;
+  struct Cluster {
+    int32_t len = 0, rows = 1, level = -1;  // level: index into `levels`, -1 a sequence
+    const int4 *tab = nullptr;
+  };
+  std::vector<Cluster> cl(nc);
+  std::vector<MsaNode> nodes(nc, MsaNode{nullptr, -1});
+  for (int32_t s = 0; s < nseq; ++s) cl[s].len = lens[s];
+  const int64_t gap_w = -((int64_t)p->gap_open + p->gap_extend);
   for (int32_t L = 1; L <= top; ++L) {
     std::vector<int32_t> ts;
     for (int32_t t = 0; t + 1 < nseq; ++t)
       if (level[nseq + t] == L) ts.push_back(t);
-    std::vector<JoinJob> jobs(ts.size());
-    int64_t tb_total = 0, ops_total = 0, m_total = 0, cnt_total = 0, pb_total = 0;
-    int max_la = 0, max_lb = 0;
+    const int32_t nj = (int32_t)ts.size();
+    std::vector<JoinJob> jobs(nj);
+    int64_t tb_total = 0, run_total = 0, col_total = 0, m_total = 0;
+    int32_t max_lb = 0, strips = 0, tiles = 0;
     bool wide = false;  // some join's DP values need int64
-    for (size_t q = 0; q < ts.size(); ++q) {
-      max_la = std::max(max_la, prof[ja[ts[q]]].len);
-      max_lb = std::max(max_lb, prof[jb[ts[q]]].len);
-    }
-    // rows per lane: the fewest that give every wave of the join a strip
-    const int jr = max_la <= 2 * JT ? 2 : max_la <= 4 * JT ? 4 : JRMAX;
-    // sizes and offsets, then each join's counts and PB on the host threads
-    for (size_t q = 0; q < ts.size(); ++q) {
-      const Profile &PA = prof[ja[ts[q]]], &PB = prof[jb[ts[q]]];
+    bool m24 = true;    // every count and PB entry fits 24 bits
+    for (int32_t q = 0; q < nj; ++q) {
+      const Cluster &ca = cl[ja[ts[q]]], &cb = cl[jb[ts[q]]];
       JoinJob &J = jobs[q];
-      J.la = PA.len; J.lb = PB.len;
-      J.w = (int64_t)PA.rows.size() * (int64_t)PB.rows.size();
+      J.a = {ca.tab ? nullptr : d_codes + off[ja[ts[q]]], ca.tab, nullptr, ca.len};
+      J.b = {cb.tab ? nullptr : d_codes + off[jb[ts[q]]], cb.tab, nullptr, cb.len};
+      J.w = (int64_t)ca.rows * cb.rows;
       // joins whose column scores could leave int32
-      if (J.w > WMAX || (int64_t)PA.len * PB.len > INT32_MAX) return TA_E_INVALID;
-      // int32 DP when every value, and -2^29 plus a gap cost, stays clear of overflow
-      const int64_t step = std::max<int64_t>(max_abs_s, (int64_t)-p->gap_open - p->gap_extend) * J.w;
-      if ((int64_t)(J.la + J.lb + 2) * step >= (1ll << 28)) wide = true;
-      J.cnt_off = cnt_total;
-      cnt_total += (int64_t)PA.len * KS;
-      J.pb_off = pb_total;
-      pb_total += (int64_t)PB.len * KS;
-      J.m_off = m_total;  // the sweep's order: strips x steps x 64 lanes x jr rows (16-byte aligned)
-      m_total += ((int64_t)(PA.len + 64 * jr - 1) / (64 * jr)) * 8 * join_blocks(PB.len) * 64 * jr;
+      if (J.w > WMAX || (int64_t)ca.len * cb.len > INT32_MAX) return TA_E_INVALID;
+      const int64_t c = (int64_t)p->gap_open - p->gap_extend;
+      const int64_t reach = std::min(ca.len, cb.len) * (max_abs_s - 2ll * p->gap_extend) +
+                            (ca.len + cb.len + 2) * std::max<int64_t>(0, c) + 4 * (gap_w + max_abs_s);
+      if (reach >= (1ll << 30) / J.w) wide = true;
+      if (std::max(ca.rows, cb.rows) * max_abs_s >= (1 << 23)) m24 = false;
+      const int64_t S = join_strips(ca.len), T = join_steps(cb.len);
+      J.m_off = m_total;
+      m_total += S * T * 64 * JR;
       J.tb_off = tb_total;
-      tb_total += (((int64_t)(PA.len + 64 * jr - 1) / (64 * jr)) * join_blocks(PB.len) * 64 * 8 * jr + 15) & ~15ll;
-      J.ops_off = ops_total;
-      ops_total += PA.len + PB.len;
+      tb_total += S * (T / 4) * 64;
+      J.run_off = run_total;
+      run_total += ca.len + cb.len + 2;
+      J.src_off = col_total;
+      col_total += ca.len + cb.len;
+      max_lb = std::max(max_lb, cb.len);
+      strips = (int32_t)std::max<int64_t>(strips, S);
+      tiles = (int32_t)std::max<int64_t>(tiles, S * ((T + 63) / 64));
+    }
+    const bool root = L == top;
+    int32_t *d_map = (int32_t *)hold(sizeof(int32_t) * (size_t)col_total);
+    int4 *d_out = root ? nullptr : (int4 *)device_alloc(sizeof(int4) * CI * (size_t)col_total);
+    if (d_out) levels.push_back({d_out, nj});
+    for (int32_t q = 0; q < nj && d_map; ++q) {
+      JoinJob &J = jobs[q];
+      J.a.map = d_map + J.src_off;
+      J.b.map = J.a.map + J.a.len;
+      J.out = d_out ? d_out + J.src_off * CI : nullptr;
+      nodes[ja[ts[q]]] = {J.a.map, nseq + ts[q]};
+      nodes[jb[ts[q]]] = {J.b.map, nseq + ts[q]};
     }
     tr.mark("level sizes");
-    // each join's tables are cleared by the thread that fills them
-    if (hcnt.size() < (size_t)cnt_total) hcnt.resize((size_t)cnt_total);
-    if (hpb.size() < (size_t)pb_total) hpb.resize((size_t)pb_total);
-    // Column counts of both sides on the host threads, joins dealt in turn;
-    // PB (K x K per column of B) is made from B's counts on the GPU.
-    const int nthr = (int)std::min<size_t>(16, ts.size());
-    parallel_tasks(nthr, [&](int t) {
-      for (size_t q = (size_t)t; q < ts.size(); q += (size_t)nthr) {
-        const Profile &PA = prof[ja[ts[q]]], &PB = prof[jb[ts[q]]];
-        const JoinJob &J = jobs[q];
-        int32_t *ca = hcnt.data() + J.cnt_off, *cb = hpb.data() + J.pb_off;
-        std::fill(ca, ca + (size_t)PA.len * KS, 0);
-        std::fill(cb, cb + (size_t)PB.len * KS, 0);
-        for (size_t r = 0; r < PA.rows.size(); ++r)
-          for (int32_t i = 0; i < PA.len; ++i) {
-            const int c = PA.cell[r * PA.len + i];
-            if (c >= 0) ca[(size_t)i * KS + c] += 1;
-          }
-        for (size_t r = 0; r < PB.rows.size(); ++r)
-          for (int32_t j = 0; j < PB.len; ++j) {
-            const int c = PB.cell[r * PB.len + j];
-            if (c >= 0) cb[(size_t)j * KS + c] += 1;
-          }
-      }
-    });
-    tr.mark("level prep");
-    const size_t lds = (wide ? sizeof(int64_t) : sizeof(int32_t)) * 2 * (size_t)(max_lb + 2);
-    JoinJob *d_jobs = (JoinJob *)device_alloc(sizeof(JoinJob) * jobs.size());
-    int32_t *d_cnt = (int32_t *)device_alloc(sizeof(int32_t) * (size_t)std::max<int64_t>(1, cnt_total));
-    int32_t *d_pb = (int32_t *)device_alloc(sizeof(int32_t) * (size_t)std::max<int64_t>(1, pb_total));
-    int32_t *d_m = (int32_t *)device_alloc(sizeof(int32_t) * (size_t)std::max<int64_t>(1, m_total));
-    int32_t *d_err = (int32_t *)device_alloc(sizeof(int32_t));
-    uint8_t *d_tb = (uint8_t *)device_alloc((size_t)std::max<int64_t>(1, tb_total));
-    uint8_t *d_ops = (uint8_t *)device_alloc((size_t)std::max<int64_t>(1, ops_total));
-    int32_t *d_nops = (int32_t *)device_alloc(sizeof(int32_t) * jobs.size());
-    std::vector<uint8_t> hops((size_t)std::max<int64_t>(1, ops_total));
-    std::vector<int32_t> hnops(jobs.size());
+    std::vector<int32_t> hnops(nj);
     int32_t herr = 0;
-    rc = (d_jobs && d_cnt && d_pb && d_m && d_err && d_tb && d_ops && d_nops) ? TA_OK : TA_E_NOMEM;
-    if (!rc && hipMemsetAsync(d_err, 0, sizeof(int32_t), st) != hipSuccess) rc = TA_E_DEVICE;
-    if (!rc && (hipMemcpyAsync(d_jobs, jobs.data(), sizeof(JoinJob) * jobs.size(), hipMemcpyHostToDevice, st) ||
-                (cnt_total > 0 &&
-                 hipMemcpyAsync(d_cnt, hcnt.data(), sizeof(int32_t) * cnt_total, hipMemcpyHostToDevice, st)) ||
-                (pb_total > 0 &&
-                 hipMemcpyAsync(d_pb, hpb.data(), sizeof(int32_t) * pb_total, hipMemcpyHostToDevice, st))))
-      rc = TA_E_DEVICE;
+    JoinArgs a{};
+    JoinJob *d_jobs = (JoinJob *)device_alloc(sizeof(JoinJob) * nj);
+    a.jobs = d_jobs;
+    a.leaf = d_leaf;
+    a.mbuf = (int32_t *)device_alloc(sizeof(int32_t) * (size_t)m_total);
+    a.tb = (uint32_t *)device_alloc(sizeof(uint32_t) * (size_t)tb_total);
+    a.runs = (uint32_t *)device_alloc(sizeof(uint32_t) * (size_t)run_total);
+    a.src = (int2 *)device_alloc(sizeof(int2) * (size_t)col_total);
+    a.nops = (int32_t *)device_alloc(sizeof(int32_t) * nj);
+    a.err = d_err;
+    a.open = p->gap_open; a.ext = p->gap_extend;
+    a.spin_limit = 1 << 22;
+    rc = (d_map && (root || d_out) && d_jobs && a.mbuf && a.tb && a.runs && a.src && a.nops) ? TA_OK : TA_E_NOMEM;
     if (!rc) {
-      JoinArgs a;
-      a.jobs = d_jobs; a.cnt = d_cnt; a.pb = d_pb; a.mbuf = d_m; a.tb = d_tb; a.ops = d_ops;
-      a.nops = d_nops; a.err = d_err;
-      a.K = K; a.open = p->gap_open; a.ext = p->gap_extend;  // K <= KS
-      a.spin_limit = 1 << 22;
       (void)hipGetLastError();
+      if (hipMemcpyAsync(d_jobs, jobs.data(), sizeof(JoinJob) * nj, hipMemcpyHostToDevice, st)) rc = TA_E_DEVICE;
       // the match scores over the whole GPU, then the joins
-      std::vector<int2> tiles;
-      for (size_t q = 0; q < jobs.size(); ++q) {
-        const int nt = ((jobs[q].la + 63) / 64) * ((jobs[q].lb + 63) / 64);
-        for (int t = 0; t < nt; ++t) tiles.push_back(make_int2((int)q, t));
-      }
-      int2 *d_tiles = (int2 *)device_alloc(sizeof(int2) * tiles.size());
-      if (!d_tiles || hipMemcpyAsync(d_tiles, tiles.data(), sizeof(int2) * tiles.size(), hipMemcpyHostToDevice, st))
-        rc = TA_E_DEVICE;
-      const int64_t pb_rows = pb_total / KS;
-      if (!rc && pb_rows > 0)
-        hipLaunchKernelGGL(msa_pb_kernel, dim3((unsigned)((pb_rows + 255) / 256)), dim3(256), 0, st, d_pb, pb_rows,
-                           d_S, K);
-      if (!rc) hipLaunchKernelGGL(msa_scores_kernel, dim3((unsigned)tiles.size()), dim3(256), 0, st, d_jobs, d_tiles, d_cnt,
-                                  d_pb, d_m, jr);
-      void (*kern)(JoinArgs) =
-          wide ? (jr == 2 ? msa_join_kernel<2, int64_t> : jr == 4 ? msa_join_kernel<4, int64_t> : msa_join_kernel<JRMAX, int64_t>)
-               : (jr == 2 ? msa_join_kernel<2, int32_t> : jr == 4 ? msa_join_kernel<4, int32_t> : msa_join_kernel<JRMAX, int32_t>);
-      if (!rc) hipLaunchKernelGGL(kern, dim3((unsigned)jobs.size()), dim3(JT), lds, st, a);
+      const dim3 grid((unsigned)nj, (unsigned)std::min(tiles, 65535));
+      if (!rc) hipLaunchKernelGGL(m24 ? msa_scores_kernel<true> : msa_scores_kernel<false>, grid, dim3(256), 0, st, a,
+                                  wide ? 0 : -p->gap_open - p->gap_extend, wide ? 0 : p->gap_extend - p->gap_open);
+      const size_t lds = wide ? 2 * sizeof(int64_t) * (size_t)(max_lb + 2) : sizeof(int2) * (size_t)join_ring(max_lb);
+      if (!rc) hipLaunchKernelGGL(wide ? msa_join_kernel<true> : msa_join_kernel<false>, dim3((unsigned)nj),
+                                  dim3(64 * std::min(strips, JWMAX)), lds, st, a);
       if (rc || hipGetLastError() != hipSuccess ||
-          hipMemcpyAsync(hops.data(), d_ops, (size_t)ops_total, hipMemcpyDeviceToHost, st) ||
-          hipMemcpyAsync(hnops.data(), d_nops, sizeof(int32_t) * jobs.size(), hipMemcpyDeviceToHost, st) ||
-          hipMemcpyAsync(&herr, d_err, sizeof(int32_t), hipMemcpyDeviceToHost, st) ||
-          hipStreamSynchronize(st))
+          hipMemcpyAsync(hnops.data(), a.nops, sizeof(int32_t) * nj, hipMemcpyDeviceToHost, st) ||
+          hipMemcpyAsync(&herr, d_err, sizeof(int32_t), hipMemcpyDeviceToHost, st) || hipStreamSynchronize(st))
         rc = TA_E_DEVICE;
-      (void)hipStreamSynchronize(st);
-      device_free(d_tiles);
+      if (rc) (void)hipStreamSynchronize(st);
       if (!rc && herr) {
-        fprintf(stderr, "tweakalign: a wait on another wave's progress gave up (msa join)\n");
+        fprintf(stderr, "tweakalign: %s gave up (msa join)\n", herr & 1 ? "a wait on another wave's progress" : "a walk");
         rc = TA_E_DEVICE;
       }
     }
-    device_free(d_jobs); device_free(d_cnt); device_free(d_pb); device_free(d_m); device_free(d_err);
-    device_free(d_tb); device_free(d_ops); device_free(d_nops);
+    device_free(d_jobs); device_free(a.mbuf); device_free(a.tb); device_free(a.runs); device_free(a.src);
+    device_free(a.nops);
     if (rc) return rc;
-    tr.mark("level gpu");
-    // apply each join's ops (walk order: read backwards)
-    for (size_t q = 0; q < ts.size(); ++q) {
-      const int32_t t = ts[q], c = nseq + t;
-      Profile &PA = prof[ja[t]], &PB = prof[jb[t]];
-      const int32_t n = hnops[q];
-      const uint8_t *o = hops.data() + jobs[q].ops_off;
-      Profile C;
-      C.rows = PA.rows;
-      C.rows.insert(C.rows.end(), PB.rows.begin(), PB.rows.end());
-      C.len = n;
-      C.cell.assign(C.rows.size() * (size_t)n, -1);
-      const size_t na = PA.rows.size(), nb = PB.rows.size();
-      int32_t ia = 0, jbb = 0;
-      for (int32_t x = 0; x < n; ++x) {
-        const uint8_t op = o[n - 1 - x];
-        if (op != 'D') {
-          for (size_t r = 0; r < na; ++r) C.cell[r * n + x] = PA.cell[r * PA.len + ia];
-          ++ia;
+    for (int32_t q = 0; q < nj; ++q) {
+      const int32_t t = ts[q];
+      for (const int32_t child : {ja[t], jb[t]})
+        if (cl[child].level >= 0 && --levels[cl[child].level].live == 0) {
+          device_free(levels[cl[child].level].p);
+          levels[cl[child].level].p = nullptr;
         }
-        if (op != 'I') {
-          for (size_t r = 0; r < nb; ++r) C.cell[(na + r) * n + x] = PB.cell[r * PB.len + jbb];
-          ++jbb;
-        }
-      }
-      prof[c] = std::move(C);
-      PA = Profile();
-      PB = Profile();
+      cl[nseq + t] = {hnops[q], cl[ja[t]].rows + cl[jb[t]].rows, root ? -1 : (int32_t)levels.size() - 1, jobs[q].out};
     }
-    tr.mark("level apply");
+    tr.mark("level gpu");
   }
 
   // 4. every residue's column
-  const Profile &F = prof[nc - 1];
-  *alen = F.len;
-  for (size_t r = 0; r < F.rows.size(); ++r) {
-    const int32_t s = F.rows[r];
-    int64_t k = off[s];
-    for (int32_t x = 0; x < F.len; ++x)
-      if (F.cell[r * F.len + x] >= 0) cols[k++] = x;
-  }
+  *alen = cl[nc - 1].len;
+  int32_t *d_cols = (int32_t *)hold(sizeof(int32_t) * (size_t)off[nseq]);
+  int64_t *d_off = (int64_t *)hold(sizeof(int64_t) * (nseq + 1));
+  MsaNode *d_nodes = (MsaNode *)hold(sizeof(MsaNode) * nc);
+  if (!d_cols || !d_off || !d_nodes) return TA_E_NOMEM;
+  const int32_t chunks = (*std::max_element(lens, lens + nseq) + 255) / 256;
+  (void)hipGetLastError();
+  if (hipMemcpyAsync(d_off, off.data(), sizeof(int64_t) * (nseq + 1), hipMemcpyHostToDevice, st) ||
+      hipMemcpyAsync(d_nodes, nodes.data(), sizeof(MsaNode) * nc, hipMemcpyHostToDevice, st))
+    return TA_E_DEVICE;
+  hipLaunchKernelGGL(msa_columns_kernel, dim3((unsigned)nseq * (unsigned)chunks), dim3(256), 0, st, d_nodes, d_off,
+                     d_cols, chunks);
+  if (hipGetLastError() != hipSuccess ||
+      hipMemcpyAsync(cols, d_cols, sizeof(int32_t) * (size_t)off[nseq], hipMemcpyDeviceToHost, st) ||
+      hipStreamSynchronize(st))
+    return TA_E_DEVICE;
+  tr.mark("columns");
   return TA_OK;
 }

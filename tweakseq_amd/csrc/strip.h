@@ -102,9 +102,9 @@ __device__ __forceinline__ bool strip_better(int h, int i, int j, int bh, int bi
 }
 
 // What most strips' surroundings have in common: direction codes kept, the
-// matrix's own left border, no columns kept.
+// matrix's own left border, no columns kept, scores from slots.
 struct StripIODefaults {
-  static constexpr bool TB = true, KEEP = false, BYTES = false;
+  static constexpr bool TB = true, KEEP = false, BYTES = false, SLOTS = true;
   static constexpr int NC = STRIP_NC;
   static constexpr const int2 *left = nullptr;
   __device__ __forceinline__ bool keeps(int) const { return false; }
@@ -114,8 +114,10 @@ struct StripIODefaults {
 
 // Strip s (0-based) of an m x n pair over T = n + 63 steps (rounded up to 8).
 // IO is the strip's surroundings:
+//   SLOTS (scores from this wave's slot):
 //   uint64_t codes(b)            the codes of this lane's 8 columns of block b <= T / 8 (pads outside the columns)
 //   uint32_t slot_add            added to every 4 packed codes (the slot's first row, in each byte)
+//   or scores(b, half, v)        the scores of 4 of this lane's steps, each row's, |open| + |ext| added, and pads
 //   void peek(), await(b)        reads the strip above's progress; waits until that strip has stored block
 //                                b's columns (b <= T / 8), of the T - 63 it stores
 //   void tops(b, half, g, f)     4 of those columns' bottom row, in lane 0, and 0 in the others; above the
@@ -138,7 +140,7 @@ template <int PR, bool LOCAL, class IO>
 __device__ __forceinline__ void strip_sweep(IO &io, int s, bool last, int m, int n, int T, int open, int ext,
                                             StripEnd &end) {
   constexpr bool TB = IO::TB;
-  constexpr int SPD = TB ? strip_spd(PR) : 1, NS = strip_slot_tables(PR, IO::BYTES);
+  constexpr int SPD = TB ? strip_spd(PR) : 1, NS = IO::SLOTS ? strip_slot_tables(PR, IO::BYTES) : PR;
   const int lane = threadIdx.x & 63;
   const int r0 = (s * 64 + lane) * PR;  // 0-based first row of the lane
   const int c = open - ext, go = -open, ge = -ext;
@@ -164,9 +166,8 @@ __device__ __forceinline__ void strip_sweep(IO &io, int s, bool last, int m, int
   io.await(0);
   io.tops(0, 0, tg, tf);
   const uint32_t lbase = 4u * (uint32_t)lane;
-  const uint32_t add = io.slot_add;
-  // Scores of 4 steps from 4 packed codes, read half a block ahead.
-  struct Sc { uint32_t v[4][NS]; } sa, sb;  // of the block's first and second half
+  // Scores of 4 steps, read half a block ahead: from 4 packed codes, or from the IO.
+  struct Sc { std::conditional_t<IO::SLOTS, uint32_t, int> v[4][NS]; } sa, sb;  // of the block's first and second half
   auto fetch = [&](uint32_t w, Sc &sc) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -177,13 +178,20 @@ __device__ __forceinline__ void strip_sweep(IO &io, int s, bool last, int m, int
     }
   };
   auto score = [](const Sc &sc, int q, int k) {
+    if constexpr (!IO::SLOTS) return (int)sc.v[q][k];
     if constexpr (IO::BYTES) return (int)(int8_t)(sc.v[q][k >> 2] >> (8 * (k & 3)));
-    const uint32_t w = sc.v[q][PR > 2 && !IO::BYTES ? k >> 1 : 0];
+    const uint32_t w = (uint32_t)sc.v[q][PR > 2 && !IO::BYTES ? k >> 1 : 0];
     return PR == 1 ? (int)w : (k & 1) ? (int)w >> 16 : (int)(int16_t)w;
   };
-  uint64_t cw = io.codes(0);
-  uint32_t w1 = (uint32_t)(cw >> 32) + add;
-  fetch((uint32_t)cw + add, sa);
+  uint64_t cw = 0;   // the codes of the next block, then its second half's
+  uint32_t w1 = 0;
+  if constexpr (IO::SLOTS) {
+    cw = io.codes(0);
+    w1 = (uint32_t)(cw >> 32) + io.slot_add;
+    fetch((uint32_t)cw + io.slot_add, sa);
+  } else {
+    io.scores(0, 0, sa.v);
+  }
   // The row whose direction bits are still to be taken, and the row at hand.
   struct Pending {
     int En, F, D, H, up, oe;
@@ -401,15 +409,20 @@ __device__ __forceinline__ void strip_sweep(IO &io, int s, bool last, int m, int
       if constexpr (MODE == 0) masked_steps(q0_tag);
       else steps(std::integral_constant<bool, MODE == 2>{}, std::integral_constant<bool, IO::KEEP && MODE >= 2>{}, q0_tag);
     };
-    const uint64_t nw = io.codes(b + 1);
+    if constexpr (IO::SLOTS) cw = io.codes(b + 1);
     io.tops(b, 1, tg, tf);
     io.peek();
-    fetch(w1, sb);
+    if constexpr (IO::SLOTS) fetch(w1, sb);
+    else io.scores(b, 1, sb.v);
     __builtin_amdgcn_sched_barrier(0);
     half(std::integral_constant<int, 0>{});
     __builtin_amdgcn_sched_barrier(0);
-    w1 = (uint32_t)(nw >> 32) + add;
-    fetch((uint32_t)nw + add, sa);
+    if constexpr (IO::SLOTS) {
+      w1 = (uint32_t)(cw >> 32) + io.slot_add;
+      fetch((uint32_t)cw + io.slot_add, sa);
+    } else {
+      io.scores(b + 1, 0, sa.v);
+    }
     io.await(b + 1);
     io.tops(b + 1, 0, tg, tf);
     __builtin_amdgcn_sched_barrier(0);
