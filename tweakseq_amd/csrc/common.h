@@ -75,7 +75,7 @@ struct ResultDev {
 };
 
 // Bytes of direction planes per strip of a task.
-inline uint64_t tb_strip_bytes(int P, int NB, int GG) {
+__host__ __device__ inline uint64_t tb_strip_bytes(int P, int NB, int GG) {
   return (uint64_t)NB * GG * 8 * (P == 2 ? 8 : 4);
 }
 

@@ -529,17 +529,55 @@ struct CodeJob {
   int32_t nrows, ncol, lo, hi, off0, off1;
 };
 
-struct Plan {
-  // [0] whole-wave groups, [1] G-lane groups (NGW per wave unit), [2] 8-lane
-  // groups (8 per wave unit; packed couples only, tasks1[2] stays empty)
-  std::vector<Task> tasks2[3], tasks1[3];
-  std::vector<CodeJob> cjobs;
-  uint64_t rows_n = 0, cols_n = 0;        // rowcodes / colcodes entries planned
-  std::vector<PairTB> ptb;
-  uint64_t ring_elems = 0, tb_bytes = 0;
+__host__ __device__ inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
+
+// Where a task's row codes, column codes, ring and direction planes start in
+// the plan's arrays, or (task_span) how many entries / bytes it takes there.
+struct TaskAt {
+  uint64_t row, col, ring, tb;
 };
 
-int ceil_div(int a, int b) { return (a + b - 1) / b; }
+// A couple (or single) that becomes a task.
+struct Unit {
+  int lo, hi;
+  bool single;
+  int m, n;  // rows and columns (maxima over the two halves)
+};
+
+// Tasks of one shape that a wave takes together: units [u0, u0 + cnt) of n
+// columns and S strips, their entries one after the other from `at`.
+struct TaskSpan {
+  TaskAt at;
+  uint32_t u0, cnt;
+  int32_t n, S;
+};
+
+// Tasks swept by groups of GG lanes, GWAVE / GG to a span (short spans are
+// filled with copies of their first task that write nothing).
+struct TaskList {
+  int P = 2, GG = GWAVE;
+  std::vector<Unit> units;
+  std::vector<TaskSpan> spans;  // in the order they are taken
+  int tasks() const { return (int)spans.size() * (GWAVE / GG); }
+};
+
+struct Plan {
+  // [0] whole-wave groups, [1] G-lane groups (NGW per wave unit), [2] 8-lane
+  // groups (8 per wave unit; packed couples only, list1[2] stays empty)
+  TaskList list2[3], list1[3];
+  uint64_t rows_n = 0, cols_n = 0;        // rowcodes / colcodes entries planned
+  uint64_t ring_elems = 0, tb_bytes = 0;
+  // Tasks written on the host (int32 reruns, the plain form)
+  std::vector<CodeJob> cjobs;
+  std::vector<PairTB> ptb;
+  Plan() {
+    const int gg[3] = {GWAVE, G, 8};
+    for (int g = 0; g < 3; ++g) {
+      list2[g].GG = list1[g].GG = gg[g];
+      list1[g].P = 1;
+    }
+  }
+};
 
 // Resident one-wave fill workgroups per CU: one per SIMD.  A fill wave keeps
 // its SIMD's VALU busy by itself (the recurrence's dependent chain per row is
@@ -552,11 +590,6 @@ int fill_waves_per_cu(int P, int Kp, bool nib, int want, bool walk = false) {
   if (walk) return WALK_FW;
   return std::max(1, std::min(want, (160 * 1024) / fill_lds_bytes(P, Kp, nib)));
 }
-
-// Append one task (pair lo / hi; hi == lo for a single) to the plan, swept
-// by groups of GG lanes.
-// n_force / S_force (wave units): columns and strips of the task's unit; extra
-// columns lead (local couples only), extra strips are pad rows.
 
 // Raw letters to residue codes in place, 16 bytes per thread step, through a
 // 256-entry map (0xff: outside the alphabet, which sets *bad).
@@ -579,44 +612,36 @@ __global__ void encode_kernel(uint4 *codes, size_t words, const uint8_t *map, in
   if (__any(any & 0x80) && (threadIdx.x & 63) == 0) atomicOr(bad, 1);
 }
 
-// The row and column codes of every planned task, expanded on the GPU from
-// the uploaded residues: row r of a half is its pair's query residue r (pad
-// past m), column j its reference residue j - off (pad before the leading
-// columns and past n).  One workgroup per task.
+// The row and column codes of a task (pairs A, B), expanded by a workgroup
+// from the uploaded residues: row r of a half is its pair's query residue r
+// (pad past m), column j its reference residue j - off (pad before the
+// leading columns and past n).
+__device__ __forceinline__ void expand_job(const CodeJob &c, const PairDev &A, const PairDev &B, const uint8_t *codes,
+                                           int pad, uint16_t *rowcodes, uint16_t *colcodes) {
+  for (int r = threadIdx.x; r < c.nrows; r += blockDim.x) {
+    const int ca = r < A.la ? codes[A.a_off + r] : pad;
+    const int cb = r < B.la ? codes[B.a_off + r] : pad;
+    rowcodes[c.row_off + r] = (uint16_t)(ca | (cb << 8));
+  }
+  for (int j = threadIdx.x; j < c.ncol; j += blockDim.x) {
+    const int ja = j - c.off0, jb = j - c.off1;
+    const int ca = (ja >= 0 && ja < A.lb) ? codes[A.b_off + ja] : pad;
+    const int cb = (jb >= 0 && jb < B.lb) ? codes[B.b_off + jb] : pad;
+    colcodes[c.col_off + j] = (uint16_t)(ca | (cb << 8));
+  }
+}
+
+// The codes of a list of tasks, one workgroup per task.
 __global__ void expand_codes_kernel(const CodeJob *jobs, int njobs, const PairDev *pairs, const uint8_t *codes,
                                     int pad, uint16_t *rowcodes, uint16_t *colcodes) {
   for (int q = blockIdx.x; q < njobs; q += gridDim.x) {
     const CodeJob c = jobs[q];
-    const PairDev A = pairs[c.lo], B = pairs[c.hi];
-    for (int r = threadIdx.x; r < c.nrows; r += blockDim.x) {
-      const int ca = r < A.la ? codes[A.a_off + r] : pad;
-      const int cb = r < B.la ? codes[B.a_off + r] : pad;
-      rowcodes[c.row_off + r] = (uint16_t)(ca | (cb << 8));
-    }
-    for (int j = threadIdx.x; j < c.ncol; j += blockDim.x) {
-      const int ja = j - c.off0, jb = j - c.off1;
-      const int ca = (ja >= 0 && ja < A.lb) ? codes[A.b_off + ja] : pad;
-      const int cb = (jb >= 0 && jb < B.lb) ? codes[B.b_off + jb] : pad;
-      colcodes[c.col_off + j] = (uint16_t)(ca | (cb << 8));
-    }
+    expand_job(c, pairs[c.lo], pairs[c.hi], codes, pad, rowcodes, colcodes);
   }
 }
 
 // Allocates a plan's row and column codes on the device and expands them
 // there (the residues and pair descriptors are already uploaded).
-// Allocates a plan's row and column codes and expands them from a job list
-// already on the device.
-int expand_jobs(const CodeJob *d_jobs, size_t njobs, uint64_t rows_n, uint64_t cols_n, const PairDev *d_pairs,
-                const uint8_t *d_codes, int Kp, uint16_t **d_rows, uint16_t **d_cols, hipStream_t st) {
-  int rc = dalloc(d_rows, (size_t)rows_n);
-  rc = rc ? rc : dalloc(d_cols, (size_t)cols_n);
-  if (rc || !njobs) return rc;
-  (void)hipGetLastError();
-  hipLaunchKernelGGL(expand_codes_kernel, dim3((unsigned)std::min<size_t>(njobs, 65536)), dim3(256), 0, st,
-                     d_jobs, (int)njobs, d_pairs, d_codes, Kp - 1, *d_rows, *d_cols);
-  return hipGetLastError() == hipSuccess ? TA_OK : TA_E_DEVICE;
-}
-
 int expand_codes(const std::vector<CodeJob> &jobs, uint64_t rows_n, uint64_t cols_n, const PairDev *d_pairs,
                  const uint8_t *d_codes, int Kp, uint16_t **d_rows, uint16_t **d_cols, hipStream_t st) {
   int rc = dalloc(d_rows, (size_t)rows_n);
@@ -635,179 +660,254 @@ int expand_codes(const std::vector<CodeJob> &jobs, uint64_t rows_n, uint64_t col
   return rc;
 }
 
-// Where a task's row codes, column codes, ring and direction planes start in
-// the plan's arrays, or (task_span) how many entries / bytes it takes there.
-struct TaskAt {
-  uint64_t row, col, ring, tb;
-};
 // Row codes: S * ST entries; column codes: 8 NB + 8 (a multiple of 8, so
 // every task's columns start 16-byte aligned); ring: two arrays of
 // 8 NB + 2 GG + 16 when there is more than one strip.
-TaskAt task_span(int P, int GG, bool trace, int n, int S) {
+__host__ __device__ inline TaskAt task_span(int P, int GG, bool trace, int n, int S) {
   const int NB = ceil_div(n + GG, 8);
   return TaskAt{(uint64_t)S * GG * R, (uint64_t)(8 * NB + 8), S > 1 ? 2ull * (8 * NB + 2 * GG + 16) : 0,
                 trace ? (uint64_t)S * tb_strip_bytes(P, NB, GG) : 0};
 }
 
-// One task (pair lo / hi; hi == lo for a single) of n columns and S strips
-// at the given offsets: the task, its code-expansion job (expanded on the
-// GPU) and the pairs' direction-plane records.
-Task make_task(const TaskAt &at, CodeJob &job, std::vector<PairTB> &ptb, int P, int GG, bool trace,
-               const std::vector<HostPair> &hp, int lo, int hi, bool single, int n, int S) {
-  const HostPair &A = hp[lo], &B = hp[hi];
+// One task (pair lo / hi; hi == lo for a single; la, lb: their lengths) of n
+// columns and S strips at the given offsets.
+__host__ __device__ inline Task make_task(const TaskAt &at, int GG, bool trace, int lo, int hi, const int (&la)[2],
+                                          const int (&lb)[2], bool single, int n, int S) {
   Task T{};
   T.pair[0] = lo; T.pair[1] = hi;
-  T.m[0] = A.la; T.m[1] = B.la;
+  T.m[0] = la[0]; T.m[1] = la[1];
   T.n = n;
-  T.off[0] = T.n - A.lb; T.off[1] = T.n - B.lb;
+  T.off[0] = n - lb[0]; T.off[1] = n - lb[1];
   T.S = S;
-  T.NB = ceil_div(T.n + GG, 8);
+  T.NB = ceil_div(n + GG, 8);
   T.single = single ? 1 : 0;
   T.row_off = at.row;
   T.col_off = at.col;
-  job = CodeJob{T.row_off, T.col_off, T.S * GG * R, 8 * T.NB + 8, lo, hi, T.off[0], T.off[1]};
-  T.ring_len = T.S > 1 ? 8 * T.NB + 2 * GG + 16 : 0;
+  T.ring_len = S > 1 ? 8 * T.NB + 2 * GG + 16 : 0;
   T.ring_off = at.ring;
   T.tb_off = trace ? at.tb : 0;
-  for (int h = 0; h < (single ? 1 : 2); ++h) {
-    PairTB &d = ptb[h ? hi : lo];
-    d.tb_off = T.tb_off; d.P = P; d.half = h; d.NB = T.NB; d.off = T.off[h]; d.GG = GG;
-  }
   return T;
 }
+// The direction-plane record of a task's half.
+__host__ __device__ inline PairTB task_ptb(const Task &T, int P, int GG, int h) {
+  PairTB d{};
+  d.tb_off = T.tb_off; d.P = P; d.half = h; d.NB = T.NB; d.off = T.off[h]; d.GG = GG;
+  return d;
+}
 
-// make_task at the plan's running offsets, appended to dst.
+// A task on the host at the plan's running offsets, appended to dst with its
+// code-expansion job and its pairs' records.
 void add_task(Plan &pl, std::vector<Task> &dst, int P, int GG, bool trace, const std::vector<HostPair> &hp,
-              int lo, int hi, bool single, int Kp, int n_force = 0, int S_force = 0) {
-  const HostPair &A = hp[lo], &B = hp[hi];
-  const int n = n_force ? n_force : std::max(A.lb, B.lb);
-  const int S = S_force ? S_force : ceil_div(std::max(A.la, B.la), GG * R);
+              int lo, int hi, bool single, int n = 0, int S = 0) {
+  const int la[2] = {hp[lo].la, hp[hi].la}, lb[2] = {hp[lo].lb, hp[hi].lb};
+  if (!n) n = std::max(lb[0], lb[1]);
+  if (!S) S = ceil_div(std::max(la[0], la[1]), GG * R);
   const TaskAt at{pl.rows_n, pl.cols_n, pl.ring_elems, pl.tb_bytes}, sz = task_span(P, GG, trace, n, S);
-  pl.cjobs.emplace_back();
-  dst.push_back(make_task(at, pl.cjobs.back(), pl.ptb, P, GG, trace, hp, lo, hi, single, n, S));
+  dst.push_back(make_task(at, GG, trace, lo, hi, la, lb, single, n, S));
+  const Task &T = dst.back();
+  pl.cjobs.push_back(CodeJob{T.row_off, T.col_off, T.S * GG * R, 8 * T.NB + 8, lo, hi, T.off[0], T.off[1]});
+  for (int h = 0; h < (single ? 1 : 2); ++h) pl.ptb[h ? hi : lo] = task_ptb(T, P, GG, h);
   pl.rows_n += sz.row; pl.cols_n += sz.col; pl.ring_elems += sz.ring; pl.tb_bytes += sz.tb;
 }
 
+// Start of a batch on the device: its pairs' fill outputs before a run (an
+// empty side: the finished result) and their direction-plane records (pairs
+// of at least long_cells cells: the long-pair kernels').
+__global__ void pairs_init_kernel(const PairDev *pairs, int n, FillOut *fo, PairTB *ptb, int local, int open, int ext,
+                                  int64_t long_cells) {
+  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
+    const int la = pairs[k].la, lb = pairs[k].lb;
+    FillOut f{0, 0, 0, 0};
+    PairTB d{};
+    if (la == 0 || lb == 0) {
+      if (local) {
+        f.flags = 8;
+      } else {
+        f.score = la + lb ? open + (la + lb - 1) * ext : 0;
+        f.end_i = la; f.end_j = lb;
+      }
+    } else if ((int64_t)la * lb >= long_cells) {
+      d.P = 3;
+    }
+    fo[k] = f;
+    ptb[k] = d;
+  }
+}
+
+// The planned tasks, their pairs' direction-plane records and their row and
+// column codes, a workgroup per task.  The host plans spans only (shapes,
+// offsets, which units): tasks, code jobs and records written there and
+// copied over were 15 of the 20 MB that the creation of a batch of 130,816
+// pairs wrote and sent.  With the pairs' table written by the host threads
+// and its copy under the planning, and sorts of packed 64-bit keys, that
+// creation takes 3.1 ms instead of 6.5.
+struct PlanArgs {
+  struct List {
+    const Unit *units;
+    const TaskSpan *spans;
+    Task *dst;
+    int32_t ntasks, P, GG;
+  } list[6];
+  int32_t trace, pad;
+  const PairDev *pairs;
+  const uint8_t *codes;
+  PairTB *ptb;
+  uint16_t *rowcodes, *colcodes;
+};
+__global__ __launch_bounds__(256) void plan_tasks_kernel(PlanArgs A, int total) {
+  for (int x = blockIdx.x; x < total; x += gridDim.x) {
+    int q = x, l = 0;
+    while (q >= A.list[l].ntasks) q -= A.list[l++].ntasks;
+    const PlanArgs::List &L = A.list[l];
+    const int NG = GWAVE / L.GG, i = q % NG;
+    const TaskSpan s = L.spans[q / NG];
+    const bool filler = i >= (int)s.cnt;
+    const int at_i = filler ? 0 : i;
+    const Unit u = L.units[s.u0 + at_i];
+    const PairDev a = A.pairs[u.lo], b = A.pairs[u.hi];
+    const TaskAt sz = task_span(L.P, L.GG, A.trace, s.n, s.S);
+    const TaskAt at{s.at.row + at_i * sz.row, s.at.col + at_i * sz.col, s.at.ring + at_i * sz.ring,
+                    s.at.tb + at_i * sz.tb};
+    const int la[2] = {a.la, b.la}, lb[2] = {a.lb, b.lb};
+    Task T = make_task(at, L.GG, A.trace, u.lo, u.hi, la, lb, u.single, s.n, s.S);
+    if (filler) T.single = 2;
+    if (threadIdx.x == 0) {
+      L.dst[q] = T;
+      if (!filler) {
+        A.ptb[u.lo] = task_ptb(T, L.P, L.GG, 0);
+        if (!u.single) A.ptb[u.hi] = task_ptb(T, L.P, L.GG, 1);
+      }
+    }
+    if (filler) continue;
+    const CodeJob c{T.row_off, T.col_off, T.S * L.GG * R, 8 * T.NB + 8, u.lo, u.hi, T.off[0], T.off[1]};
+    expand_job(c, a, b, A.codes, A.pad, A.rowcodes, A.colcodes);
+  }
+}
+
 // Positions 0..n-1 in ascending order of key, equal keys in position order:
-// an LSD radix sort over 11-bit digits, as many as the largest key needs.
-// The planner orders tens of thousands of pairs and units per batch, where
-// comparison sorts that read their keys through the pair table cost
-// milliseconds.
-std::vector<int32_t> order_by_key(std::vector<uint64_t> key) {
+// key and position packed in 64 bits, an LSD radix sort over the 11-bit
+// digits in which the keys differ.  The planner orders tens of thousands of
+// pairs and units per batch, where comparison sorts that read their keys
+// through the pair table cost milliseconds.  `key` is used up.
+std::vector<int32_t> order_by_key(std::vector<uint64_t> &key) {
   const size_t n = key.size();
-  std::vector<int32_t> idx(n), ti(n);
-  std::vector<uint64_t> tk(n);
-  for (size_t t = 0; t < n; ++t) idx[t] = (int32_t)t;
+  std::vector<int32_t> idx;
+  vec_take(idx);
+  idx.resize(n);
+  if (!n) return idx;
+  uint64_t lo = key[0], hi = key[0];
+  for (uint64_t k : key) { lo = std::min(lo, k); hi = std::max(hi, k); }
+  int nb = 0, kb = 0;  // bits of a position, of a key's range
+  while ((uint64_t)(n - 1) >> nb) ++nb;
+  while (kb < 64 && (hi - lo) >> kb) ++kb;
+  if (nb + kb > 64) {
+    for (size_t t = 0; t < n; ++t) idx[t] = (int32_t)t;
+    std::stable_sort(idx.begin(), idx.end(), [&](int32_t a, int32_t b) { return key[a] < key[b]; });
+    return idx;
+  }
   uint64_t any = 0;
-  for (uint64_t k : key) any |= k;
-  for (int sh = 0; sh < 64 && (any >> sh) != 0; sh += 11) {
-    std::vector<size_t> at(2049, 0);
+  for (size_t t = 0; t < n; ++t) {
+    key[t] = nb < 64 ? (key[t] - lo) << nb | t : t;
+    any |= key[t] ^ key[0];
+  }
+  std::vector<uint64_t> tmp;
+  vec_take(tmp);
+  tmp.resize(n);
+  for (int sh = nb; sh < nb + kb; sh += 11) {
+    if (!(any >> sh & 2047)) continue;
+    size_t at[2049] = {0};
     for (uint64_t k : key) ++at[((k >> sh) & 2047) + 1];
     for (int d = 0; d < 2048; ++d) at[d + 1] += at[d];
-    for (size_t t = 0; t < n; ++t) {
-      const size_t q = at[(key[t] >> sh) & 2047]++;
-      ti[q] = idx[t];
-      tk[q] = key[t];
-    }
-    idx.swap(ti);
-    key.swap(tk);
+    for (uint64_t k : key) tmp[at[(k >> sh) & 2047]++] = k;
+    key.swap(tmp);
   }
+  const uint64_t mask = (1ull << nb) - 1;
+  for (size_t t = 0; t < n; ++t) idx[t] = (int32_t)(key[t] & mask);
+  vec_give(tmp);
   return idx;
 }
 
-// `v` reordered by ascending key[v's position].
+// `v` reordered by ascending key[v's position]; `key` is used up.
 template <typename T>
-void gather_by_key(std::vector<T> &v, std::vector<uint64_t> key) {
-  const std::vector<int32_t> o = order_by_key(std::move(key));
+void gather_by_key(std::vector<T> &v, std::vector<uint64_t> &key) {
+  std::vector<int32_t> o = order_by_key(key);
   std::vector<T> w;
-  w.reserve(v.size());
-  for (int32_t t : o) w.push_back(std::move(v[t]));
+  vec_take(w);
+  w.resize(v.size());
+  for (size_t t = 0; t < o.size(); ++t) w[t] = v[o[t]];
   v.swap(w);
+  vec_give(w);
+  vec_give(o);
 }
 
 // Lengths are at most 1,000,000 (< 2^20), strips of STRIP rows at most 2^13.
 constexpr uint64_t LEN_TOP = (1u << 20) - 1, STRIPS_TOP = (1u << 13) - 1;
 static_assert((1000000 + STRIP - 1) / STRIP <= (int)STRIPS_TOP, "strip count exceeds its key field");
 
-// A couple (or single) waiting to be grouped into a wave unit of G-lane tasks.
-struct Unit {
-  int lo, hi;
-  bool single;
-  int m, n;  // rows and columns (maxima over the two halves)
-};
-
 // Wave units: GWAVE / GG tasks of GG lanes and one shape that one wave runs
 // in lockstep.  Local couples are ordered by (strips, columns) and take their
 // unit's column count as leading pad columns; global couples need equal
 // column counts (H(m, n) is read at the last column), so they are grouped by
-// columns.  A unit short of its tasks is filled with copies of its first
-// task that write nothing.  Units go out largest first, flattened (GWAVE /
-// GG tasks per unit).
-void add_units(Plan &pl, std::vector<Task> &dst, int P, int GG, std::vector<Unit> u, bool local, bool trace,
-               const std::vector<HostPair> &hp, int Kp) {
-  const int NG = GWAVE / GG;
+// columns.  Whole-wave tasks are units of one.  Units go out largest first
+// (more 8-step blocks first, S * NB < 2^40, stable), with offsets in that order.
+void plan_units(Plan &pl, TaskList &L, bool local, bool trace) {
+  const int GG = L.GG, NG = GWAVE / GG;
+  std::vector<Unit> &u = L.units;
   auto strips = [GG](int m) { return ceil_div(std::max(m, 1), GG * R); };
-  {  // local: more strips first, then more columns; global: columns first
-    std::vector<uint64_t> key(u.size());
+  std::vector<uint64_t> key;
+  vec_take(key);
+  if (NG > 1) {  // local: more strips first, then more columns; global: columns first
+    key.resize(u.size());
     for (size_t t = 0; t < u.size(); ++t) {
       const uint64_t sk = STRIPS_TOP - (uint64_t)strips(u[t].m), nk = LEN_TOP - (uint64_t)u[t].n;
       key[t] = local ? (sk << 20 | nk) : (nk << 13 | sk);
     }
-    gather_by_key(u, std::move(key));
+    gather_by_key(u, key);
   }
-  // The units' extents and shapes first, then their tasks straight into dst
-  // in order of cost (more 8-step blocks first, S * NB < 2^40).
-  struct Span { uint32_t k, e; int nq, mq; };
-  std::vector<Span> spans;
-  spans.reserve(u.size() / NG + 1);
-  std::vector<uint64_t> key;
-  key.reserve(u.size() / NG + 1);
+  std::vector<TaskSpan> spans;
+  vec_take(spans);
+  key.clear();
   for (size_t k = 0; k < u.size();) {
     size_t e = k;
-    while (e < u.size() && e - k < (size_t)NG && (local || u[e].n == u[k].n)) ++e;
     int nq = 0, mq = 0;
-    for (size_t i = k; i < e; ++i) { nq = std::max(nq, u[i].n); mq = std::max(mq, u[i].m); }
-    spans.push_back(Span{(uint32_t)k, (uint32_t)e, nq, mq});
+    for (; e < u.size() && e - k < (size_t)NG && (local || u[e].n == u[k].n); ++e) {
+      nq = std::max(nq, u[e].n);
+      mq = std::max(mq, u[e].m);
+    }
+    spans.push_back(TaskSpan{TaskAt{0, 0, 0, 0}, (uint32_t)k, (uint32_t)(e - k), nq, strips(mq)});
     key.push_back((1ull << 40) - (uint64_t)strips(mq) * (uint64_t)ceil_div(nq + GG, 8));
     k = e;
   }
-  const std::vector<int32_t> o = order_by_key(std::move(key));
-  // Offsets in unit order (every task of a unit has the unit's shape), then
-  // the tasks, jobs and plane records on the host threads: each unit's
-  // entries, and its pairs' records, are its own.
-  struct UnitAt { TaskAt at, sz; size_t dst, job; };
-  std::vector<UnitAt> ua(o.size());
-  size_t nd = dst.size(), nj = pl.cjobs.size();
-  for (size_t x = 0; x < o.size(); ++x) {
-    const Span &sp = spans[o[x]];
-    const uint64_t cnt = sp.e - sp.k;
-    UnitAt &a = ua[x];
-    a.at = TaskAt{pl.rows_n, pl.cols_n, pl.ring_elems, pl.tb_bytes};
-    a.sz = task_span(P, GG, trace, sp.nq, strips(sp.mq));
-    a.dst = nd;
-    a.job = nj;
-    pl.rows_n += cnt * a.sz.row; pl.cols_n += cnt * a.sz.col;
-    pl.ring_elems += cnt * a.sz.ring; pl.tb_bytes += cnt * a.sz.tb;
-    nd += NG;
-    nj += cnt;
+  gather_by_key(spans, key);
+  vec_give(key);
+  for (TaskSpan &s : spans) {
+    const TaskAt sz = task_span(L.P, GG, trace, s.n, s.S);
+    s.at = TaskAt{pl.rows_n, pl.cols_n, pl.ring_elems, pl.tb_bytes};
+    pl.rows_n += s.cnt * sz.row; pl.cols_n += s.cnt * sz.col;
+    pl.ring_elems += s.cnt * sz.ring; pl.tb_bytes += s.cnt * sz.tb;
   }
-  dst.resize(nd);
-  pl.cjobs.resize(nj);
-  parallel_for(o.size(), [&](size_t x) {
-    const Span &sp = spans[o[x]];
-    const UnitAt &a = ua[x];
-    for (uint32_t i = sp.k; i < sp.e; ++i) {
-      const uint64_t q = i - sp.k;
-      const TaskAt at{a.at.row + q * a.sz.row, a.at.col + q * a.sz.col, a.at.ring + q * a.sz.ring,
-                      a.at.tb + q * a.sz.tb};
-      dst[a.dst + q] = make_task(at, pl.cjobs[a.job + q], pl.ptb, P, GG, trace, hp, u[i].lo, u[i].hi, u[i].single,
-                                 sp.nq, strips(sp.mq));
+  L.spans.swap(spans);
+  vec_give(spans);
+}
+
+// The wave units of int32 singles `u`, written on the host.
+void add_units(Plan &pl, std::vector<Task> &dst, std::vector<Unit> u, bool local, bool trace,
+               const std::vector<HostPair> &hp) {
+  TaskList L;
+  L.P = 1; L.GG = G;
+  L.units.swap(u);
+  Plan shapes;
+  plan_units(shapes, L, local, trace);
+  for (const TaskSpan &s : L.spans) {
+    const size_t first = dst.size();
+    for (uint32_t i = s.u0; i < s.u0 + s.cnt; ++i)
+      add_task(pl, dst, 1, G, trace, hp, L.units[i].lo, L.units[i].hi, L.units[i].single, s.n, s.S);
+    for (uint32_t q = s.cnt; q < (uint32_t)NGW; ++q) {  // fillers: copies that write nothing
+      Task f = dst[first];
+      f.single = 2;
+      dst.push_back(f);
     }
-    for (uint32_t q = sp.e - sp.k; q < (uint32_t)NG; ++q) {  // fillers: copies that write nothing
-      dst[a.dst + q] = dst[a.dst];
-      dst[a.dst + q].single = 2;
-    }
-  });
+  }
 }
 
 // Steps a G-lane group needs for a task of these shapes, in 8-step blocks.
@@ -866,7 +966,6 @@ struct ta_batch {
   bool may_saturate = false;
   int64_t cells = 0;
   std::vector<HostPair> hp;
-  std::vector<FillOut> fo_init;
   FillOut *d_fo_init = nullptr;
   int32_t *d_order = nullptr;  // traceback walker -> pair, longest first
   // Walks inside the fill kernel (direction planes, no int32 rerun possible):
@@ -877,7 +976,6 @@ struct ta_batch {
   int32_t ncoop2 = 0, ncoop1 = 0;
   int32_t n_rest = 0;
   int32_t *d_order_rest = nullptr;
-  std::vector<PairDev> pairs_h;
   uint64_t cig_bytes = 0;
   Plan plan;
   // device
@@ -1005,13 +1103,11 @@ void ta_batch_destroy(ta_batch *B) {
   if (B->gexec) (void)hipGraphExecDestroy(B->gexec);
   if (B->graph) (void)hipGraphDestroy(B->graph);
   vec_give(B->hp);
-  vec_give(B->fo_init);
-  vec_give(B->pairs_h);
-  vec_give(B->plan.ptb);
-  vec_give(B->plan.cjobs);
   for (int g = 0; g < 3; ++g) {
-    vec_give(B->plan.tasks2[g]);
-    vec_give(B->plan.tasks1[g]);
+    vec_give(B->plan.list2[g].units);
+    vec_give(B->plan.list2[g].spans);
+    vec_give(B->plan.list1[g].units);
+    vec_give(B->plan.list1[g].spans);
   }
   delete B;
 }
@@ -1069,7 +1165,7 @@ static void plan_strips(ta_ctx *ctx, ta_batch *B) {
     const HostPair &h = B->hp[ks[t]];
     key[t] = (1ull << 32) - (uint64_t)h.lb - 100ull * ceil_div(h.la, 64 * STRIPS_PR);
   }
-  gather_by_key(ks, std::move(key));
+  gather_by_key(ks, key);
   B->spairs.reserve(ks.size());
   B->sitems.reserve((size_t)strips);
   for (int32_t k : ks) {
@@ -1119,7 +1215,9 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
   } else {
     std::lock_guard<std::mutex> g(ctx->tune_mu);
     int bucket = 0;
-    if (res) {  // the bucket from the resident sequences' lengths
+    if (ctx->tune.empty()) {
+      // (the defaults)
+    } else if (res) {  // the bucket from the resident sequences' lengths
       std::vector<ta_pair> lens((size_t)n);
       for (int32_t k = 0; k < n; ++k) lens[k] = ta_pair{nullptr, res->la[k], nullptr, res->lb[k]};
       bucket = ta_tune_bucket(lens.data(), n);
@@ -1153,11 +1251,39 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
     const int32_t la = res->la[k], lb = res->lb[k];
     return ta_pair{la ? "" : nullptr, la, lb ? "" : nullptr, lb};
   };
-  for (int32_t k = 0; k < n; ++k)
-    if (!pair_ok(*p, pair_at(k))) {
+  // The pairs in contiguous shares, one per host thread: sums first, then the
+  // tables at the offsets they give.
+  struct Share {
+    bool ok = true, maysat = false;
+    int64_t cells = 0;
+    uint64_t cig = 0;
+    size_t n16 = 0, n32 = 0;
+  };
+  const int NS = n >= 4096 ? (int)std::max(1u, std::min(16u, std::thread::hardware_concurrency())) : 1;
+  auto share_at = [&](int t) { return (int32_t)((int64_t)n * t / NS); };
+  std::vector<Share> shares(NS);
+  parallel_tasks(NS, [&](int t) {
+    Share s;
+    for (int32_t k = share_at(t); k < share_at(t + 1); ++k) {
+      const ta_pair q = pair_at(k);
+      if (!pair_ok(*p, q)) s.ok = false;
+      s.cells += (int64_t)q.la * q.lb;
+      s.cig += (uint64_t)(p->traceback ? 4 * (q.la + q.lb + 1) : 0);  // one dword per run at most
+    }
+    shares[t] = s;
+  });
+  uint64_t cig = 0;
+  for (Share &s : shares) {
+    if (!s.ok) {
       delete B;
       return TA_E_INVALID;
     }
+    B->cells += s.cells;
+    const uint64_t at = cig;
+    cig += s.cig;
+    s.cig = at;
+  }
+  B->cig_bytes = cig;
   tr.mark("validate");
   auto mix = [](const char *s) -> uint64_t {
     uint64_t x = (uint64_t)(uintptr_t)s;
@@ -1178,6 +1304,7 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
   std::vector<std::vector<Uniq>> &part = tl_part;
   std::vector<Uniq> &uq = tl_uq;
   size_t ctotal = 0;  // bytes of the unique sequences' codes
+  std::vector<int32_t> base(T + 1, 0);  // first unique entry of each thread's share
   if (!res) {
     ua.resize((size_t)n);
     ub.resize((size_t)n);
@@ -1226,7 +1353,6 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
     // Global order: partition by partition; each sequence starts 16-byte
     // aligned (walker windows).  Offsets and the flat array, per partition on
     // the threads, from the partitions' counts and byte totals.
-    std::vector<int32_t> base(T + 1, 0);
     std::vector<size_t> bbase(T + 1, 0);
     for (int t = 0; t < T; ++t) {
       base[t + 1] = base[t] + (int32_t)part[t].size();
@@ -1247,12 +1373,6 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
     });
     ctotal = bbase[T];
     tr.mark("dedupe offsets");
-    if (T > 1)
-      parallel_for((size_t)n, [&](size_t k) {
-        ua[k] += base[part_of(mix(pairs[k].a))];
-        ub[k] += base[part_of(mix(pairs[k].b))];
-      });
-    tr.mark("dedupe");
   }
   // The walker reads 32-byte windows: 32 bytes of slack after the last
   // sequence.  The raw letters go up as they are, each sequence followed by
@@ -1292,17 +1412,16 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
   int maxbest = 0;
   for (int r = 0; r < B->alph.K; ++r) maxbest = std::max(maxbest, best[r]);
   const int64_t sat_limit = 32767 - 2L * B->alph.maxS;
-  auto bound = [&](int32_t u) -> int64_t {
-    Uniq &e = uq[u];
-    if ((int64_t)e.len * maxbest <= sat_limit) return (int64_t)e.len * maxbest;
-    if (e.bound < 0) {
+  if (local && !res)
+    parallel_for(uq.size(), [&](size_t u) {
+      Uniq &e = uq[u];
+      e.bound = (int64_t)e.len * maxbest;
+      if (e.bound <= sat_limit) return;
       int64_t sum = 0;
       const unsigned char *src = (const unsigned char *)e.s;
       for (int32_t i = 0; i < e.len; ++i) sum += map[src[i]] < 0x80 ? best[map[src[i]]] : 0;
       e.bound = sum;
-    }
-    return e.bound;
-  };
+    });
   // The letters go up while the host plans: from the pinned block the copy
   // runs on the DMA engine alone; the encoding kernel follows on the stream.
   hipStream_t st = B->stream;
@@ -1339,46 +1458,75 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
     return rc;
   }
   tr.mark("upload-encode");
+  // The pairs' table goes up while the host plans, too.
+  StageHold ptab;
+  ptab.s = stage_take(sizeof(PairDev) * (size_t)std::max(n, 1));
+  if (!ptab.s.p) rc = TA_E_NOMEM;
+  PairDev *pairs_h = (PairDev *)ptab.s.p;
   vec_take(B->hp);
-  vec_take(B->fo_init);
-  vec_take(B->pairs_h);
   B->hp.resize(n);
-  B->fo_init.assign(n, FillOut{0, 0, 0, 0});
-  B->pairs_h.resize(n);
-  for (int32_t k = 0; k < n; ++k) {
-    const ta_pair q = pair_at(k);
-    HostPair &h = B->hp[k];
-    h.a_off = res ? res->a_off[k] : uq[ua[k]].off;
-    h.b_off = res ? res->b_off[k] : uq[ub[k]].off;
-    h.la = q.la; h.lb = q.lb;
-    B->cells += (int64_t)q.la * q.lb;
-    if (q.la == 0 || q.lb == 0) {
-      h.path = 0;
-      FillOut &f = B->fo_init[k];
-      if (local) { f.flags = 8; }
-      else {
-        const int len = q.la + q.lb;
-        f.score = len ? p->gap_open + (len - 1) * p->gap_extend : 0;
-        f.end_i = q.la; f.end_j = q.lb;
+  if (!rc) parallel_tasks(NS, [&](int t) {
+    Share &s = shares[t];
+    uint64_t cig_at = s.cig;
+    for (int32_t k = share_at(t); k < share_at(t + 1); ++k) {
+      const ta_pair q = pair_at(k);
+      HostPair h{};
+      int32_t a = 0, b = 0;
+      if (!res) {
+        a = ua[k] + (T > 1 ? base[part_of(mix(q.a))] : 0);
+        b = ub[k] + (T > 1 ? base[part_of(mix(q.b))] : 0);
       }
-    } else if (long_pair(*p, q.la, q.lb)) {
-      h.path = 3;
-    } else if (lanes == TA_LANES_I32 || (!B->nib && !B->trace)) {
-      h.path = 1;
-    } else if (local && q.lb > 32767) {
-      h.path = 1;  // packed end-cell keys hold the column in 15 bits
-    } else if (local) {
-      h.path = 2;
-      h.maysat = (res ? std::min(res->a_bound[k], res->b_bound[k]) : std::min(bound(ua[k]), bound(ub[k]))) > sat_limit;
-      if (h.maysat) B->may_saturate = true;
-    } else {
-      h.path = global_i16_safe(*p, B->alph.maxS, q.la, q.lb) ? 2 : 1;
+      h.a_off = res ? res->a_off[k] : uq[a].off;
+      h.b_off = res ? res->b_off[k] : uq[b].off;
+      h.la = q.la; h.lb = q.lb;
+      if (q.la == 0 || q.lb == 0) {
+        h.path = 0;
+      } else if (long_pair(*p, q.la, q.lb)) {
+        h.path = 3;
+      } else if (lanes == TA_LANES_I32 || (!B->nib && !B->trace)) {
+        h.path = 1;
+      } else if (local && q.lb > 32767) {
+        h.path = 1;  // packed end-cell keys hold the column in 15 bits
+      } else if (local) {
+        h.path = 2;
+        h.maysat = (res ? std::min(res->a_bound[k], res->b_bound[k]) : std::min(uq[a].bound, uq[b].bound)) > sat_limit;
+        if (h.maysat) s.maysat = true;
+      } else {
+        h.path = global_i16_safe(*p, B->alph.maxS, q.la, q.lb) ? 2 : 1;
+      }
+      s.n16 += h.path == 2;
+      s.n32 += h.path == 1;
+      B->hp[k] = h;
+      PairDev d{};
+      d.a_off = h.a_off; d.b_off = h.b_off; d.la = q.la; d.lb = q.lb;
+      d.cig_cap = p->traceback ? 4 * (q.la + q.lb + 1) : 0;
+      d.cig_off = cig_at;
+      cig_at += (uint64_t)d.cig_cap;
+      pairs_h[k] = d;
     }
-    PairDev &d = B->pairs_h[k];
-    d.a_off = h.a_off; d.b_off = h.b_off; d.la = q.la; d.lb = q.lb;
-    d.cig_cap = p->traceback ? 4 * (q.la + q.lb + 1) : 0;  // one dword per run at most
-    d.cig_off = B->cig_bytes;
-    B->cig_bytes += (uint64_t)d.cig_cap;
+  });
+  for (const Share &s : shares) B->may_saturate = B->may_saturate || s.maysat;
+  rc = rc ? rc : dalloc(&B->d_pairs, (size_t)std::max(n, 1));
+  rc = rc ? rc : dalloc(&B->d_fo_init, (size_t)std::max(n, 1));
+  rc = rc ? rc : dalloc(&B->d_ptb, (size_t)std::max(n, 1));
+  if (!rc && n) {
+    ptab.stream = st;
+    ptab.queued = true;
+    const int64_t long_cells = local ? INT64_MAX : p->lanes == TA_LANES_LONG ? 1
+                                     : p->lanes == TA_LANES_AUTO ? kLongCells : INT64_MAX;
+    (void)hipGetLastError();
+    if (hipMemcpyAsync(B->d_pairs, pairs_h, sizeof(PairDev) * n, hipMemcpyHostToDevice, st) != hipSuccess)
+      rc = TA_E_DEVICE;
+    if (!rc) hipLaunchKernelGGL(pairs_init_kernel, dim3((unsigned)std::min(1024, (n + 255) / 256)), dim3(256), 0, st,
+                                B->d_pairs, n, B->d_fo_init, B->d_ptb, (int)local, p->gap_open, p->gap_extend, long_cells);
+    if (hipGetLastError() != hipSuccess) rc = TA_E_DEVICE;
+  }
+  if (rc) {
+    (void)hipStreamSynchronize(st);
+    dfree(d_map);
+    dfree(d_bad);
+    ta_batch_destroy(B);
+    return rc;
   }
 
   tr.mark("pairs");
@@ -1386,64 +1534,70 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
   // Couples: local pairs pad to the longer column count; global couples
   // need equal column counts (so H(m, n) of both sits in the last column).
   Plan &pl = B->plan;
-  vec_take(pl.ptb);
-  vec_take(pl.cjobs);
   for (int g = 0; g < 3; ++g) {
-    vec_take(pl.tasks2[g]);
-    vec_take(pl.tasks1[g]);
+    vec_take(pl.list2[g].units);
+    vec_take(pl.list1[g].units);
   }
-  pl.ptb.assign(n, PairTB{0, 0, 0, 0, 0, 0, 0});
-  pl.cjobs.reserve((size_t)n / 2 + NGW);
-  std::vector<int> i16, i32;
-  for (int32_t k = 0; k < n && !B->strips; ++k) {
-    if (B->hp[k].path == 2) i16.push_back(k);
-    else if (B->hp[k].path == 1) i32.push_back(k);
-  }
+  std::vector<int32_t> i16, i32;
+  std::vector<uint64_t> key;
+  vec_take(i16);
+  vec_take(i32);
+  vec_take(key);
   // More strips first, then more columns, then lower pair index (the lists
   // hold ascending pair indices).
   // Local pairs are ranked by 64-row strips (those of 8-lane units), which
   // keeps them in order of 128-row strips too.
   const int rank_rows = local ? 8 * R : STRIP;
   static_assert((1000000 + 8 * R - 1) / (8 * R) < (1 << 15), "strip count exceeds its key field");
-  auto sort_bigger = [&](std::vector<int> &v) {
-    std::vector<uint64_t> key(v.size());
-    for (size_t t = 0; t < v.size(); ++t) {
-      const HostPair &h = B->hp[v[t]];
-      key[t] = ((1ull << 15) - (uint64_t)ceil_div(h.la, rank_rows)) << 20 | (LEN_TOP - (uint64_t)h.lb);
+  // Global couples: groups of equal columns in ascending order, each ranked so.
+  if (!B->strips) {
+    size_t n16 = 0, n32 = 0;
+    std::vector<size_t> at16(NS), at32(NS);
+    for (int t = 0; t < NS; ++t) {
+      at16[t] = n16; at32[t] = n32;
+      n16 += shares[t].n16; n32 += shares[t].n32;
     }
-    gather_by_key(v, std::move(key));
-  };
-  std::vector<std::pair<int, int>> couples;
-  if (local) {
-    sort_bigger(i16);
-    for (size_t t = 0; t < i16.size(); t += 2)
-      couples.push_back({i16[t], t + 1 < i16.size() ? i16[t + 1] : -1});
-  } else {
-    // Groups of equal columns in ascending order, each ranked as above; the
-    // members of a group pair off in turn, the odd one out alone.  One sort
-    // over all pairs (the key leads with the column count).
-    std::vector<uint64_t> key(i16.size());
-    for (size_t t = 0; t < i16.size(); ++t) {
-      const HostPair &h = B->hp[i16[t]];
-      key[t] = (uint64_t)h.lb << 35 | ((1ull << 15) - (uint64_t)ceil_div(h.la, rank_rows)) << 20;
-    }
-    gather_by_key(i16, std::move(key));
-    for (size_t t = 0; t < i16.size();) {
-      const bool two = t + 1 < i16.size() && B->hp[i16[t + 1]].lb == B->hp[i16[t]].lb;
-      couples.push_back({i16[t], two ? i16[t + 1] : -1});
-      t += two ? 2 : 1;
-    }
+    i16.resize(n16);
+    i32.resize(n32);
+    key.resize(n16);
+    parallel_tasks(NS, [&](int t) {
+      size_t a = at16[t], b = at32[t];
+      for (int32_t k = share_at(t); k < share_at(t + 1); ++k) {
+        const HostPair &h = B->hp[k];
+        if (h.path == 1) i32[b++] = k;
+        if (h.path != 2) continue;
+        const uint64_t rank = (1ull << 15) - (uint64_t)ceil_div(h.la, rank_rows);
+        key[a] = local ? rank << 20 | (LEN_TOP - (uint64_t)h.lb) : (uint64_t)h.lb << 16 | rank;
+        i16[a++] = k;
+      }
+    });
+    gather_by_key(i16, key);
+  }
+  tr.mark("ranks");
+  // Neighbours pair off; globally, within a group of equal columns, whose odd
+  // one out goes alone.
+  // (the lengths gathered on the host threads first: a read of a table that
+  // they wrote is a miss in one thread's caches)
+  std::vector<std::pair<int32_t, int32_t>> len;
+  vec_take(len);
+  len.resize(i16.size());
+  parallel_for(i16.size(), [&](size_t t) {
+    const HostPair &h = B->hp[i16[t]];
+    len[t] = {h.la, h.lb};
+  });
+  std::vector<Unit> couples;
+  vec_take(couples);
+  couples.reserve(local ? (i16.size() + 1) / 2 : i16.size());
+  double work = 0;  // mean group-slot work decides which tasks get whole-wave groups
+  for (size_t t = 0; t < i16.size();) {
+    const bool two = t + 1 < i16.size() && (local || len[t + 1].second == len[t].second);
+    const size_t u = two ? t + 1 : t;
+    couples.push_back(Unit{i16[t], i16[u], !two, std::max(len[t].first, len[u].first),
+                           std::max(len[t].second, len[u].second)});
+    work += group_cost(couples.back().m, couples.back().n);
+    t += two ? 2 : 1;
   }
   tr.mark("couples");
-  // Mean group-slot work decides which tasks get whole-wave groups.
-  double work = 0;
-  auto shape = [&](int lo, int hi) {
-    return std::make_pair(std::max(B->hp[lo].la, B->hp[hi].la), std::max(B->hp[lo].lb, B->hp[hi].lb));
-  };
-  for (auto &c : couples) {
-    auto sh = shape(c.first, c.second < 0 ? c.first : c.second);
-    work += group_cost(sh.first, sh.second);
-  }
   for (int k : i32) work += group_cost(B->hp[k].la, B->hp[k].lb);
   // Walks in the fill kernel: batches with direction planes whose int16 fill
   // cannot saturate (a rerun would replace some pairs' planes after the fill),
@@ -1457,51 +1611,38 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
   const double slots = (double)ctx->cus * wpc * NGW;
   const double mean_slot = work / slots;
   const bool few = B->wave_tasks || couples.size() + i32.size() <= (size_t)ctx->cus * wpc;
-  std::vector<Unit> u2, u1, u8;
-  pl.tasks2[0].reserve(couples.size());
-  pl.tasks1[0].reserve(i32.size());
   const double lim8 = !few ? eight_lane_limit() * mean_slot : -1.0;
-  for (auto &c : couples) {
-    const bool single = c.second < 0;
-    const int hi = single ? c.first : c.second;
-    auto sh = shape(c.first, hi);
-    if (pick_gg(sh.first, sh.second, mean_slot, few) == GWAVE)
-      add_task(pl, pl.tasks2[0], 2, GWAVE, B->trace, B->hp, c.first, hi, single, B->Kp);
-    else if (cost8(sh.first, sh.second) <= lim8 && ceil_div(sh.first, 8 * R) <= (int)STRIPS_TOP)
-      u8.push_back(Unit{c.first, hi, single, sh.first, sh.second});  // (strip counts fit the unit sort key)
-    else
-      u2.push_back(Unit{c.first, hi, single, sh.first, sh.second});
+  for (const Unit &c : couples) {
+    const int g = pick_gg(c.m, c.n, mean_slot, few) == GWAVE ? 0
+                  : cost8(c.m, c.n) <= lim8 && ceil_div(c.m, 8 * R) <= (int)STRIPS_TOP ? 2  // (fits the unit sort key)
+                                                                                       : 1;
+    pl.list2[g].units.push_back(c);
   }
   for (int k : i32) {
-    if (pick_gg(B->hp[k].la, B->hp[k].lb, mean_slot, few) == GWAVE)
-      add_task(pl, pl.tasks1[0], 1, GWAVE, B->trace, B->hp, k, k, true, B->Kp);
-    else
-      u1.push_back(Unit{k, k, true, B->hp[k].la, B->hp[k].lb});
+    const HostPair &h = B->hp[k];
+    pl.list1[pick_gg(h.la, h.lb, mean_slot, few) == GWAVE ? 0 : 1].units.push_back(Unit{k, k, true, h.la, h.lb});
   }
+  vec_give(couples);
+  vec_give(len);
+  vec_give(i16);
+  vec_give(i32);
+  vec_give(key);
   tr.mark("task kinds");
-  add_units(pl, pl.tasks2[1], 2, G, u2, local, B->trace, B->hp, B->Kp);
-  add_units(pl, pl.tasks2[2], 2, 8, u8, local, B->trace, B->hp, B->Kp);
-  add_units(pl, pl.tasks1[1], 1, G, u1, local, B->trace, B->hp, B->Kp);
+  for (int g = 0; g < 3; ++g) plan_units(pl, pl.list2[g], local, B->trace);
+  for (int g = 0; g < 2; ++g) plan_units(pl, pl.list1[g], local, B->trace);
   tr.mark("wave units");
-  // costlier (more 8-step blocks, S * NB < 2^40) first, stable
-  auto by_cost = [](std::vector<Task> &v) {
-    std::vector<uint64_t> key(v.size());
-    for (size_t t = 0; t < v.size(); ++t) key[t] = (1ull << 40) - (uint64_t)v[t].S * v[t].NB;
-    gather_by_key(v, std::move(key));
-  };
-  by_cost(pl.tasks2[0]);
-  by_cost(pl.tasks1[0]);
   // With few tasks the run lasts as long as its longest whole-wave task, so
   // tasks of two or more strips get a workgroup's fill waves each (strips
   // pipelined across them), as long as there are at most two per CU.
   const char *cenv = getenv("TWEAKALIGN_COOP");  // "0": never
   if (B->walk && few && !(cenv && cenv[0] == '0')) {
-    auto multi = [](const Task &t) { return t.S >= 2; };
-    const size_t c2 = std::count_if(pl.tasks2[0].begin(), pl.tasks2[0].end(), multi);
-    const size_t c1 = std::count_if(pl.tasks1[0].begin(), pl.tasks1[0].end(), multi);
+    auto multi = [](const TaskSpan &t) { return t.S >= 2; };
+    std::vector<TaskSpan> &s2 = pl.list2[0].spans, &s1 = pl.list1[0].spans;
+    const size_t c2 = std::count_if(s2.begin(), s2.end(), multi);
+    const size_t c1 = std::count_if(s1.begin(), s1.end(), multi);
     if (c2 + c1 > 0 && c2 + c1 <= (size_t)(2 * ctx->cus)) {
-      std::stable_partition(pl.tasks2[0].begin(), pl.tasks2[0].end(), multi);
-      std::stable_partition(pl.tasks1[0].begin(), pl.tasks1[0].end(), multi);
+      std::stable_partition(s2.begin(), s2.end(), multi);
+      std::stable_partition(s1.begin(), s1.end(), multi);
       B->ncoop2 = (int32_t)c2;
       B->ncoop1 = (int32_t)c1;
     }
@@ -1541,7 +1682,6 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
       B->longs.push_back(L);
       LongGroup &g = B->lgroups.back();
       g.npairs += 1; g.nitems += L.S; g.ring_n = ring;
-      pl.ptb[k].P = 3;
     }
     if (!lk.empty() && p->traceback) B->long_wgs = std::max(1, std::min((int)lk.size(), 2 * ctx->cus));
     if (const char *e = getenv("TWEAKALIGN_SPIN_LIMIT")) B->spin_limit = std::max(1, atoi(e));
@@ -1557,35 +1697,55 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
     table_nib = nibble_table(B->alph);
     up.add(&B->d_table_nib, table_nib);
   }
-  for (int g = 0; g < 3; ++g) {
-    up.add(&B->d_tasks2[g], pl.tasks2[g]);
-    up.add(&B->d_tasks1[g], pl.tasks1[g]);
+  PlanArgs pa{};
+  int32_t total = 0;
+  Unit *d_units[6] = {nullptr};       // freed after the final drain
+  TaskSpan *d_spans[6] = {nullptr};
+  for (int l = 0; l < 6; ++l) {
+    TaskList &L = l < 3 ? pl.list2[l] : pl.list1[l - 3];
+    pa.list[l].ntasks = L.tasks(); pa.list[l].P = L.P; pa.list[l].GG = L.GG;
+    total += L.tasks();
+    up.add(&d_units[l], L.units);
+    up.add(&d_spans[l], L.spans);
   }
-  up.add(&B->d_ptb, pl.ptb);
-  up.add(&B->d_pairs, B->pairs_h);
-  CodeJob *d_jobs = nullptr;  // freed after the final drain
-  up.add(&d_jobs, pl.cjobs);
-  up.add(&B->d_fo_init, B->fo_init);
-  std::vector<int32_t> order, rest;
-  {
-    std::vector<uint64_t> key(n);  // longer pairs (la + lb <= 2,000,000) first
-    for (int32_t k = 0; k < n; ++k) key[k] = 2000000 - (uint64_t)(B->hp[k].la + B->hp[k].lb);
-    order = order_by_key(std::move(key));
+  std::vector<int32_t> order, rest;  // longer pairs first
+  auto longest_first = [&](std::vector<int32_t> &v) {
+    std::vector<uint64_t> len(v.size());
+    for (size_t t = 0; t < v.size(); ++t) len[t] = 2000000 - (uint64_t)(B->hp[v[t]].la + B->hp[v[t]].lb);
+    gather_by_key(v, len);
+  };
+  if (B->walk || B->strips) {  // pairs without a fill task: empty and long pairs
+    for (int32_t k = 0; k < n; ++k)
+      if (B->hp[k].path == 0 || (B->hp[k].path == 3 && !B->strips)) rest.push_back(k);
+    longest_first(rest);
+    B->n_rest = (int32_t)rest.size();
+    up.add(&B->d_order_rest, rest);
+  } else if (B->trace) {
+    order.resize(n);
+    for (int32_t k = 0; k < n; ++k) order[k] = k;
+    longest_first(order);
     up.add(&B->d_order, order);
-    if (B->walk || B->strips) {  // pairs without a fill task: empty and long pairs
-      for (int32_t k : order)
-        if (B->strips ? B->hp[k].path == 0 : pl.ptb[k].P != 1 && pl.ptb[k].P != 2) rest.push_back(k);
-      B->n_rest = (int32_t)rest.size();
-      up.add(&B->d_order_rest, rest);
-    }
   }
   up.add(&B->d_lp, B->longs);
   up.add(&B->d_litems, B->litems);
   up.add(&B->d_spairs, B->spairs);
   up.add(&B->d_sitems, B->sitems);
   rc = rc ? rc : up.commit(st);
-  rc = rc ? rc : expand_jobs(d_jobs, pl.cjobs.size(), pl.rows_n, pl.cols_n, B->d_pairs, B->d_codes, B->Kp,
-                             &B->d_rowcodes, &B->d_colcodes, st);
+  rc = rc ? rc : dalloc(&B->d_rowcodes, (size_t)pl.rows_n);
+  rc = rc ? rc : dalloc(&B->d_colcodes, (size_t)pl.cols_n);
+  for (int l = 0; l < 6; ++l) {
+    Task **dst = l < 3 ? &B->d_tasks2[l] : &B->d_tasks1[l - 3];
+    rc = rc ? rc : dalloc(dst, (size_t)pa.list[l].ntasks);
+    pa.list[l].units = d_units[l]; pa.list[l].spans = d_spans[l]; pa.list[l].dst = *dst;
+  }
+  if (!rc && total) {
+    pa.trace = B->trace; pa.pad = B->Kp - 1;
+    pa.pairs = B->d_pairs; pa.codes = B->d_codes; pa.ptb = B->d_ptb;
+    pa.rowcodes = B->d_rowcodes; pa.colcodes = B->d_colcodes;
+    (void)hipGetLastError();
+    hipLaunchKernelGGL(plan_tasks_kernel, dim3((unsigned)std::min(total, 65536)), dim3(256), 0, st, pa, total);
+    if (hipGetLastError() != hipSuccess) rc = TA_E_DEVICE;
+  }
   tr.mark("uploads");
   rc = rc ? rc : dalloc(&B->d_ring, pl.ring_elems);
   rc = rc ? rc : dalloc(&B->d_tb, pl.tb_bytes);
@@ -1613,7 +1773,10 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
     rc = TA_E_DEVICE;
   dfree(d_map);
   dfree(d_bad);
-  dfree(d_jobs);
+  for (int l = 0; l < 6; ++l) {
+    dfree(d_units[l]);
+    dfree(d_spans[l]);
+  }
   tr.mark("drain");
   if (!rc && bad_letter) rc = TA_E_ALPHABET;
   if (rc) {
@@ -1645,8 +1808,8 @@ int ta_batch_info(ta_batch *B, int64_t *cells, int64_t *tb_bytes, int32_t *tasks
   if (tb_bytes)
     *tb_bytes = (int64_t)(B->plan.tb_bytes + 4 * kLongPlanes * B->long_wgs + 8 * B->lcol_n + 4 * B->splanes_n);
   if (tasks)
-    *tasks = (int32_t)(B->plan.tasks2[0].size() + B->plan.tasks2[1].size() + B->plan.tasks2[2].size() +
-                       B->plan.tasks1[0].size() + B->plan.tasks1[1].size() + B->litems.size() + B->sitems.size());
+    *tasks = (int32_t)(B->plan.list2[0].tasks() + B->plan.list2[1].tasks() + B->plan.list2[2].tasks() +
+                       B->plan.list1[0].tasks() + B->plan.list1[1].tasks() + B->litems.size() + B->sitems.size());
   return TA_OK;
 }
 
@@ -1840,20 +2003,21 @@ int rerun_saturated(ta_ctx *ctx, ta_batch *B) {
   free_rerun(B);
   if (bad.empty()) return TA_OK;
   Plan pl;
-  pl.ptb = B->plan.ptb;
+  pl.ptb.resize(B->n);
+  std::vector<Task> wave, group;
   std::vector<Unit> u;
   for (int k : bad) {
     if (pick_gg(B->hp[k].la, B->hp[k].lb, 0.0, bad.size() <= (size_t)ctx->cus * 4) == GWAVE) {
-      add_task(pl, pl.tasks1[0], 1, GWAVE, B->trace, B->hp, k, k, true, B->Kp);
-      pl.tasks1[0].back().flags_or = TA_F_RERUN;
+      add_task(pl, wave, 1, GWAVE, B->trace, B->hp, k, k, true);
+      wave.back().flags_or = TA_F_RERUN;
     } else {
       u.push_back(Unit{k, k, true, B->hp[k].la, B->hp[k].lb});
     }
   }
-  add_units(pl, pl.tasks1[1], 1, G, u, B->p.mode == TA_LOCAL, B->trace, B->hp, B->Kp);
-  for (Task &t : pl.tasks1[1]) t.flags_or = TA_F_RERUN;
-  std::vector<Task> all(pl.tasks1[0]);
-  all.insert(all.end(), pl.tasks1[1].begin(), pl.tasks1[1].end());
+  add_units(pl, group, u, B->p.mode == TA_LOCAL, B->trace, B->hp);
+  for (Task &t : group) t.flags_or = TA_F_RERUN;
+  std::vector<Task> all(wave);
+  all.insert(all.end(), group.begin(), group.end());
   hipStream_t st = B->stream;
   int rc = TA_OK;
   rc = rc ? rc : upload(&B->d_tasks_r, all, st);
@@ -1865,15 +2029,17 @@ int rerun_saturated(ta_ctx *ctx, ta_batch *B) {
   B->n_rerun = (int)bad.size();
   // Rerun pairs read their planes from the rerun arena: point their PairTB there
   // by offsetting against the main arena base.
-  std::vector<PairTB> ptb(B->plan.ptb);
+  std::vector<PairTB> ptb(B->n);
+  HIPCHK(hipMemcpyAsync(ptb.data(), B->d_ptb, sizeof(PairTB) * B->n, hipMemcpyDeviceToHost, st));
+  HIPCHK(hipStreamSynchronize(st));
   for (int k : bad) {
     ptb[k] = pl.ptb[k];
     ptb[k].tb_off += (uint64_t)(B->d_tb_r - B->d_tb);
   }
   HIPCHK(hipMemcpyAsync(B->d_ptb, ptb.data(), sizeof(PairTB) * B->n, hipMemcpyHostToDevice, st));
   HIPCHK(hipMemsetAsync(B->d_ctr + 4, 0, 2 * sizeof(int32_t), st));
-  Task *const tk[3] = {B->d_tasks_r, B->d_tasks_r + pl.tasks1[0].size(), nullptr};
-  const int nt[3] = {(int)pl.tasks1[0].size(), (int)pl.tasks1[1].size() / NGW, 0};
+  Task *const tk[3] = {B->d_tasks_r, B->d_tasks_r + wave.size(), nullptr};
+  const int nt[3] = {(int)wave.size(), (int)group.size() / NGW, 0};
   return launch_fill<1>(ctx, B, tk, nt, B->d_rowcodes_r, B->d_colcodes_r, B->d_ring_r, B->d_tb_r, B->d_ctr + 4, 0);
 }
 
@@ -1891,8 +2057,8 @@ int launch_init(ta_batch *B) {
 
 int launch_fills(ta_ctx *ctx, ta_batch *B) {
   const Plan &pl = B->plan;
-  const int n2[3] = {(int)pl.tasks2[0].size(), (int)pl.tasks2[1].size() / NGW, (int)pl.tasks2[2].size() / 8};
-  const int n1[3] = {(int)pl.tasks1[0].size(), (int)pl.tasks1[1].size() / NGW, 0};
+  const int n2[3] = {(int)pl.list2[0].spans.size(), (int)pl.list2[1].spans.size(), (int)pl.list2[2].spans.size()};
+  const int n1[3] = {(int)pl.list1[0].spans.size(), (int)pl.list1[1].spans.size(), 0};
   int rc = launch_fill<2>(ctx, B, B->d_tasks2, n2, B->d_rowcodes, B->d_colcodes, B->d_ring, B->d_tb, B->d_ctr, 0,
                           B->walk);
   if (!rc) rc = launch_fill<1>(ctx, B, B->d_tasks1, n1, B->d_rowcodes, B->d_colcodes, B->d_ring, B->d_tb,
@@ -2062,7 +2228,6 @@ struct Fetched {
 };
 
 int fetch_results(ta_batch *B, Fetched &F) {
-  F.off.assign(B->n, 0);
   std::vector<int64_t> &off = F.off;
   hipStream_t st = B->stream;
   if (B->n) {
@@ -2076,6 +2241,7 @@ int fetch_results(ta_batch *B, Fetched &F) {
   HIPCHK(hipStreamSynchronize(st));
   if (!B->p.traceback) return TA_OK;
   const ResultDev *res = F.res;
+  off.assign(B->n, 0);
   int64_t total = 0;
   for (int32_t k = 0; k < B->n; ++k) {
     off[k] = total;
@@ -2141,7 +2307,7 @@ int ta_batch_results(ta_ctx *ctx, ta_batch *B, ta_result *out, char *cigar_buf, 
   }
   if (used) *used = pos;
   if (pos > 0 && (!cigar_buf || pos > cap)) return TA_E_SPACE;
-  parallel_for((size_t)B->n, [&](size_t k) {
+  if (pos > 0) parallel_for((size_t)B->n, [&](size_t k) {
     if (out[k].cigar_len > 0)
       format_runs(runs + off[k] / 4, res[k].cigar_len / 4, cigar_buf + out[k].cigar_off);
   });
@@ -2369,12 +2535,12 @@ int ta_batch_run_plain(ta_ctx *ctx, ta_batch *B, int32_t first, int32_t count) {
         pl.tb_bytes = tb0; pl.ring_elems = r0;
         fill_unit(v);
       };
-      add_task(pl, tasks, P, GG, B->trace, B->hp, k, k, true, B->Kp);
+      add_task(pl, tasks, P, GG, B->trace, B->hp, k, k, true);
       rebase(tasks);
       if (h.maysat) {  // the int32 task a saturated int16 fill reruns as
         const PairTB p16 = pl.ptb[k];
         rerun_of[k] = (int32_t)rtasks.size();
-        add_task(pl, rtasks, 1, GG, B->trace, B->hp, k, k, true, B->Kp);
+        add_task(pl, rtasks, 1, GG, B->trace, B->hp, k, k, true);
         rtasks.back().flags_or = TA_F_RERUN;
         rebase(rtasks);
         ptb_r[k] = pl.ptb[k];
