@@ -984,6 +984,7 @@ struct ta_batch {
   int8_t *d_table = nullptr;
   int8_t *d_table_nib = nullptr;  // packed couples: 4-bit biased scores
   bool nib = false;
+  bool shift = false;             // packed couples, score only: shifted values fit (shift_fits)
   int fill_waves = 0;             // resident fill waves per CU (0: default_waves)
   bool wave_tasks = false;        // whole-wave groups for every multi-strip task
   Task *d_tasks2[3] = {nullptr, nullptr, nullptr}, *d_tasks1[3] = {nullptr, nullptr, nullptr};
@@ -1110,6 +1111,20 @@ void ta_batch_destroy(ta_batch *B) {
     vec_give(B->plan.list1[g].spans);
   }
   delete B;
+}
+
+// Origin of a shifted fill's values, which makes the lowest one -32,700.
+static int shift_base(const ta_params &p) { return -32700 - 3 * (p.gap_open - p.gap_extend); }
+
+// Whether score-only global couples take the shifted fill: it takes 26% fewer
+// instructions and is the faster one wherever its values fit.  Opening must
+// cost at least extending (or gaps raise the values), and the nibbles'
+// constant must be a byte's (0..240).  A pair that global_i16_safe admits
+// has 3 |open| + (la + lb) |ext| < 16,000 and min(la, lb) max S < 32,000, so
+// its largest value is below -32,700 + 48,000.
+static bool shift_fits(const ta_params &p, const Alphabet &A) {
+  const int k0 = A.minS - p.gap_open - p.gap_extend;
+  return p.gap_open <= p.gap_extend && k0 >= 0 && k0 <= 240;
 }
 
 // A pair the batch runtime takes: lengths in range, letters present, and
@@ -1506,6 +1521,7 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
     }
   });
   for (const Share &s : shares) B->may_saturate = B->may_saturate || s.maysat;
+  B->shift = B->nib && !B->trace && shift_fits(*p, B->alph);
   rc = rc ? rc : dalloc(&B->d_pairs, (size_t)std::max(n, 1));
   rc = rc ? rc : dalloc(&B->d_fo_init, (size_t)std::max(n, 1));
   rc = rc ? rc : dalloc(&B->d_ptb, (size_t)std::max(n, 1));
@@ -1846,6 +1862,7 @@ int launch_fill(ta_ctx *ctx, ta_batch *B, Task *const d_tasks[3], const int ntas
   a.ctr8 = B->d_ctr + (P == 2 ? 14 : 15);  // 8-lane units come only from the batch plan
   a.table = nib ? B->d_table_nib : B->d_table; a.Kp = B->Kp;
   a.bias = -B->alph.minS;
+  a.shift_base = shift_base(B->p);
   a.rowcodes = rows; a.colcodes = cols; a.ring = ring; a.tb = tb; a.out = B->d_fo;
   a.open = B->p.gap_open; a.ext = B->p.gap_extend;
   a.sat_limit = 32767 - 2 * B->alph.maxS;
@@ -1868,7 +1885,8 @@ int launch_fill(ta_ctx *ctx, ta_batch *B, Task *const d_tasks[3], const int ntas
   const bool local = B->p.mode == TA_LOCAL;
   void (*k)(FillArgs) = nullptr;
   if (local) k = B->trace ? fill_kernel<P, true, true> : fill_kernel<P, true, false>;
-  else k = B->trace ? fill_kernel<P, false, true> : fill_kernel<P, false, false>;
+  else k = B->trace ? fill_kernel<P, false, true> : fill_kernel<P, false, false, false>;
+  if (P == 2 && B->shift) k = fill_kernel<2, false, false, true>;
   (void)hipGetLastError();  // drop an earlier, already-handled error
   hipLaunchKernelGGL(k, dim3(groups), dim3(walk ? 128 * WALK_FW : 64), lds, B->stream, a);
   HIPCHK(hipGetLastError());
