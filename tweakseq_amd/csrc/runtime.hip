@@ -612,18 +612,18 @@ __global__ void encode_kernel(uint4 *codes, size_t words, const uint8_t *map, in
   if (__any(any & 0x80) && (threadIdx.x & 63) == 0) atomicOr(bad, 1);
 }
 
-// The row and column codes of a task (pairs A, B), expanded by a workgroup
-// from the uploaded residues: row r of a half is its pair's query residue r
+// The row and column codes of a task (pairs A, B), expanded by threads
+// tid < nthr from the uploaded residues: row r of a half is its pair's query residue r
 // (pad past m), column j its reference residue j - off (pad before the
 // leading columns and past n).
 __device__ __forceinline__ void expand_job(const CodeJob &c, const PairDev &A, const PairDev &B, const uint8_t *codes,
-                                           int pad, uint16_t *rowcodes, uint16_t *colcodes) {
-  for (int r = threadIdx.x; r < c.nrows; r += blockDim.x) {
+                                           int pad, uint16_t *rowcodes, uint16_t *colcodes, int tid, int nthr) {
+  for (int r = tid; r < c.nrows; r += nthr) {
     const int ca = r < A.la ? codes[A.a_off + r] : pad;
     const int cb = r < B.la ? codes[B.a_off + r] : pad;
     rowcodes[c.row_off + r] = (uint16_t)(ca | (cb << 8));
   }
-  for (int j = threadIdx.x; j < c.ncol; j += blockDim.x) {
+  for (int j = tid; j < c.ncol; j += nthr) {
     const int ja = j - c.off0, jb = j - c.off1;
     const int ca = (ja >= 0 && ja < A.lb) ? codes[A.b_off + ja] : pad;
     const int cb = (jb >= 0 && jb < B.lb) ? codes[B.b_off + jb] : pad;
@@ -636,7 +636,7 @@ __global__ void expand_codes_kernel(const CodeJob *jobs, int njobs, const PairDe
                                     int pad, uint16_t *rowcodes, uint16_t *colcodes) {
   for (int q = blockIdx.x; q < njobs; q += gridDim.x) {
     const CodeJob c = jobs[q];
-    expand_job(c, pairs[c.lo], pairs[c.hi], codes, pad, rowcodes, colcodes);
+    expand_job(c, pairs[c.lo], pairs[c.hi], codes, pad, rowcodes, colcodes, threadIdx.x, blockDim.x);
   }
 }
 
@@ -735,7 +735,8 @@ __global__ void pairs_init_kernel(const PairDev *pairs, int n, FillOut *fo, Pair
 }
 
 // The planned tasks, their pairs' direction-plane records and their row and
-// column codes, a workgroup per task.  The host plans spans only (shapes,
+// column codes, a wave per task (a workgroup each took 132 us: a chain of
+// dependent reads before a few codes a thread).  The host plans spans only (shapes,
 // offsets, which units): tasks, code jobs and records written there and
 // copied over were 15 of the 20 MB that the creation of a batch of 130,816
 // pairs wrote and sent.  With the pairs' table written by the host threads
@@ -755,8 +756,9 @@ struct PlanArgs {
   uint16_t *rowcodes, *colcodes;
 };
 __global__ __launch_bounds__(256) void plan_tasks_kernel(PlanArgs A, int total) {
-  for (int x = blockIdx.x; x < total; x += gridDim.x) {
-    int q = x, l = 0;
+  const int lane = threadIdx.x & 63;
+  for (int x = blockIdx.x * 4 + (int)(threadIdx.x >> 6); x < total; x += 4 * gridDim.x) {
+    int q = __builtin_amdgcn_readfirstlane(x), l = 0;
     while (q >= A.list[l].ntasks) q -= A.list[l++].ntasks;
     const PlanArgs::List &L = A.list[l];
     const int NG = GWAVE / L.GG, i = q % NG;
@@ -771,7 +773,7 @@ __global__ __launch_bounds__(256) void plan_tasks_kernel(PlanArgs A, int total) 
     const int la[2] = {a.la, b.la}, lb[2] = {a.lb, b.lb};
     Task T = make_task(at, L.GG, A.trace, u.lo, u.hi, la, lb, u.single, s.n, s.S);
     if (filler) T.single = 2;
-    if (threadIdx.x == 0) {
+    if (lane == 0) {
       L.dst[q] = T;
       if (!filler) {
         A.ptb[u.lo] = task_ptb(T, L.P, L.GG, 0);
@@ -780,7 +782,7 @@ __global__ __launch_bounds__(256) void plan_tasks_kernel(PlanArgs A, int total) 
     }
     if (filler) continue;
     const CodeJob c{T.row_off, T.col_off, T.S * L.GG * R, 8 * T.NB + 8, u.lo, u.hi, T.off[0], T.off[1]};
-    expand_job(c, a, b, A.codes, A.pad, A.rowcodes, A.colcodes);
+    expand_job(c, a, b, A.codes, A.pad, A.rowcodes, A.colcodes, lane, 64);
   }
 }
 
@@ -1759,7 +1761,7 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
     pa.pairs = B->d_pairs; pa.codes = B->d_codes; pa.ptb = B->d_ptb;
     pa.rowcodes = B->d_rowcodes; pa.colcodes = B->d_colcodes;
     (void)hipGetLastError();
-    hipLaunchKernelGGL(plan_tasks_kernel, dim3((unsigned)std::min(total, 65536)), dim3(256), 0, st, pa, total);
+    hipLaunchKernelGGL(plan_tasks_kernel, dim3((unsigned)std::min((total + 3) / 4, 65536)), dim3(256), 0, st, pa, total);
     if (hipGetLastError() != hipSuccess) rc = TA_E_DEVICE;
   }
   tr.mark("uploads");
