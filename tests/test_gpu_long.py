@@ -205,3 +205,21 @@ def test_region_and_checkpoint_edges(eng, la, lb):
     for go, ge, ma, mi in ((-5, -2, 2, -3), (-2, -9, 2, -3), (0, 0, 1, -1), (-100, -60, 90, -90)):
         run_check(eng, pairs, "regions %d %d" % (go, ge), lanes=ta.LANES_LONG, mode=ta.GLOBAL, alphabet=ta.DNA,
                   gap_open=go, gap_extend=ge, match=ma, mismatch=mi)
+
+
+@pytest.mark.parametrize("npairs", [200, 700])
+def test_regions_ahead_and_not(eng, npairs):
+    # pairs of one to three forward strips: with fewer strips than CUs times the longest pair's the regions are
+    # computed ahead, with more each pair computes its own; shifted, repetitive and unrelated second sequences
+    # put the path off the guesses
+    rng = random.Random(npairs)
+    pairs = []
+    for k in range(npairs):
+        a = "".join(rng.choice("ACGT") for _ in range(rng.choice((60, 512, 513, 700)) if npairs > 200 else
+                                                      rng.choice((511, 1025, 1500))))
+        cut = rng.randint(0, len(a))
+        junk = "".join(rng.choice("ACGT") for _ in range(rng.randint(1, 600)))
+        b = (a[:cut] + junk + a[cut:], a[cut:] + junk, junk, "A" * 300 + a, a[:64] * 9)[k % 5]
+        pairs.append((a, b) if k % 2 else (b, a))
+    run_check(eng, pairs, "ahead %d" % npairs, lanes=ta.LANES_LONG, mode=ta.GLOBAL, alphabet=ta.DNA, gap_open=-6,
+              gap_extend=-1)

@@ -27,10 +27,21 @@
 // is columns + 64 strips of dependent steps, and the columns beyond the
 // diagonal (LMARGIN, half a CKX) are what a region computes for nothing.
 //
+// One after the other, the regions of the longest pair (120 us each) would set
+// the time of a batch of few pairs.  So where the path will pass is guessed
+// first: at every strip's bottom row, the column of the largest H near the
+// diagonal (long_cross_kernel) -- for related sequences on the path, or next
+// to it.  A region around every guess is recomputed by a workgroup of its own
+// (long_regions_kernel), all over the GPU at once, and the walk uses such a
+// region wherever it contains the walk's cell (a region's codes are exact
+// whatever made it), else recomputes one itself as above.  Batches whose
+// pairs fill the GPU by themselves do without.
+//
 // 48 DNA pairs of 10,000 to 60,000 with CIGARs: forward 36 -> 19 ms, traceback
-// 63 -> 17 ms; 256 of 10,000 to 100,000: 449 -> 277 ms a run.  (Before: plain
-// recurrence, progress counters every 64 columns, regions of 4,096 rows on 8
-// waves, a walk of one thread.)
+// 63 -> 17 ms with small regions and run walks, -> 2.8 ms with regions ahead;
+// 256 of 10,000 to 100,000: 449 -> 277 -> 242 ms a run.  (Before: plain recurrence,
+// progress counters every 64 columns, regions of 4,096 rows on 8 waves, a walk
+// of one thread.)
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -49,12 +60,16 @@ constexpr int LMARGIN = 256;              // region columns beyond the diagonal 
 constexpr int LREG = LST + LMARGIN + CKX; // columns of a region at most
 constexpr int LREG_T = (LREG + 63 + 7) & ~7;
 constexpr int LTW = LST / 128;            // waves of a traceback workgroup: strips of a region
+constexpr int LAHEAD = 128;               // columns of a region ahead on either side of its guesses
+constexpr int LGUESS = 8192;              // columns on either side of the diagonal a guess is looked for in
+constexpr size_t LPLANES = (size_t)LTW * LREG_T / strip_spd(2) * 64;  // dwords of a region's codes
 
 struct LongPair {
   uint64_t a_off, b_off;  // residue codes (16-byte aligned, 32 bytes readable past the end)
   uint64_t ring;          // (G, F) entries: S - 1 rows of T + 8
   uint64_t colck;         // (G, E) entries: (n - 1) / CKX columns x S * LST rows
   int32_t pid, m, n, S, T;
+  int32_t item0;          // its first queue item
 };
 
 struct LongItem {
@@ -71,7 +86,10 @@ struct LongArgs {
   int32_t Kp;
   const uint8_t *codes;
   int2 *ring, *colck;
-  uint32_t *wpl;        // traceback workgroups: direction codes, LTW * LREG_T / 4 * 64 dwords each
+  uint32_t *wpl;        // traceback workgroups: direction codes, LPLANES dwords each
+  uint32_t *ahead;      // codes of the regions ahead, an item's at LPLANES (item - ahead0); null: none
+  int32_t *cross;       // per item: the column (1-based) its strip's bottom row is guessed to be left at
+  int32_t ahead0;
   const PairDev *pd;
   FillOut *fo;
   ResultDev *res;
@@ -195,28 +213,157 @@ __global__ __launch_bounds__(64, 2) void long_fwd_kernel(LongArgs A) {
   }
 }
 
-// LDS of a traceback workgroup.
+// LDS of a traceback workgroup.  Its strips share one ring: each stores its
+// bottom row over the one it read, 63 columns behind.
 enum { LT_TAB = 0, LT_SYNC = 1024, LT_SLOTS = 1280, LT_CODES = LT_SLOTS + LTW * strip_slot_bytes(2),
-       LT_RINGS = LT_CODES + ((64 + LREG_T + 32 + 15) & ~15), LT_RING = (LREG_T + 80) * 8,
-       LT_WIN = LT_RINGS + LTW * LT_RING, LONG_TB_LDS = LT_WIN + StripWindow<2>::WL * StripWindow<2>::WD * 4 };
+       LT_RING = LT_CODES + ((64 + LREG_T + 32 + 15) & ~15), LT_WIN = LT_RING + (LREG_T + 80) * 8,
+       LONG_TB_LDS = LT_WIN + StripWindow<2>::WL * StripWindow<2>::WD * 4 };
 // Its sync words.
 enum { LS_PAIR = 0, LS_I = 1, LS_J = 2, LS_PROG = 4, LS_READY = 25, LS_ZERO = 32, LS_EDGE = 48 };
 
-// Traceback: one workgroup of LTW waves per pair (pairs off a counter).
-template <int = 0>
-__global__ __launch_bounds__(64 * LTW) void long_tb_kernel(LongArgs A) {
-  extern __shared__ __align__(256) uint8_t lds[];
+// What a traceback workgroup's regions share.
+__device__ __forceinline__ void long_tb_setup(const LongArgs &A, uint8_t *lds, int32_t *sy) {
   static_assert(LT_SLOTS % STRIP_ROW == 0 && LT_SLOTS + LTW * strip_slot_bytes(2) <= 256 * STRIP_ROW, "slot rows");
-  int32_t *sy = (int32_t *)(lds + LT_SYNC);
-  uint8_t *bcode = lds + LT_CODES;
-  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), K = A.Kp - 1;
-  uint32_t *pl = A.wpl + (uint64_t)blockIdx.x * (LTW * LREG_T / strip_spd(2) * 64);
+  const int tid = threadIdx.x, K = A.Kp - 1;
   for (int x = tid; x < 1024; x += 64 * LTW) {
     const int r = x >> 5, c = x & 31;
     lds[LT_TAB + x] = r < K && c < K ? (uint8_t)A.table[r * A.Kp + c] : (uint8_t)PAD_SCORE;
   }
   if (tid < 64) sy[tid] = tid == LS_READY ? 0x7fffffff : tid >= LS_EDGE ? 2 * (A.open - A.ext) : 0;
-  if (tid < 64) bcode[tid] = (uint8_t)K;
+  if (tid < 64) lds[LT_CODES + tid] = (uint8_t)K;
+}
+
+// A region's codes: rows of strip beta up to row i (1-based), columns
+// c_left + 1 .. c_left + ncols (c_left: 0 or a checkpoint), by the workgroup.
+__device__ __forceinline__ void long_region(const LongArgs &A, const LongPair &P, uint8_t *lds, int32_t *sy, int beta,
+                                            int i, int c_left, int ncols, uint32_t *pl, bool &lost) {
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), K = A.Kp - 1;
+  const int top = beta * LST, T = (ncols + 63 + 7) & ~7, S = (i - top + 127) / 128;
+  uint8_t *bcode = lds + LT_CODES;
+  int2 *ring = (int2 *)(lds + LT_RING);
+  const uint8_t *cb = A.codes + P.b_off + c_left;
+  for (int x = 4 * tid; x < T + 16; x += 256 * LTW) {
+    const int left = ncols - x;
+    const uint32_t keep = left >= 4 ? 0xffffffffu : left <= 0 ? 0u : (1u << (8 * left)) - 1u;
+    *(uint32_t *)(bcode + 64 + x) =
+        ((left > 0 ? *(const uint32_t *)(cb + x) : 0u) & keep) | ((0x01010101u * (uint32_t)K) & ~keep);
+  }
+  if (beta) {  // the row above: the forward strip's bottom row
+    const int2 *row = A.ring + P.ring + (uint64_t)(beta - 1) * (P.T + 8) + c_left;
+    for (int x = tid; x < ncols; x += 64 * LTW) ring[64 + x] = row[x];
+  }
+  if (tid < LTW) sy[LS_PROG + tid] = 0;
+  __syncthreads();
+  if (wv < S) {
+    const int sa = top / 128 + wv, r0 = (sa * 64 + lane) * 2;  // strips of 128 rows, counted over the pair
+    const uint8_t *line[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) line[k] = lds + LT_TAB + 32 * (r0 + k < P.m ? A.codes[P.a_off + r0 + k] : 31);
+    const int slot = LT_SLOTS + wv * strip_slot_bytes(2);
+    strip_slot<2>(lds + slot, line, K, -A.open - A.ext, A.ext - A.open);
+    struct IO : StripGroupIO {
+      const int2 *left;
+    } io;
+    io.left = c_left ? A.colck + P.colck + (uint64_t)(c_left / CKX - 1) * P.S * LST + r0 : nullptr;
+    io.bcode = bcode + 64 - lane;
+    io.slot_add = 0x01010101u * ((uint32_t)((uint32_t)(uintptr_t)(lds_u8 *)lds + slot) >> 8);
+    io.status = A.err;
+    io.gave_up = 1;
+    io.spin_limit = 1 << 22;
+    io.lost = lost;
+    io.pin = sy + (wv ? LS_PROG + wv - 1 : LS_READY);
+    io.pout = sy + LS_PROG + wv;
+    io.rin = lane ? (int2 *)(sy + LS_ZERO) : wv || beta ? ring + 64 : (int2 *)(sy + LS_EDGE);
+    io.rin_step = lane == 0 && (wv || beta) ? 8 : 0;
+    io.rout = ring;
+    io.need0 = wv << 20;
+    io.s = wv;
+    io.cols = T - 63;
+    io.pl = pl + (uint64_t)wv * (T / strip_spd(2)) * 64 + lane;
+    io.pl_step = 64;
+    asm volatile("" ::: "memory");  // staged by all lanes (a wave's LDS accesses keep their order)
+    StripEnd end;
+    strip_sweep<2, false>(io, sa, wv + 1 == S, i, ncols, T, A.open, A.ext, end);
+    lost = io.lost;
+  }
+  __syncthreads();  // the codes are in place
+}
+
+// The columns of the region ahead of strip beta (item x): from a checkpoint
+// left of where the strip above is guessed to be left, to right of this one's
+// guess, at most LREG of them.
+__device__ __forceinline__ void long_ahead_cols(const LongArgs &A, const LongPair &P, int beta, int &c_left, int &right) {
+  const int32_t *cross = A.cross + P.item0 + beta;
+  const int here = cross[0], up = beta ? cross[-1] : 0;
+  right = here + LAHEAD < P.n ? here + LAHEAD : P.n;
+  const int from = (up < here ? up : here) - LAHEAD;
+  c_left = from <= 0 ? 0 : from / CKX * CKX;
+  if (right - c_left > LREG) c_left = (right - LREG + CKX - 1) / CKX * CKX;
+}
+
+// Guesses: per queue item, the column of the largest H of its strip's bottom
+// row near the diagonal (the last strip's: n).  Also clears the pair counter
+// of the traceback that follows.
+template <int = 0>
+__global__ __launch_bounds__(256) void long_cross_kernel(LongArgs A) {
+  __shared__ int2 part[4];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const LongItem it = A.items[blockIdx.x];
+  const LongPair P = A.lp[it.lp];
+  if (blockIdx.x == 0 && tid == 0) A.ctr[1] = 0;
+  if (it.s == P.S - 1) {
+    if (tid == 0) A.cross[P.item0 + it.s] = P.n;
+    return;
+  }
+  const int2 *row = A.ring + P.ring + (uint64_t)it.s * (P.T + 8);
+  const int mid = (int)((int64_t)P.n * (it.s + 1) * LST / P.m);
+  const int lo = mid > LGUESS ? mid - LGUESS : 0, hi = mid + LGUESS < P.n ? mid + LGUESS : P.n;
+  int best = INT32_MIN, col = lo;
+  for (int x = lo + tid; x < hi; x += 256) {
+    const int h = row[x].x + A.ext * x;
+    if (h > best) { best = h; col = x; }
+  }
+  auto join = [&](int h, int c) {
+    if (h > best || (h == best && c < col)) { best = h; col = c; }
+  };
+#pragma unroll
+  for (int w = 32; w >= 1; w >>= 1) {
+    const int h = __shfl_xor(best, w, 64), c = __shfl_xor(col, w, 64);
+    join(h, c);
+  }
+  if (lane == 0) part[tid >> 6] = make_int2(best, col);
+  __syncthreads();
+  if (tid == 0) {
+    for (int w = 1; w < 4; ++w) join(part[w].x, part[w].y);
+    A.cross[P.item0 + it.s] = col + 1;
+  }
+}
+
+// The regions ahead, a workgroup per queue item.
+template <int = 0>
+__global__ __launch_bounds__(64 * LTW, 4) void long_regions_kernel(LongArgs A) {
+  extern __shared__ __align__(256) uint8_t lds[];
+  int32_t *sy = (int32_t *)(lds + LT_SYNC);
+  const LongItem it = A.items[blockIdx.x];
+  const LongPair P = A.lp[it.lp];
+  long_tb_setup(A, lds, sy);
+  __syncthreads();
+  int c_left, right;
+  long_ahead_cols(A, P, it.s, c_left, right);
+  const int i = (it.s + 1) * LST < P.m ? (it.s + 1) * LST : P.m;
+  bool lost = false;
+  long_region(A, P, lds, sy, it.s, i, c_left, right - c_left, A.ahead + (uint64_t)(P.item0 + it.s - A.ahead0) * LPLANES,
+              lost);
+}
+
+// Traceback: one workgroup of LTW waves per pair (pairs off a counter).
+template <int = 0>
+__global__ __launch_bounds__(64 * LTW) void long_tb_kernel(LongArgs A) {
+  extern __shared__ __align__(256) uint8_t lds[];
+  int32_t *sy = (int32_t *)(lds + LT_SYNC);
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  uint32_t *const own = A.wpl + (uint64_t)blockIdx.x * LPLANES;
+  long_tb_setup(A, lds, sy);
   bool lost = false;
   for (;;) {
     __syncthreads();
@@ -232,59 +379,22 @@ __global__ __launch_bounds__(64 * LTW) void long_tb_kernel(LongArgs A) {
     int i = P.m, j = P.n, state = 0;
     bool failed = false;
     while (i > 0 && j > 0) {
-      // Region: rows of the strip holding row i, columns c_left + 1 .. j.
+      // Region: rows of the strip holding row i, columns c_left + 1 .. j (or more).
       const int beta = (i - 1) / LST, top = beta * LST;
-      int c_left = j - (i - top) - LMARGIN;
-      c_left = c_left <= 0 ? 0 : (c_left / CKX) * CKX;
-      const int ncols = j - c_left, T = (ncols + 63 + 7) & ~7, S = (i - top + 127) / 128;
-      const uint8_t *cb = A.codes + P.b_off + c_left;
-      for (int x = 4 * tid; x < T + 16; x += 256 * LTW) {
-        const int left = ncols - x;
-        const uint32_t keep = left >= 4 ? 0xffffffffu : left <= 0 ? 0u : (1u << (8 * left)) - 1u;
-        *(uint32_t *)(bcode + 64 + x) =
-            ((left > 0 ? *(const uint32_t *)(cb + x) : 0u) & keep) | ((0x01010101u * (uint32_t)K) & ~keep);
+      int c_left = 0, right = 0;
+      const uint32_t *pl = own;
+      if (A.ahead) {
+        long_ahead_cols(A, P, beta, c_left, right);
+        pl = A.ahead + (uint64_t)(P.item0 + beta - A.ahead0) * LPLANES;
       }
-      if (beta) {  // the row above: the forward strip's bottom row
-        const int2 *row = A.ring + P.ring + (uint64_t)(beta - 1) * (P.T + 8) + c_left;
-        int2 *ring = (int2 *)(lds + LT_RINGS) + 64;
-        for (int x = tid; x < ncols; x += 64 * LTW) ring[x] = row[x];
+      if (j <= c_left || j > right) {  // no region ahead, or not this cell in it
+        c_left = j - (i - top) - LMARGIN;
+        c_left = c_left <= 0 ? 0 : (c_left / CKX) * CKX;
+        right = j;
+        pl = own;
+        long_region(A, P, lds, sy, beta, i, c_left, right - c_left, own, lost);
       }
-      if (tid < LTW) sy[LS_PROG + tid] = 0;
-      __syncthreads();
-      if (wv < S) {
-        const int sa = top / 128 + wv, r0 = (sa * 64 + lane) * 2;  // strips of 128 rows, counted over the pair
-        const uint8_t *line[2];
-#pragma unroll
-        for (int k = 0; k < 2; ++k) line[k] = lds + LT_TAB + 32 * (r0 + k < P.m ? A.codes[P.a_off + r0 + k] : 31);
-        const int slot = LT_SLOTS + wv * strip_slot_bytes(2);
-        strip_slot<2>(lds + slot, line, K, -A.open - A.ext, A.ext - A.open);
-        struct IO : StripGroupIO {
-          const int2 *left;
-        } io;
-        io.left = c_left ? A.colck + P.colck + (uint64_t)(c_left / CKX - 1) * P.S * LST + r0 : nullptr;
-        io.bcode = bcode + 64 - lane;
-        io.slot_add = 0x01010101u * ((uint32_t)((uint32_t)(uintptr_t)(lds_u8 *)lds + slot) >> 8);
-        io.status = A.err;
-        io.gave_up = 1;
-        io.spin_limit = 1 << 22;
-        io.lost = lost;
-        io.pin = sy + (wv ? LS_PROG + wv - 1 : LS_READY);
-        io.pout = sy + LS_PROG + wv;
-        io.rin = lane ? (int2 *)(sy + LS_ZERO)
-                      : wv || beta ? (int2 *)(lds + LT_RINGS + wv * LT_RING) + 64 : (int2 *)(sy + LS_EDGE);
-        io.rin_step = lane == 0 && (wv || beta) ? 8 : 0;
-        io.rout = (int2 *)(lds + LT_RINGS + (wv + 1) * LT_RING);
-        io.need0 = wv << 20;
-        io.s = wv;
-        io.cols = T - 63;
-        io.pl = pl + (uint64_t)wv * (T / strip_spd(2)) * 64 + lane;
-        io.pl_step = 64;
-        asm volatile("" ::: "memory");  // staged by all lanes (a wave's LDS accesses keep their order)
-        StripEnd end;
-        strip_sweep<2, false>(io, sa, wv + 1 == S, i, ncols, T, A.open, A.ext, end);
-        lost = io.lost;
-      }
-      __syncthreads();  // the codes are in place
+      const int T = (right - c_left + 63 + 7) & ~7;
       if (wv == 0) {
         StripWindow<2> src{pl, (uint32_t *)(lds + LT_WIN), T, -1, -1};
         int li = i - top, lj = j - c_left, h = 0, steps = 0;

@@ -520,8 +520,8 @@ int64_t long_estimate(const std::vector<HostPair> &hp, const std::vector<int> &l
   return t;
 }
 
-// Dwords of region codes of a long-pair traceback workgroup.
-constexpr size_t kLongPlanes = (size_t)LTW * LREG_T / strip_spd(2) * 64;
+// Regions a long-pair traceback computes ahead at most (344 KB each).
+constexpr int kLongAhead = 32768;
 
 // Residue codes one task's strips and columns read (expand_codes_kernel).
 struct CodeJob {
@@ -1008,12 +1008,15 @@ struct ta_batch {
   // long-pair pipeline
   std::vector<LongPair> longs;
   std::vector<LongItem> litems;
-  std::vector<int32_t> litem_first;  // per long pair: its first queue item
   std::vector<LongGroup> lgroups;
   LongPair *d_lp = nullptr;
   LongItem *d_litems = nullptr;
   int2 *d_lring = nullptr, *d_lcol = nullptr;
   uint32_t *d_wpl = nullptr;  // region codes of the traceback workgroups
+  // Regions computed ahead (0: none), and the guesses they are placed by.
+  int32_t lahead = 0;
+  uint32_t *d_lahead = nullptr;
+  int32_t *d_lcross = nullptr;
   uint64_t lring_n = 0, lcol_n = 0;
   int32_t long_wgs = 0, spin_limit = 1 << 20;  // about a second of polling
   // Most steps a traceback walk may take (TWEAKALIGN_WALK_GUARD lowers it so
@@ -1097,6 +1100,7 @@ void ta_batch_destroy(ta_batch *B) {
   dfree(B->d_ctr); dfree(B->d_fo_init); dfree(B->d_order); dfree(B->d_order_rest);
   free_rerun(B);
   dfree(B->d_lp); dfree(B->d_litems); dfree(B->d_lring); dfree(B->d_lcol); dfree(B->d_wpl);
+  dfree(B->d_lahead); dfree(B->d_lcross);
   dfree(B->d_spairs); dfree(B->d_sitems); dfree(B->d_sring); dfree(B->d_splanes); dfree(B->d_sbest);
   dfree(B->d_sscore);
   dfree(B->d_plain_tasks); dfree(B->d_prow); dfree(B->d_pcol); dfree(B->d_pring);
@@ -1695,13 +1699,23 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
       ring += nr; col += nc;
       B->lring_n = std::max(B->lring_n, ring);
       B->lcol_n = std::max(B->lcol_n, col);
-      B->litem_first.push_back((int32_t)B->litems.size());
+      L.item0 = (int32_t)B->litems.size();
       for (int s = 0; s < L.S; ++s) B->litems.push_back(LongItem{(int32_t)B->longs.size(), s});
       B->longs.push_back(L);
       LongGroup &g = B->lgroups.back();
       g.npairs += 1; g.nitems += L.S; g.ring_n = ring;
     }
-    if (!lk.empty() && p->traceback) B->long_wgs = std::max(1, std::min((int)lk.size(), 2 * ctx->cus));
+    if (!lk.empty() && p->traceback) {
+      B->long_wgs = std::max(1, std::min((int)lk.size(), 2 * ctx->cus));
+      // Regions ahead, where the pairs alone would not keep every CU at a
+      // region until the longest ends: 48 pairs (S up to 118, 3,300 in all)
+      // 16.7 -> 2.8 ms, 256 (S up to 196, 27,400) 41 -> 6.7; beyond, the same
+      // regions are computed either way.
+      int most = 0;
+      for (const LongPair &L : B->longs) most = std::max(most, L.S);
+      if ((int64_t)B->litems.size() < (int64_t)most * ctx->cus)
+        B->lahead = std::max(most, (int)std::min<size_t>(B->litems.size(), kLongAhead));
+    }
     if (const char *e = getenv("TWEAKALIGN_SPIN_LIMIT")) B->spin_limit = std::max(1, atoi(e));
     if (const char *e = getenv("TWEAKALIGN_WALK_GUARD")) B->guard_cap = std::max(0, atoi(e));
   }
@@ -1778,7 +1792,11 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
   rc = rc ? rc : dalloc(&B->d_splanes, B->splanes_n);
   rc = rc ? rc : dalloc(&B->d_sbest, B->spairs.size());
   rc = rc ? rc : dalloc(&B->d_sscore, B->spairs.size());
-  rc = rc ? rc : dalloc(&B->d_wpl, kLongPlanes * B->long_wgs);
+  rc = rc ? rc : dalloc(&B->d_wpl, LPLANES * B->long_wgs);
+  if (!rc && B->lahead) {
+    rc = dalloc(&B->d_lcross, B->litems.size());
+    if (!rc && dalloc(&B->d_lahead, LPLANES * B->lahead)) B->lahead = 0;  // (not needed for the result)
+  }
   for (auto &e : B->ev)
     if (!rc && hipEventCreate(&e) != hipSuccess) rc = TA_E_DEVICE;
   tr.mark("allocations");
@@ -1824,7 +1842,7 @@ int ta_batch_info(ta_batch *B, int64_t *cells, int64_t *tb_bytes, int32_t *tasks
   if (!B) return TA_E_INVALID;
   if (cells) *cells = B->cells;
   if (tb_bytes)
-    *tb_bytes = (int64_t)(B->plan.tb_bytes + 4 * kLongPlanes * B->long_wgs + 8 * B->lcol_n + 4 * B->splanes_n);
+    *tb_bytes = (int64_t)(B->plan.tb_bytes + 4 * LPLANES * (B->long_wgs + B->lahead) + 8 * B->lcol_n + 4 * B->splanes_n);
   if (tasks)
     *tasks = (int32_t)(B->plan.list2[0].tasks() + B->plan.list2[1].tasks() + B->plan.list2[2].tasks() +
                        B->plan.list1[0].tasks() + B->plan.list1[1].tasks() + B->litems.size() + B->sitems.size());
@@ -1957,14 +1975,27 @@ int launch_long_fwd(ta_ctx *ctx, ta_batch *B, int it0, int nit, uint64_t ring0, 
   return TA_OK;
 }
 
-// Traceback of long pairs [lp0, lp0 + nlp): one workgroup per pair.
-int launch_long_tb(ta_ctx *ctx, ta_batch *B, int lp0, int nlp) {
+// Traceback of long pairs [lp0, lp0 + nlp): one workgroup per pair, with
+// regions ahead as many pairs at a time as their memory holds.
+int launch_long_tb(ta_ctx *ctx, ta_batch *B, int lp0, int nlp, bool ahead) {
   if (nlp <= 0 || !B->p.traceback) return TA_OK;
-  const LongArgs a = long_args(B, 0, 0, lp0, nlp);
-  (void)hipGetLastError();
-  hipLaunchKernelGGL(long_tb_kernel<0>, dim3(std::max(1, std::min(nlp, B->long_wgs))), dim3(64 * LTW), LONG_TB_LDS,
-                     B->stream, a);
-  HIPCHK(hipGetLastError());
+  const int end = lp0 + nlp;
+  while (lp0 < end) {
+    int n = ahead ? 0 : nlp, items = 0;
+    while (lp0 + n < end && items + B->longs[lp0 + n].S <= B->lahead) items += B->longs[lp0 + n++].S;
+    LongArgs a = long_args(B, B->longs[lp0].item0, items, 0, 0);
+    (void)hipGetLastError();
+    if (ahead) {
+      a.ahead = B->d_lahead; a.cross = B->d_lcross; a.ahead0 = B->longs[lp0].item0;
+      hipLaunchKernelGGL(long_cross_kernel<0>, dim3(items), dim3(256), 0, B->stream, a);
+      hipLaunchKernelGGL(long_regions_kernel<0>, dim3(items), dim3(64 * LTW), LONG_TB_LDS, B->stream, a);
+    }
+    a.lp = B->d_lp + lp0; a.nlp = n;
+    hipLaunchKernelGGL(long_tb_kernel<0>, dim3(std::max(1, std::min(n, B->long_wgs))), dim3(64 * LTW), LONG_TB_LDS,
+                       B->stream, a);
+    HIPCHK(hipGetLastError());
+    lp0 += n;
+  }
   return TA_OK;
 }
 
@@ -2088,7 +2119,7 @@ int launch_fills(ta_ctx *ctx, ta_batch *B) {
   for (size_t g = 0; !rc && g < B->lgroups.size(); ++g) {
     const LongGroup &L = B->lgroups[g];
     rc = launch_long_fwd(ctx, B, L.it0, L.nitems, 0, L.ring_n);
-    if (!rc && g + 1 < B->lgroups.size()) rc = launch_long_tb(ctx, B, L.lp0, L.npairs);
+    if (!rc && g + 1 < B->lgroups.size()) rc = launch_long_tb(ctx, B, L.lp0, L.npairs, B->lahead > 0);
   }
   return rc;
 }
@@ -2107,7 +2138,7 @@ int launch_tracebacks(ta_ctx *ctx, ta_batch *B) {
                        B->stream, a);
     HIPCHK(hipGetLastError());
   }
-  if (!rc && !B->lgroups.empty()) rc = launch_long_tb(ctx, B, B->lgroups.back().lp0, B->lgroups.back().npairs);
+  if (!rc && !B->lgroups.empty()) rc = launch_long_tb(ctx, B, B->lgroups.back().lp0, B->lgroups.back().npairs, B->lahead > 0);
   return rc;
 }
 
@@ -2594,9 +2625,9 @@ int ta_batch_run_plain(ta_ctx *ctx, ta_batch *B, int32_t first, int32_t count) {
     if (h.path == 3) {
       const int q = lp_of[k];
       const LongPair &L = B->longs[q];
-      int rc = launch_long_fwd(ctx, B, B->litem_first[q], L.S, L.ring, (uint64_t)(L.S - 1) * (L.T + 8));
+      int rc = launch_long_fwd(ctx, B, L.item0, L.S, L.ring, (uint64_t)(L.S - 1) * (L.T + 8));
       if (!rc) rc = launch_traceback(ctx, B, B->d_pairs, B->d_pptb, B->d_ptbuf, k, 1);
-      if (!rc) rc = launch_long_tb(ctx, B, q, 1);
+      if (!rc) rc = launch_long_tb(ctx, B, q, 1, false);
       if (rc) return rc;
       continue;
     }
