@@ -397,9 +397,9 @@ __global__ __launch_bounds__(64 * LTW) void long_tb_kernel(LongArgs A) {
       const int T = (right - c_left + 63 + 7) & ~7;
       if (wv == 0) {
         StripWindow<2> src{pl, (uint32_t *)(lds + LT_WIN), T, -1, -1};
-        int li = i - top, lj = j - c_left, h = 0, steps = 0;
+        int li = i - top, lj = j - c_left, steps = 0;
         src.refill(li, lj);
-        if (wave_walk<WALK_GLOBAL>(src, rw, li, lj, state, h, A.open, A.ext, INT32_MAX, steps) == WALK_GAVE_UP) {
+        if (wave_walk<WALK_GLOBAL>(src, rw, li, lj, state, INT32_MAX, steps) == WALK_GAVE_UP) {
           failed = true;  // cannot happen: end the walk rather than loop
           li = lj = 0;
         }

@@ -337,9 +337,9 @@ __global__ __launch_bounds__(64 * JWMAX) void msa_join_kernel(JoinArgs A) {
     rw.end = rend;
     rw.cap = cap;
     StripWindow<JR> src{tb, win, T, -1, -1};
-    int i = la, j = lb, state = 0, h = 0, steps = 0;
+    int i = la, j = lb, state = 0, steps = 0;
     src.refill(i, j);
-    const int how = wave_walk<WALK_GLOBAL>(src, rw, i, j, state, h, go, ge, la + lb, steps);
+    const int how = wave_walk<WALK_GLOBAL>(src, rw, i, j, state, la + lb, steps);
     if (how != WALK_GAVE_UP) {
       if (i == 0 && j > 0) rw.emit(1, j);
       if (j == 0 && i > 0) rw.emit(2, i);

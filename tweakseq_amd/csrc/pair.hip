@@ -113,6 +113,7 @@ struct PairCodes {
     const uint32_t dw = pl[__umul24(s, strip_dw) + __umul24(t / SPD, s == last ? last_lanes : 64u) + l];
     return strip_code<PR>(dw, t % SPD, r % PR);
   }
+  __device__ __forceinline__ int direct(int i, int j) const { return code(i, j); }
   __device__ __forceinline__ bool refill(int, int) { return false; }
 };
 
@@ -257,15 +258,15 @@ __global__ __launch_bounds__(64 * PAIR_WAVES) __attribute__((amdgpu_waves_per_eu
   rw.cap = cap;
   if (walk) {
     constexpr int KIND = LOCAL ? WALK_MARKED : WALK_GLOBAL;
-    int state = 0, h = 0, steps = 0, how;
+    int state = 0, steps = 0, how;
     if constexpr (GP) {
       StripWindow<PR> src{(const uint32_t *)A.planes, (uint32_t *)(lds + Y.window), T, -1, -1};
       src.refill(i, j);
-      how = wave_walk<KIND>(src, rw, i, j, state, h, A.open, A.ext, A.walk_cap, steps);
+      how = wave_walk<KIND>(src, rw, i, j, state, A.walk_cap, steps);
     } else {
       PairCodes<PR> src{(const uint32_t *)(lds + Y.planes), (uint32_t)(T / SPD) * 64, (uint32_t)S - 1,
                         (uint32_t)last_lanes};
-      how = wave_walk<KIND>(src, rw, i, j, state, h, A.open, A.ext, A.walk_cap, steps);
+      how = wave_walk<KIND>(src, rw, i, j, state, A.walk_cap, steps);
     }
     if (how == WALK_GAVE_UP) {
       r.flags |= TA_F_WALK_FAILED;
@@ -325,7 +326,7 @@ PairLayout pair_layout(int m, int n, int K, int lds_max) {
   // after the fill: the CIGAR runs and, with the codes in device memory, the walk's window
   L.runs = L.slots;
   L.window = (int)(L.slots + up(4L * L.runs_cap, 16));
-  const long spd = strip_spd(L.R), after = L.window + 32 * (32 / spd + 1) * 4, strips = (long)L.T / spd * 4;
+  const long spd = strip_spd(L.R), after = L.window + 64 * (32 / spd + 1) * 4, strips = (long)L.T / spd * 4;
   const long last = (m - (long)(L.S - 1) * 64 * L.R + L.R - 1) / L.R;
   L.planes = (int)std::max(off, (long)L.window);
   const long with = L.planes + strips * ((L.S - 1) * 64L + last);

@@ -521,42 +521,64 @@ struct StripGroupIO : StripIODefaults {
 };
 
 // Codes in device memory ([strip][t / SPD][64 lanes]): a window of them in
-// LDS, 32 lanes' rows up from the walk's cell, for each lane WD dwords
-// around the diagonal through it.
+// LDS, 64 strip lanes' rows up from the walk's cell, for each lane WD dwords
+// around the diagonal through it.  A thread brings one strip lane's dwords:
+// one address and WD loads.  The window above is on its way while one is
+// walked, placed on the same diagonal; a walk that leaves it fetches its own.
+// (Windows of 32 lanes fetched when needed, and the shorter lookups of long
+// gaps and gaps of one, before / now: 48 DNA pairs 1,662 / 1,068 us, requests
+// of 8 pairs of up to 2,500 202 / 137, 16 unrelated pairs of up to 5,000
+// 239 / 219, a pair of 1,500 53 / 43.)
 template <int PR>
 struct StripWindow {
-  static constexpr int SPD = strip_spd(PR), WL = 32, WD = 32 / SPD + 1;
+  static constexpr int SPD = strip_spd(PR), WL = 64, WD = 32 / SPD + 1;
   const uint32_t *pl;
   uint32_t *win;  // WL x WD
   int T;
   int L0, u0;     // the window's first (lowest) lane, counted over all strips, and its 0-based column
-  // first staged dword of lane L0 - q
-  __device__ __forceinline__ int first(int q) const {
-    const int t = u0 - q * PR + ((L0 - q) & 63), d = t / SPD - WD / 2, top = T / SPD - WD;
-    return d > top ? (top < 0 ? 0 : top) : (d < 0 ? 0 : d);
+  uint32_t nx[WD] = {};    // the next window: this thread's lane
+  int nL0 = -1, nu0 = 0;   // (nL0 < 0: none)
+  // (arithmetic shifts: positions left of the columns are negative)
+  static __device__ __forceinline__ int dword(int t) { return t >> (SPD == 8 ? 3 : SPD == 4 ? 2 : 1); }
+  // where a window on (l0, c0) holds the dword of lane L's column u; -1: not
+  __device__ __forceinline__ int at(int l0, int c0, int L, int u) const {
+    const int q = l0 - L, s = L & 63, d = dword(u + s) - dword(c0 - q * PR + s) + WD / 2;
+    return (uint32_t)q < (uint32_t)WL && (uint32_t)d < (uint32_t)WD ? q * WD + d : -1;
   }
   __device__ __forceinline__ int code(int i, int j) const {
-    const int L = (int)((uint32_t)(i - 1) / PR), q = L0 - L, t = j - 1 + (L & 63);
-    const int d = (int)((uint32_t)t / SPD) - first(q);
-    if (q < 0 || q >= WL || d < 0 || d >= WD) return -1;
-    return strip_code<PR>(win[q * WD + d], (uint32_t)t % SPD, (uint32_t)(i - 1) % PR);
+    const int L = (int)((uint32_t)(i - 1) / PR), x = at(L0, u0, L, j - 1);
+    const int c = strip_code<PR>(win[x < 0 ? 0 : x], (uint32_t)(j - 1 + (L & 63)) % SPD, (uint32_t)(i - 1) % PR);
+    return x < 0 ? -1 : c;
+  }
+  __device__ __forceinline__ int direct(int i, int j) const {
+    const int L = (int)((uint32_t)(i - 1) / PR), t = j - 1 + (L & 63);
+    return strip_code<PR>(pl[((size_t)(L >> 6) * (T / SPD) + dword(t)) * 64 + (L & 63)], (uint32_t)t % SPD,
+                          (uint32_t)(i - 1) % PR);
+  }
+  __device__ __forceinline__ void fetch(int l0, int c0) {
+    const int q = min((int)(threadIdx.x & 63), l0), L = l0 - q, s = L & 63;
+    const uint32_t *p = pl + (size_t)(L >> 6) * (T / SPD) * 64 + s;
+    const int d = dword(c0 - q * PR + s) - WD / 2;
+#pragma unroll
+    for (int k = 0; k < WD; ++k) nx[k] = p[min(max(d + k, 0), T / SPD - 1) * 64];
   }
   __device__ __forceinline__ bool refill(int i, int j) {
-    const bool moved = (i - 1) / PR != L0 || j - 1 != u0;
-    L0 = (i - 1) / PR;
-    u0 = j - 1;
-    constexpr int N = WL * WD, U = (N + 63) / 64;
-    uint32_t v[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int x = u * 64 + (int)(threadIdx.x & 63), q = x / WD, d = first(q) + x % WD, L = L0 - q;
-      v[u] = x < N && L >= 0 && d < T / SPD ? pl[((size_t)(L >> 6) * (T / SPD) + d) * 64 + (L & 63)] : 0;
+    const int L = (i - 1) / PR, u = j - 1;
+    bool moved = true;
+    if (nL0 < 0 || at(nL0, nu0, L, u) < 0) {
+      moved = L != L0 || u != u0;
+      nL0 = L;
+      nu0 = u;
+      fetch(L, u);
     }
+    L0 = nL0;
+    u0 = nu0;
+    uint32_t *w = win + (threadIdx.x & 63) * WD;
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int x = u * 64 + (int)(threadIdx.x & 63);
-      if (x < N) win[x] = v[u];
-    }
+    for (int k = 0; k < WD; ++k) w[k] = nx[k];
+    nL0 = L0 - WL;
+    nu0 = u - (L - nL0) * PR;
+    if (nL0 >= 0) fetch(nL0, nu0);
     return moved;
   }
 };

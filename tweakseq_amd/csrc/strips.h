@@ -283,10 +283,10 @@ __global__ __launch_bounds__(64) void strips_walk_kernel(StripsArgs A) {
     rw.cap = pd.cig_cap / 4;
     Win src{A.planes + P.planes, win, P.T, -1, -1};
     src.refill(i, j);
-    int state = 0, h = 0, steps = 0;
+    int state = 0, steps = 0;
     // a walk may take fewer than `cap` steps, or end on that step (local)
     const int full = 2 * (pd.la + pd.lb) + 2, cap = (full < A.tb.guard_cap ? full : A.tb.guard_cap) - (LOCAL ? 0 : 1);
-    const int how = wave_walk<LOCAL ? WALK_MARKED : WALK_GLOBAL>(src, rw, i, j, state, h, A.open, A.ext, cap, steps);
+    const int how = wave_walk<LOCAL ? WALK_MARKED : WALK_GLOBAL>(src, rw, i, j, state, cap, steps);
     if (how == WALK_GAVE_UP) r.flags |= WALK_FAILED;
     if (!LOCAL && how != WALK_GAVE_UP) {
       if (i == 0 && j > 0) rw.emit(1, j);

@@ -19,8 +19,7 @@ namespace ta {
 
 // How a walk ends other than at the matrix border.
 enum { WALK_GLOBAL = 0,   // only there
-       WALK_MARKED = 1,   // on a cell whose code is d = 0, x = 1: its H is 0
-       WALK_CARRIED = 2 };  // on a diagonal move into a cell whose H is 0, known by carrying H back
+       WALK_MARKED = 1 }; // on a cell whose code is d = 0, x = 1: its H is 0
 
 enum { WALK_AT_BORDER = 0, WALK_STOPPED = 1, WALK_GAVE_UP = 2 };
 
@@ -59,38 +58,26 @@ struct WaveRuns {
 // Walks from (i, j) (1-based) in `state` (0 H, 1 E, 2 F) until it ends;
 // every value is the same in all lanes.  Src gives
 //   int code(i, j)        a lane's cell: e f d x in bits 0..3, -1 if not at hand
+//   int direct(i, j)      the same from where the codes are, at hand or not
 //   bool refill(i, j)     (whole wave) brings cell (i, j) and its surroundings
 //                         to hand; false if it cannot
-//   int score(i, j)       WALK_CARRIED: the cell's substitution score
-// `h` is carried for WALK_CARRIED; `steps` counts cells passed, and the walk
-// gives up when they exceed `cap`.
+// `steps` counts cells passed, and the walk gives up when they exceed `cap`.
 template <int KIND, class Src>
-__device__ __forceinline__ int wave_walk(Src &src, WaveRuns &w, int &i, int &j, int &state, int &h, int open, int ext,
-                                         int cap, int &steps) {
+__device__ __forceinline__ int wave_walk(Src &src, WaveRuns &w, int &i, int &j, int &state, int cap,
+                                         int &steps) {
   const int lane = threadIdx.x & 63;
   if (i <= 0 || j <= 0) return WALK_AT_BORDER;
+  auto look = [&](int ci, int cj, bool far) {  // a lane's cell; -1 beyond the border (no branch: an inner cell stands in)
+    const int c = far ? src.direct(max(ci, 1), max(cj, 1)) : src.code(max(ci, 1), max(cj, 1));
+    return min(ci, cj) >= 1 ? c : -1;
+  };
+  bool far = false;  // a gap goes on beyond what is at hand
   for (;;) {
     if (state == 0) {
       const int ci = i - lane, cj = j - lane;
-      const int c = ci >= 1 && cj >= 1 ? src.code(ci, cj) : -1;
+      const int c = look(ci, cj, false);
       const uint64_t stop = __ballot((c & (KIND == WALK_MARKED ? 12 : 4)) != 0);
       const int run = stop ? __builtin_ctzll(stop) : 64;
-      if constexpr (KIND == WALK_CARRIED) {
-        int sum = lane < run ? src.score(ci, cj) : 0;  // scores of the moves up to this lane's
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-          const int o = __shfl_up(sum, d, 64);
-          sum += lane >= d ? o : 0;
-        }
-        const uint64_t over = __ballot(lane < run && (h == sum || ci == 1 || cj == 1));
-        if (over) {
-          const int k = __builtin_ctzll(over) + 1;
-          w.emit(0, k);
-          i -= k; j -= k; steps += k;
-          return steps > cap ? WALK_GAVE_UP : WALK_STOPPED;
-        }
-        if (run) h -= __builtin_amdgcn_readlane(sum, run - 1);
-      }
       if (run) {
         w.emit(0, run);
         i -= run; j -= run; steps += run;
@@ -105,15 +92,22 @@ __device__ __forceinline__ int wave_walk(Src &src, WaveRuns &w, int &i, int &j, 
       }
       if (KIND == WALK_MARKED && (at & 12) == 8) return WALK_STOPPED;
       state = (at & 8) ? 2 : 1;
+      if (!(at & state)) {  // a gap of one: the same cell opened it
+        w.emit(state, 1);
+        i -= state == 2;
+        j -= state == 1;
+        state = 0;
+        if (++steps > cap) return WALK_GAVE_UP;
+        continue;
+      }
     }
     // the gap: cells that extend it, then the one that opened it
     const int ci = i - (state == 2 ? lane : 0), cj = j - (state == 1 ? lane : 0);
-    const int c = ci >= 1 && cj >= 1 ? src.code(ci, cj) : -1;
+    const int c = look(ci, cj, far);
     const uint64_t stop = __ballot(c < 0 || (c & state) == 0);
     const int run = stop ? __builtin_ctzll(stop) : 64;
     const int at = run < 64 ? __builtin_amdgcn_readlane(c, run & 63) : -1;
     const int len = at >= 0 ? run + 1 : run;
-    if constexpr (KIND == WALK_CARRIED) h -= run * ext + (at >= 0 ? open : 0);
     if (len) w.emit(state, len);
     i -= state == 2 ? len : 0;
     j -= state == 1 ? len : 0;
@@ -121,9 +115,11 @@ __device__ __forceinline__ int wave_walk(Src &src, WaveRuns &w, int &i, int &j, 
     if (steps > cap) return WALK_GAVE_UP;
     if (at >= 0) {
       state = 0;
+      far = false;
     } else if (run < 64) {
       if (i <= 0 || j <= 0) return WALK_AT_BORDER;
-      if (!src.refill(i, j)) return WALK_GAVE_UP;
+      if (far) return WALK_GAVE_UP;  // cannot happen
+      far = true;
     }
   }
 }
