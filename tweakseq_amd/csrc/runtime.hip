@@ -345,10 +345,11 @@ void vec_give(std::vector<T> &x) {
   }
 }
 
-// Host vectors bound for their own device buffers, gathered into one pinned
-// staging block and sent with one asynchronous copy each (a copy from
-// pageable memory is staged by the runtime and waits for the link).  The
-// vectors must live until commit(); the block until the stream drains.
+// Host vectors bound for the device, gathered into one pinned staging block
+// and sent with one asynchronous copy into one device block (a copy from
+// pageable memory is staged by the runtime and waits for the link; a copy
+// per vector took a small batch's creation 3.4 us each).  The vectors must
+// live until commit(); the staging block until the stream drains.
 struct BulkUpload {
   struct Item { void **dst; const void *src; size_t bytes, at; };
   std::vector<Item> items;
@@ -356,9 +357,10 @@ struct BulkUpload {
   template <typename T>
   void add(T **dst, const std::vector<T> &v) {
     *dst = nullptr;
-    items.push_back(Item{(void **)dst, v.data(), v.size() * sizeof(T), 0});
+    if (!v.empty()) items.push_back(Item{(void **)dst, v.data(), v.size() * sizeof(T), 0});
   }
-  int commit(hipStream_t st) {
+  int commit(void **block, hipStream_t st) {
+    *block = nullptr;
     size_t total = 0;
     for (Item &x : items) {
       x.at = total;
@@ -367,17 +369,14 @@ struct BulkUpload {
     if (!total) return TA_OK;
     hold.s = stage_take(total);
     if (!hold.s.p) return TA_E_NOMEM;
-    for (Item &x : items)
-      if (x.bytes) memcpy(hold.s.p + x.at, x.src, x.bytes);
-    hold.stream = st;
+    if (!(*block = cache_alloc(total))) return TA_E_NOMEM;
     for (Item &x : items) {
-      if (!x.bytes) continue;
-      if (!(*x.dst = cache_alloc(x.bytes))) return TA_E_NOMEM;
-      hold.queued = true;
-      if (hipMemcpyAsync(*x.dst, hold.s.p + x.at, x.bytes, hipMemcpyHostToDevice, st) != hipSuccess)
-        return TA_E_DEVICE;
+      memcpy(hold.s.p + x.at, x.src, x.bytes);
+      *x.dst = (uint8_t *)*block + x.at;
     }
-    return TA_OK;
+    hold.stream = st;
+    hold.queued = true;
+    return hipMemcpyAsync(*block, hold.s.p, total, hipMemcpyHostToDevice, st) == hipSuccess ? TA_OK : TA_E_DEVICE;
   }
 };
 
@@ -593,9 +592,12 @@ int fill_waves_per_cu(int P, int Kp, bool nib, int want, bool walk = false) {
 
 // Raw letters to residue codes in place, 16 bytes per thread step, through a
 // 256-entry map (0xff: outside the alphabet, which sets *bad).
-__global__ void encode_kernel(uint4 *codes, size_t words, const uint8_t *map, int32_t *bad) {
+struct LetterMap {
+  uint32_t w[64];
+};
+__global__ __launch_bounds__(256) void encode_kernel(uint4 *codes, size_t words, LetterMap map, int32_t *bad) {
   __shared__ uint8_t m[256];
-  for (int i = threadIdx.x; i < 256; i += blockDim.x) m[i] = map[i];
+  if (threadIdx.x < 64) ((uint32_t *)m)[threadIdx.x] = map.w[threadIdx.x];
   __syncthreads();
   uint32_t any = 0;
   for (size_t w = (size_t)blockIdx.x * blockDim.x + threadIdx.x; w < words; w += (size_t)gridDim.x * blockDim.x) {
@@ -983,6 +985,7 @@ struct ta_batch {
   // device
   uint8_t *d_codes = nullptr;
   std::shared_ptr<uint8_t> codes_owner;  // set when d_codes is a resident-sequence arena (held, not freed)
+  void *d_bulk = nullptr;         // the block of the tables that go up in one copy (BulkUpload)
   int8_t *d_table = nullptr;
   int8_t *d_table_nib = nullptr;  // packed couples: 4-bit biased scores
   bool nib = false;
@@ -1093,15 +1096,15 @@ void ta_batch_destroy(ta_batch *B) {
   // holds even where the run's stream is gone.
   if (B->ev[3]) (void)hipEventSynchronize(B->ev[3]);
   if (B->codes_owner) B->d_codes = nullptr;
-  dfree(B->d_codes); dfree(B->d_table); dfree(B->d_table_nib);
+  dfree(B->d_codes); dfree(B->d_bulk);
   for (int g = 0; g < 3; ++g) { dfree(B->d_tasks2[g]); dfree(B->d_tasks1[g]); }
   dfree(B->d_rowcodes); dfree(B->d_colcodes); dfree(B->d_ring); dfree(B->d_tb);
   dfree(B->d_ptb); dfree(B->d_pairs); dfree(B->d_fo); dfree(B->d_res); dfree(B->d_cig);
-  dfree(B->d_ctr); dfree(B->d_fo_init); dfree(B->d_order); dfree(B->d_order_rest);
+  dfree(B->d_ctr); dfree(B->d_fo_init);
   free_rerun(B);
-  dfree(B->d_lp); dfree(B->d_litems); dfree(B->d_lring); dfree(B->d_lcol); dfree(B->d_wpl);
+  dfree(B->d_lring); dfree(B->d_lcol); dfree(B->d_wpl);
   dfree(B->d_lahead); dfree(B->d_lcross);
-  dfree(B->d_spairs); dfree(B->d_sitems); dfree(B->d_sring); dfree(B->d_splanes); dfree(B->d_sbest);
+  dfree(B->d_sring); dfree(B->d_splanes); dfree(B->d_sbest);
   dfree(B->d_sscore);
   dfree(B->d_plain_tasks); dfree(B->d_prow); dfree(B->d_pcol); dfree(B->d_pring);
   dfree(B->d_ptbuf); dfree(B->d_pptb); dfree(B->d_plain_rtasks); dfree(B->d_pptb_r);
@@ -1447,13 +1450,14 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
   // runs on the DMA engine alone; the encoding kernel follows on the stream.
   hipStream_t st = B->stream;
   int rc = TA_OK;
-  uint8_t *d_map = nullptr;
-  int32_t *d_bad = nullptr;
-  int32_t bad_letter = 0;
+  // the counters, and behind them whether a letter was outside the alphabet
+  rc = dalloc(&B->d_ctr, 32);
+  if (!rc && hipMemsetAsync(B->d_ctr, 0, 32 * sizeof(int32_t), st) != hipSuccess) rc = TA_E_DEVICE;
+  int32_t *d_bad = B->d_ctr + 16;
   if (res) {  // resident sequences: the codes are on the device already
     B->codes_owner = res->arena;
     B->d_codes = res->arena.get();
-  } else {
+  } else if (!rc) {
     rc = dalloc(&B->d_codes, cend);
   }
   if (!rc && !res) {
@@ -1461,29 +1465,27 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
     codes.queued = true;
     if (hipMemcpyAsync(B->d_codes, codes.s.p, cend, hipMemcpyHostToDevice, st) != hipSuccess) rc = TA_E_DEVICE;
   }
-  rc = rc || res ? rc : upload(&d_map, std::vector<uint8_t>(map, map + 256), st);
-  rc = rc || res ? rc : dalloc(&d_bad, 1);
-  if (!rc && !res && hipMemsetAsync(d_bad, 0, sizeof(int32_t), st) != hipSuccess) rc = TA_E_DEVICE;
   if (!rc && !res) {
     (void)hipGetLastError();
+    LetterMap lm;
+    memcpy(lm.w, map, 256);
     const size_t words = cend / 16;
     hipLaunchKernelGGL(encode_kernel, dim3((unsigned)std::min<size_t>((words + 255) / 256, 4096)), dim3(256), 0, st,
-                       (uint4 *)B->d_codes, words, d_map, d_bad);
+                       (uint4 *)B->d_codes, words, lm, d_bad);
     if (hipGetLastError() != hipSuccess) rc = TA_E_DEVICE;
   }
   if (rc) {
     (void)hipStreamSynchronize(st);
-    dfree(d_map);
-    dfree(d_bad);
     ta_batch_destroy(B);
     return rc;
   }
   tr.mark("upload-encode");
   // The pairs' table goes up while the host plans, too.
   StageHold ptab;
-  ptab.s = stage_take(sizeof(PairDev) * (size_t)std::max(n, 1));
+  ptab.s = stage_take(sizeof(PairDev) * (size_t)n + 64);  // (and where the letter check comes back)
   if (!ptab.s.p) rc = TA_E_NOMEM;
   PairDev *pairs_h = (PairDev *)ptab.s.p;
+  int32_t *bad_letter = (int32_t *)(pairs_h + n);
   vec_take(B->hp);
   B->hp.resize(n);
   if (!rc) parallel_tasks(NS, [&](int t) {
@@ -1545,8 +1547,6 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
   }
   if (rc) {
     (void)hipStreamSynchronize(st);
-    dfree(d_map);
-    dfree(d_bad);
     ta_batch_destroy(B);
     return rc;
   }
@@ -1731,7 +1731,7 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
   }
   PlanArgs pa{};
   int32_t total = 0;
-  Unit *d_units[6] = {nullptr};       // freed after the final drain
+  Unit *d_units[6] = {nullptr};
   TaskSpan *d_spans[6] = {nullptr};
   for (int l = 0; l < 6; ++l) {
     TaskList &L = l < 3 ? pl.list2[l] : pl.list1[l - 3];
@@ -1762,7 +1762,7 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
   up.add(&B->d_litems, B->litems);
   up.add(&B->d_spairs, B->spairs);
   up.add(&B->d_sitems, B->sitems);
-  rc = rc ? rc : up.commit(st);
+  rc = rc ? rc : up.commit(&B->d_bulk, st);
   rc = rc ? rc : dalloc(&B->d_rowcodes, (size_t)pl.rows_n);
   rc = rc ? rc : dalloc(&B->d_colcodes, (size_t)pl.cols_n);
   for (int l = 0; l < 6; ++l) {
@@ -1784,8 +1784,6 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
   rc = rc ? rc : dalloc(&B->d_fo, (size_t)std::max(n, 1));
   rc = rc ? rc : dalloc(&B->d_res, (size_t)std::max(n, 1));
   rc = rc ? rc : dalloc(&B->d_cig, B->cig_bytes);
-  rc = rc ? rc : dalloc(&B->d_ctr, 16);
-  if (!rc && hipMemsetAsync(B->d_ctr, 0, 16 * sizeof(int32_t), st) != hipSuccess) rc = TA_E_DEVICE;
   rc = rc ? rc : dalloc(&B->d_lring, B->lring_n);
   rc = rc ? rc : dalloc(&B->d_lcol, B->lcol_n);
   rc = rc ? rc : dalloc(&B->d_sring, B->sring_n);
@@ -1801,20 +1799,15 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
     if (!rc && hipEventCreate(&e) != hipSuccess) rc = TA_E_DEVICE;
   tr.mark("allocations");
   // Drained on every path: the blocks of a failed creation go back to the
-  // cache only after the copies queued into them.
-  if (hipStreamSynchronize(st) != hipSuccess && !rc) rc = TA_E_DEVICE;
-  // the letter check, read once the stream has drained (a copy into
-  // pageable memory queued earlier would have waited for the upload)
-  if (!rc && d_bad && hipMemcpy(&bad_letter, d_bad, sizeof(int32_t), hipMemcpyDeviceToHost) != hipSuccess)
+  // cache only after the copies queued into them.  The letter check comes
+  // back on the way.
+  if (!rc && hipMemcpyAsync(bad_letter, d_bad, sizeof(int32_t), hipMemcpyDeviceToHost, st) != hipSuccess)
     rc = TA_E_DEVICE;
-  dfree(d_map);
-  dfree(d_bad);
-  for (int l = 0; l < 6; ++l) {
-    dfree(d_units[l]);
-    dfree(d_spans[l]);
-  }
+  ptab.stream = st;
+  ptab.queued = true;
+  if (hipStreamSynchronize(st) != hipSuccess && !rc) rc = TA_E_DEVICE;
   tr.mark("drain");
-  if (!rc && bad_letter) rc = TA_E_ALPHABET;
+  if (!rc && *bad_letter) rc = TA_E_ALPHABET;
   if (rc) {
     ta_batch_destroy(B);
     return rc;
@@ -2268,9 +2261,9 @@ __global__ void gather_runs_kernel(const uint32_t *cig, const ResultDev *res, co
 }
 
 // Results and CIGAR runs of a finished batch on the host, in pinned staging
-// blocks: `res` per pair, `runs` dense, pair k's runs at runs[off[k] / 4 ...]
-// (cigar_len bytes).  Only the runs cross PCIe, not the per-pair worst-case
-// regions.
+// blocks: `res` per pair, pair k's runs at runs[off[k] / 4 ...] (cigar_len
+// bytes).  Of large batches only the runs cross PCIe (gathered, dense), not
+// the per-pair worst-case regions.
 struct Fetched {
   StageHold resb, runsb;
   const ResultDev *res = nullptr;
@@ -2289,10 +2282,26 @@ int fetch_results(ta_batch *B, Fetched &F) {
     HIPCHK(hipMemcpyAsync(F.resb.s.p, B->d_res, sizeof(ResultDev) * B->n, hipMemcpyDeviceToHost, st));
     F.res = (const ResultDev *)F.resb.s.p;
   }
+  // Where the pairs' regions take 1 MB at most they come back whole, in one
+  // go with the results: 20 us of link at most, against an upload, a kernel,
+  // a copy and a second wait (35 us) for the runs alone.
+  const bool small = B->p.traceback && B->n && B->cig_bytes && B->cig_bytes <= (1 << 20);
+  if (small) {
+    F.runsb.s = stage_take(B->cig_bytes);
+    if (!F.runsb.s.p) return TA_E_NOMEM;
+    F.runsb.stream = st;
+    F.runsb.queued = true;
+    HIPCHK(hipMemcpyAsync(F.runsb.s.p, B->d_cig, B->cig_bytes, hipMemcpyDeviceToHost, st));
+  }
   HIPCHK(hipStreamSynchronize(st));
   if (!B->p.traceback) return TA_OK;
   const ResultDev *res = F.res;
   off.assign(B->n, 0);
+  if (small) {
+    for (int32_t k = 0; k < B->n; ++k) off[k] = res[k].cigar_off;
+    F.runs = (const uint32_t *)F.runsb.s.p;
+    return TA_OK;
+  }
   int64_t total = 0;
   for (int32_t k = 0; k < B->n; ++k) {
     off[k] = total;
