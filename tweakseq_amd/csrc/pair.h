@@ -29,7 +29,8 @@ struct PairOut {
   ResultDev r;
   int32_t nruns;
   int32_t status;           // PAIR_BAD_LETTER, PAIR_GAVE_UP
-  int32_t pad_[2];
+  int32_t done;             // set last, where the caller polls it
+  int32_t pad_;
 };
 
 struct PairArgs {
@@ -38,6 +39,7 @@ struct PairArgs {
   int32_t alphabet, match, mismatch;
   int32_t open, ext, local, traceback;
   int32_t spin_limit;
+  int32_t polled;           // set PairOut::done when everything else is stored
   int32_t walk_cap;         // most steps the walk may take before it ends flagged (above any walk normally)
   PairLayout lay;
   uint8_t *planes;          // lay.plane_bytes of device memory, where the codes do not fit in LDS

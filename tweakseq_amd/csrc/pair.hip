@@ -23,9 +23,9 @@
 // Bound by dependent steps: n + 80 (strips) of the fill, each as long as one
 // wave takes to issue it, and a lookup per CIGAR run of the walk.  Call to
 // CIGAR, with two rows per lane, 322 cycles a step and a walk of 430 cycles a
-// cell, and now: 24 x 28 global protein 36 / 24 us, 300 x 320 155 / 76 us (of
+// cell, and now: 24 x 28 global protein 36 / 19 us, 300 x 320 155 / 71 us (of
 // 2.4 GHz cycles: fill 117,000, walk 28,000, tables and letters 7,500),
-// 400 x 420 local DNA 217 / 105 us.
+// 400 x 420 local DNA 217 / 100 us.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -169,7 +169,10 @@ __global__ __launch_bounds__(64 * PAIR_WAVES) __attribute__((amdgpu_waves_per_eu
   if (bad) atomicOr(&sy[SY_STATUS], PAIR_BAD_LETTER);
   __syncthreads();
   if (sy[SY_STATUS] & PAIR_BAD_LETTER) {
-    if (tid == 0) A.out->status = sy[SY_STATUS];
+    if (tid == 0) {
+      A.out->status = sy[SY_STATUS];
+      if (A.polled) __hip_atomic_store(&A.out->done, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
     return;
   }
 
@@ -289,6 +292,8 @@ __global__ __launch_bounds__(64 * PAIR_WAVES) __attribute__((amdgpu_waves_per_eu
     A.out->nruns = A.traceback ? nr : 0;
     A.out->status = sy[SY_STATUS];
   }
+  // (the wave's own stores: one release covers the runs of all its lanes)
+  if (A.polled && lane == 0) __hip_atomic_store(&A.out->done, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 template <int PR>
@@ -443,7 +448,7 @@ int ta_align_pair(ta_ctx *ctx, const ta_params *p, const char *a, int32_t la, co
     ctx->pair_stage = nullptr;
     ctx->pair_stage_cap = 0;
     const size_t want = std::max(need, (size_t)64 << 10);
-    if (hipHostMalloc(&ctx->pair_stage, want, hipHostMallocDefault) != hipSuccess) {
+    if (hipHostMalloc(&ctx->pair_stage, want, hipHostMallocCoherent) != hipSuccess) {
       (void)hipGetLastError();
       ctx->pair_stage = nullptr;
       return TA_E_NOMEM;
@@ -455,12 +460,22 @@ int ta_align_pair(ta_ctx *ctx, const ta_params *p, const char *a, int32_t la, co
   memcpy(st + o_b, b, (size_t)lb);
   PairOut *o = (PairOut *)st;
   o->status = 0;
+  o->done = 0;
+  A.polled = 1;
   A.a = (const char *)(st + o_a);
   A.b = (const char *)(st + o_b);
   A.out = o;
   int rc = pair_launch(A, ctx->stream);
   if (rc) return rc;
-  if (hipStreamSynchronize(ctx->stream) != hipSuccess) return TA_E_DEVICE;
+  // The kernel's last store says that the result is there, a few microseconds
+  // before the stream is seen idle; a wait longer than any pair takes is the
+  // stream's (which reports errors).
+  const auto t0 = std::chrono::steady_clock::now();
+  while (!__atomic_load_n(&o->done, __ATOMIC_ACQUIRE)) {
+    if (std::chrono::steady_clock::now() - t0 < std::chrono::microseconds(500)) continue;
+    if (hipStreamSynchronize(ctx->stream) != hipSuccess) return TA_E_DEVICE;
+    break;
+  }
   return pair_finish(*o, (const uint32_t *)(st + o_runs), p, out, cigar_buf, cap, used);
 }
 
