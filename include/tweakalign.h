@@ -111,10 +111,11 @@ int ta_align_batch(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32_
 /* One pair at low latency: the editor's "realign selection" of two rows
  * (tweakseq/UI/SeqEditMainWin.cpp:1616-1663 runs an external aligner on the
  * selection; tweakseq/Core/Project.cpp:964-1026 splices its output back).
- * One kernel launch with the letters read from mapped host staging, the
- * direction codes kept on chip, and the result written back to staging; no
- * device allocation.  Same result and conventions as ta_align_batch with
- * n = 1 (which pairs too large for the on-chip form, or with an empty side,
+ * One kernel launch with the letters read from mapped host staging, and the
+ * result written back to staging; the direction codes are kept on chip, or in
+ * a block of device memory that the context keeps where they do not fit beside
+ * the kernel's tables.  Same result and conventions as ta_align_batch with
+ * n = 1 (which pairs with more codes than a CU's LDS, or with an empty side,
  * go through).  Results carry TA_F_I32 (the pair kernel computes in int32). */
 int ta_align_pair(ta_ctx *ctx, const ta_params *p, const char *a, int32_t la, const char *b, int32_t lb,
                   ta_result *out, char *cigar_buf, int64_t cap, int64_t *used);
@@ -125,8 +126,8 @@ int ta_align_pair(ta_ctx *ctx, const ta_params *p, const char *a, int32_t la, co
  * comes back from, a fixed device array of TA_PAIR_STATIC_SCRATCH bytes that
  * each GPU holds until the process ends (set up by ta_create); host staging
  * is the calling thread's stack.  Limits: la + lb <= TA_PAIR_STATIC_MAX and
- * the pair's direction codes must fit on chip (the form ta_align_pair uses
- * for such pairs); larger pairs get TA_E_LIMIT, never a fallback.  Calls
+ * the pair must be one that ta_align_pair's kernel takes (direction codes of
+ * at most about a CU's LDS); larger pairs get TA_E_LIMIT, never a fallback.  Calls
  * that overlap on one GPU (several contexts or threads) race on its array. */
 #define TA_PAIR_STATIC_MAX 4096
 #define TA_PAIR_STATIC_SCRATCH 32768

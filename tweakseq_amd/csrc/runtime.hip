@@ -1125,8 +1125,9 @@ void ta_batch_destroy(ta_batch *B) {
 // Origin of a shifted fill's values, which makes the lowest one -32,700.
 static int shift_base(const ta_params &p) { return -32700 - 3 * (p.gap_open - p.gap_extend); }
 
-// Whether score-only global couples take the shifted fill: it takes 26% fewer
-// instructions and is the faster one wherever its values fit.  Opening must
+// Whether score-only global couples take the shifted fill: it takes 17% fewer
+// instructions (1.75e9 against 2.12e9 for 130,816 pairs, 3.2 ms against 3.9)
+// and is the faster one wherever its values fit.  Opening must
 // cost at least extending (or gaps raise the values), and the nibbles'
 // constant must be a byte's (0..240).  A pair that global_i16_safe admits
 // has 3 |open| + (la + lb) |ext| < 16,000 and min(la, lb) max S < 32,000, so

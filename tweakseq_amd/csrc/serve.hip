@@ -89,8 +89,9 @@ struct Serve {
 };
 
 // Requests the device queue can take, in arrival order, while it has room
-// (lock held).  The queue is created on first use; without it (no room on the
-// device, or TWEAKALIGN_DEVICE_QUEUE=0) every request goes to a batch.
+// (lock held).  The queue is created on first use; without it (not asked for
+// with TWEAKALIGN_DEVICE_QUEUE=1, or no room on the device) every request goes
+// to a batch.
 void Serve::admit_dq() {
   if (!dq_tried) {
     dq_tried = true;
@@ -298,6 +299,22 @@ void Serve::loop() {
     // Admission in arrival order while memory and in-flight slots allow;
     // requests with the parameters of the first admitted one form the batch.
     if (!pending.empty() && inflight < max_inflight) {
+      // Requests of a burst come microseconds apart: as long as the next comes
+      // within 20 us, for 500 us at most, they join the batch.  (A batch runs
+      // as long as its longest pair, so a burst's first few, admitted one by
+      // one, would hold every slot meanwhile: 64 requests submitted together
+      // 2.6-3.2 ms so, 2.05 gathered; 2.4 with 10 us and 100 us.  A lone
+      // request waits the 20 us.)
+      using Clock = std::chrono::steady_clock;
+      const Clock::time_point t0 = Clock::now();
+      for (uint64_t n = changes;; n = changes) {
+        lk.unlock();
+        const Clock::time_point t1 = Clock::now();
+        while (Clock::now() - t1 < std::chrono::microseconds(20)) std::this_thread::yield();
+        lk.lock();
+        if (changes == n || stop || Clock::now() - t0 > std::chrono::microseconds(500)) break;
+      }
+      if (stop) break;
       Group g;
       for (auto it = pending.begin(); it != pending.end();) {
         Request *r = *it;
