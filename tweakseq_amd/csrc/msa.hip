@@ -666,15 +666,17 @@ int ta_msa(ta_ctx *ctx, const ta_params *p, const char *const *seqs, const int32
   if (!d_cols || !d_off || !d_nodes) return TA_E_NOMEM;
   const int32_t chunks = (*std::max_element(lens, lens + nseq) + 255) / 256;
   (void)hipGetLastError();
-  if (hipMemcpyAsync(d_off, off.data(), sizeof(int64_t) * (nseq + 1), hipMemcpyHostToDevice, st) ||
-      hipMemcpyAsync(d_nodes, nodes.data(), sizeof(MsaNode) * nc, hipMemcpyHostToDevice, st))
-    return TA_E_DEVICE;
-  hipLaunchKernelGGL(msa_columns_kernel, dim3((unsigned)nseq * (unsigned)chunks), dim3(256), 0, st, d_nodes, d_off,
-                     d_cols, chunks);
-  if (hipGetLastError() != hipSuccess ||
-      hipMemcpyAsync(cols, d_cols, sizeof(int32_t) * (size_t)off[nseq], hipMemcpyDeviceToHost, st) ||
-      hipStreamSynchronize(st))
-    return TA_E_DEVICE;
+  rc = hipMemcpyAsync(d_off, off.data(), sizeof(int64_t) * (nseq + 1), hipMemcpyHostToDevice, st) ||
+               hipMemcpyAsync(d_nodes, nodes.data(), sizeof(MsaNode) * nc, hipMemcpyHostToDevice, st)
+           ? TA_E_DEVICE
+           : TA_OK;
+  if (!rc)
+    hipLaunchKernelGGL(msa_columns_kernel, dim3((unsigned)nseq * (unsigned)chunks), dim3(256), 0, st, d_nodes, d_off,
+                       d_cols, chunks);
+  if (rc || hipGetLastError() != hipSuccess ||
+      hipMemcpyAsync(cols, d_cols, sizeof(int32_t) * (size_t)off[nseq], hipMemcpyDeviceToHost, st))
+    rc = TA_E_DEVICE;
+  if (hipStreamSynchronize(st) != hipSuccess || rc) return TA_E_DEVICE;  // (nothing queued reads the blocks after)
   tr.mark("columns");
   return TA_OK;
 }

@@ -520,7 +520,7 @@ int64_t long_estimate(const std::vector<HostPair> &hp, const std::vector<int> &l
 }
 
 // Regions a long-pair traceback computes ahead at most (344 KB each).
-constexpr int kLongAhead = 32768;
+constexpr int kLongAhead = 16384;
 
 // Residue codes one task's strips and columns read (expand_codes_kernel).
 struct CodeJob {
