@@ -17,8 +17,8 @@
 // running wave, so the pipeline cannot deadlock; waits are bounded.
 //
 // What it takes (from run to results in place, one wave or workgroup per task
-// against this): 16 pairs of 50 to 5,000 residues, global, 10.6 -> 1.15 ms a
-// call; one 1,500 x 1,571 pair 2.88 -> 0.52 ms; 1,024 local pairs of 300 to
+// against this): 16 pairs of 50 to 5,000 residues, global, 10.6 -> 1.13 ms a
+// call; one 1,500 x 1,571 pair 2.88 -> 0.43 ms; 1,024 local pairs of 300 to
 // 600 890 -> 423 us.
 //
 // Direction codes go to device memory, and a second kernel walks each pair
