@@ -411,6 +411,9 @@ __global__ __launch_bounds__(64 * LTW) void long_tb_kernel(LongArgs A) {
       __syncthreads();
       i = __builtin_amdgcn_readfirstlane(sy[LS_I]);
       j = __builtin_amdgcn_readfirstlane(sy[LS_J]);
+      // Read by every wave before wave 0 stores the next cell: where the next
+      // region is one computed ahead, no other barrier lies between the two.
+      __syncthreads();
     }
     if (wv == 0) {
       if (i == 0 && j > 0) rw.emit(1, j);
