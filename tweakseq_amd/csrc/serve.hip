@@ -83,7 +83,7 @@ struct Serve {
 
   void loop();
   void worker();
-  void run_group(Group &g, hipStream_t st);
+  void run_requests(Request *const *reqs, size_t n, hipStream_t st);
   void dq_loop();
   void admit_dq();
 };
@@ -191,16 +191,18 @@ void Serve::dq_loop() {
   }
 }
 
-// One batch from build to per-request results (a worker, without the lock).
-// A group is all letters or all resident sequences of one arena.
-void Serve::run_group(Group &g, hipStream_t st) {
+// One batch of n requests from build to per-request results (a worker,
+// without the lock): all letters or all resident sequences of one arena.
+// Where a request makes the batch fail (a letter outside the alphabet, a side
+// too long, memory) its halves run by themselves, so that it fails alone.
+void Serve::run_requests(Request *const *reqs, size_t n, hipStream_t st) {
   std::vector<ta_pair> pairs;
   ResidentBatch rb;
-  const bool resident = g.reqs[0]->resident;
+  const bool resident = reqs[0]->resident;
   if (resident) {
-    rb.arena = g.reqs[0]->rb.arena;
-    for (Request *r : g.reqs) {
-      const ResidentBatch &x = r->rb;
+    rb.arena = reqs[0]->rb.arena;
+    for (size_t q = 0; q < n; ++q) {
+      const ResidentBatch &x = reqs[q]->rb;
       rb.a_off.insert(rb.a_off.end(), x.a_off.begin(), x.a_off.end());
       rb.b_off.insert(rb.b_off.end(), x.b_off.begin(), x.b_off.end());
       rb.la.insert(rb.la.end(), x.la.begin(), x.la.end());
@@ -209,27 +211,35 @@ void Serve::run_group(Group &g, hipStream_t st) {
       rb.b_bound.insert(rb.b_bound.end(), x.b_bound.begin(), x.b_bound.end());
     }
   } else {
-    for (Request *r : g.reqs)
+    for (size_t q = 0; q < n; ++q) {
+      const Request *r = reqs[q];
       for (size_t k = 0; k < r->a.size(); ++k)
         pairs.push_back({r->a[k].data(), (int32_t)r->a[k].size(), r->b[k].data(), (int32_t)r->b[k].size()});
+    }
   }
   const int32_t np = resident ? (int32_t)rb.la.size() : (int32_t)pairs.size();
   ta_batch *B = nullptr;
   std::vector<ta_result> res;
   std::string text;
-  int rc = resident ? batch_create_on(ctx, &g.reqs[0]->p, nullptr, np, st, &B, nullptr, &rb)
-                    : batch_create_on(ctx, &g.reqs[0]->p, pairs.data(), np, st, &B);
+  int rc = resident ? batch_create_on(ctx, &reqs[0]->p, nullptr, np, st, &B, nullptr, &rb)
+                    : batch_create_on(ctx, &reqs[0]->p, pairs.data(), np, st, &B);
   if (!rc) rc = ta_batch_run(ctx, B);
   if (!rc) rc = ta_batch_wait(ctx, B);
   if (!rc) rc = batch_results_text(ctx, B, res, text);
   if (B) ta_batch_destroy(B);
+  if (n > 1 && rc != TA_OK && rc != TA_E_DEVICE) {
+    run_requests(reqs, n / 2, st);
+    run_requests(reqs + n / 2, n - n / 2, st);
+    return;
+  }
   std::lock_guard<std::mutex> lk(mu);
   int32_t k = 0;
-  for (Request *r : g.reqs) {
-    const int32_t n = (int32_t)r->npairs();
+  for (size_t q = 0; q < n; ++q) {
+    Request *r = reqs[q];
+    const int32_t np = (int32_t)r->npairs();
     r->rb = ResidentBatch();  // the arena is no longer read by this request
     if (r->state == RState::Cancelled) {  // cancelled while in flight: retire now
-      k += n;
+      k += np;
       all.erase(r->ticket);
       delete r;
       continue;
@@ -238,8 +248,8 @@ void Serve::run_group(Group &g, hipStream_t st) {
       r->state = RState::Failed;
       r->err = rc;
     } else {
-      r->res.assign(res.begin() + k, res.begin() + k + n);
-      const int64_t base = n ? r->res[0].cigar_off : 0;
+      r->res.assign(res.begin() + k, res.begin() + k + np);
+      const int64_t base = np ? r->res[0].cigar_off : 0;
       int64_t len = 0;
       for (auto &x : r->res) len += x.cigar_len;
       r->cigar.assign(text.data() + base, (size_t)len);
@@ -251,7 +261,7 @@ void Serve::run_group(Group &g, hipStream_t st) {
       r->a.clear(); r->a.shrink_to_fit();
       r->b.clear(); r->b.shrink_to_fit();
     }
-    k += n;
+    k += np;
   }
 }
 
@@ -267,7 +277,7 @@ void Serve::worker() {
     groups.pop_front();
     lk.unlock();
     if (have_stream) {
-      run_group(g, st);
+      run_requests(g.reqs.data(), g.reqs.size(), st);
     } else {
       std::lock_guard<std::mutex> g2(mu);
       for (Request *r : g.reqs) {
