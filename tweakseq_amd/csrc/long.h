@@ -46,23 +46,17 @@
 #include <hip/hip_runtime.h>
 
 #include "common.h"
+#include "longplan.h"
 #include "strips.h"
 #include "traceback.h"
 #include "walk.h"
 
 namespace ta {
 
-constexpr int LR = 8;                     // rows per lane of a forward strip
 constexpr int LONG_WAVES = 8;             // forward waves per CU
-constexpr int LST = GWAVE * LR;           // rows of a forward strip, and of a region at most
-constexpr int CKX = 512;                  // column checkpoint spacing
-constexpr int LMARGIN = 256;              // region columns beyond the diagonal through the walk's rows
-constexpr int LREG = LST + LMARGIN + CKX; // columns of a region at most
-constexpr int LREG_T = (LREG + 63 + 7) & ~7;
-constexpr int LTW = LST / 128;            // waves of a traceback workgroup: strips of a region
 constexpr int LAHEAD = 128;               // columns of a region ahead on either side of its guesses
 constexpr int LGUESS = 8192;              // columns on either side of the diagonal a guess is looked for in
-constexpr size_t LPLANES = (size_t)LTW * LREG_T / strip_spd(2) * 64;  // dwords of a region's codes
+static_assert(LST == GWAVE * LR && strip_spd(2) == 4, "shapes of longplan.h");
 
 struct LongPair {
   uint64_t a_off, b_off;  // residue codes (16-byte aligned, 32 bytes readable past the end)

@@ -499,28 +499,10 @@ bool long_pair(const ta_params &p, int la, int lb) {
   return p.lanes == TA_LANES_AUTO && (int64_t)la * lb >= kLongCells;
 }
 
-// Long pairs whose bottom rows and checkpoints share memory with other groups':
-// pairs [lp0, + npairs), queue items [it0, + nitems), ring entries [0, ring_n).
-struct LongGroup {
-  int lp0, npairs, it0, nitems;
-  uint64_t ring_n;
-};
-
-// Device memory a long pair is admitted for: a checkpoint row every 4,096 rows, a
-// checkpoint column every 1,024 columns, one region's codes.  (What a batch takes
-// is limited to this, or 16 GB where that is more.)
-int64_t long_pair_estimate(int64_t la, int64_t lb) {
-  const int64_t rl = ((lb + 7) & ~7ll) + 80, S = (la + 511) / 512;
-  return (S - 1) / 8 * 8 * rl + (lb - 1) / 1024 * S * 512 * 8 + 8 * 64 * ((std::min<int64_t>(lb, 5376) + 71) / 8) * 32;
+// Direction-plane bytes a pair of the other paths is admitted for.
+int64_t planes_estimate(int la, int lb) {
+  return (int64_t)((la + STRIP - 1) / STRIP) * ((lb + G + 7) / 8) * (G * R * 4);
 }
-int64_t long_estimate(const std::vector<HostPair> &hp, const std::vector<int> &lk) {
-  int64_t t = 0;
-  for (int k : lk) t += long_pair_estimate(hp[k].la, hp[k].lb);
-  return t;
-}
-
-// Regions a long-pair traceback computes ahead at most (344 KB each).
-constexpr int kLongAhead = 16384;
 
 // Residue codes one task's strips and columns read (expand_codes_kernel).
 struct CodeJob {
@@ -1014,7 +996,7 @@ struct ta_batch {
   std::vector<LongGroup> lgroups;
   LongPair *d_lp = nullptr;
   LongItem *d_litems = nullptr;
-  int2 *d_lring = nullptr, *d_lcol = nullptr;
+  int2 *d_lring = nullptr;    // bottom rows, then checkpoint columns, of a group
   uint32_t *d_wpl = nullptr;  // region codes of the traceback workgroups
   // Regions computed ahead (0: none), and the guesses they are placed by.
   int32_t lahead = 0;
@@ -1102,7 +1084,7 @@ void ta_batch_destroy(ta_batch *B) {
   dfree(B->d_ptb); dfree(B->d_pairs); dfree(B->d_fo); dfree(B->d_res); dfree(B->d_cig);
   dfree(B->d_ctr); dfree(B->d_fo_init);
   free_rerun(B);
-  dfree(B->d_lring); dfree(B->d_lcol); dfree(B->d_wpl);
+  dfree(B->d_lring); dfree(B->d_wpl);
   dfree(B->d_lahead); dfree(B->d_lcross);
   dfree(B->d_sring); dfree(B->d_splanes); dfree(B->d_sbest);
   dfree(B->d_sscore);
@@ -1215,7 +1197,7 @@ int ta_batch_create(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
 }
 
 int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32_t n, hipStream_t stream,
-                    ta_batch **out, const ta_tuning *force, const ResidentBatch *res) {
+                    ta_batch **out, const ta_tuning *force, const ResidentBatch *res, int64_t admitted) {
   if (!ctx || !p || !out || n < 0 || (n > 0 && !pairs && !res)) return TA_E_INVALID;
   *out = nullptr;
   if (params_check(p)) return TA_E_INVALID;
@@ -1680,43 +1662,30 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
     std::stable_sort(lk.begin(), lk.end(), [&](int x, int y) {
       return (int64_t)B->hp[x].la * B->hp[x].lb > (int64_t)B->hp[y].la * B->hp[y].lb;
     });
-    // Bottom rows and column checkpoints take about 1/32 byte a cell: pairs
-    // go in groups that share the memory one after the other.
-    const uint64_t limit = (uint64_t)std::max<int64_t>((int64_t)16 << 30, long_estimate(B->hp, lk));
-    uint64_t ring = 0, col = 0;
-    for (int k : lk) {
-      const HostPair &h = B->hp[k];
+    std::vector<std::pair<int32_t, int32_t>> shape;
+    for (int k : lk) shape.push_back({B->hp[k].la, B->hp[k].lb});
+    int64_t limit = -1;  // bytes they may take
+    if (admitted >= 0 && !lk.empty()) {
+      limit = admitted;
+      for (const HostPair &h : B->hp)
+        if (B->trace && h.path != 0 && h.path != 3) limit -= planes_estimate(h.la, h.lb);
+    }
+    if (const char *e = getenv("TWEAKALIGN_LONG_BYTES")) limit = std::max(0ll, atoll(e));
+    LongPlan lpl = long_plan(shape, p->traceback != 0, ctx->cus, limit);
+    for (size_t q = 0; q < lk.size(); ++q) {
+      const HostPair &h = B->hp[lk[q]];
       LongPair L{};
-      L.pid = k; L.m = h.la; L.n = h.lb; L.S = ceil_div(h.la, LST);
-      L.T = (h.lb + 63 + 7) & ~7;
+      L.pid = lk[q]; L.m = h.la; L.n = h.lb; L.S = long_strips(h.la);
+      L.T = (int32_t)long_steps(h.lb);
       L.a_off = h.a_off; L.b_off = h.b_off;
-      const uint64_t nr = (uint64_t)(L.S - 1) * (L.T + 8);
-      const uint64_t nc = p->traceback ? (uint64_t)((L.n - 1) / CKX) * L.S * LST : 0;
-      if (B->lgroups.empty() || (ring + col && 8 * (ring + col + nr + nc) > limit)) {
-        ring = col = 0;
-        B->lgroups.push_back(LongGroup{(int)B->longs.size(), 0, (int)B->litems.size(), 0, 0});
-      }
-      L.ring = ring; L.colck = col;
-      ring += nr; col += nc;
-      B->lring_n = std::max(B->lring_n, ring);
-      B->lcol_n = std::max(B->lcol_n, col);
-      L.item0 = (int32_t)B->litems.size();
-      for (int s = 0; s < L.S; ++s) B->litems.push_back(LongItem{(int32_t)B->longs.size(), s});
+      L.ring = lpl.at[q].ring; L.colck = lpl.at[q].col;
+      L.item0 = lpl.at[q].item0;
+      for (int s = 0; s < L.S; ++s) B->litems.push_back(LongItem{(int32_t)q, s});
       B->longs.push_back(L);
-      LongGroup &g = B->lgroups.back();
-      g.npairs += 1; g.nitems += L.S; g.ring_n = ring;
     }
-    if (!lk.empty() && p->traceback) {
-      B->long_wgs = std::max(1, std::min((int)lk.size(), 2 * ctx->cus));
-      // Regions ahead, where the pairs alone would not keep every CU at a
-      // region until the longest ends: 48 pairs (S up to 118, 3,300 in all)
-      // 16.7 -> 2.8 ms, 256 (S up to 196, 27,400) 41 -> 6.7; beyond, the same
-      // regions are computed either way.
-      int most = 0;
-      for (const LongPair &L : B->longs) most = std::max(most, L.S);
-      if ((int64_t)B->litems.size() < (int64_t)most * ctx->cus)
-        B->lahead = std::max(most, (int)std::min<size_t>(B->litems.size(), kLongAhead));
-    }
+    B->lgroups.swap(lpl.groups);
+    B->lring_n = lpl.entries; B->lcol_n = lpl.col_n;
+    B->long_wgs = lpl.wgs; B->lahead = lpl.ahead;
     if (const char *e = getenv("TWEAKALIGN_SPIN_LIMIT")) B->spin_limit = std::max(1, atoi(e));
     if (const char *e = getenv("TWEAKALIGN_WALK_GUARD")) B->guard_cap = std::max(0, atoi(e));
   }
@@ -1786,7 +1755,6 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
   rc = rc ? rc : dalloc(&B->d_res, (size_t)std::max(n, 1));
   rc = rc ? rc : dalloc(&B->d_cig, B->cig_bytes);
   rc = rc ? rc : dalloc(&B->d_lring, B->lring_n);
-  rc = rc ? rc : dalloc(&B->d_lcol, B->lcol_n);
   rc = rc ? rc : dalloc(&B->d_sring, B->sring_n);
   rc = rc ? rc : dalloc(&B->d_splanes, B->splanes_n);
   rc = rc ? rc : dalloc(&B->d_sbest, B->spairs.size());
@@ -1817,18 +1785,20 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
   return TA_OK;
 }
 
-int64_t batch_tb_estimate(const ta_params *p, const ta_pair *pairs, int32_t n) {
-  if (!p || (p->mode != TA_LOCAL && !p->traceback)) return 0;
-  int64_t t = 0;
+AdmitBytes batch_tb_estimate(const ta_params *p, const ta_pair *pairs, int32_t n) {
+  AdmitBytes t;
+  if (!p) return t;
+  const bool trace = p->mode == TA_LOCAL || p->traceback;
+  LongNeed longs;
+  longs.trace = p->traceback != 0;
   for (int32_t k = 0; k < n; ++k) {
     const int la = pairs[k].la, lb = pairs[k].lb;
     if (la <= 0 || lb <= 0) continue;
-    if (long_pair(*p, la, lb)) {
-      t += long_pair_estimate(la, lb);
-    } else {
-      t += (int64_t)ceil_div(la, STRIP) * ceil_div(lb + G, 8) * (G * R * 4);
-    }
+    if (long_pair(*p, la, lb)) longs.add(la, lb);
+    else if (trace) t.least += planes_estimate(la, lb);
   }
+  t.full = t.least + longs.full();
+  t.least += longs.least();
   return t;
 }
 
@@ -1935,7 +1905,7 @@ LongArgs long_args(ta_batch *B, int it0, int nit, int lp0, int nlp) {
   a.items = B->d_litems + it0; a.nitems = nit;
   a.ctr = B->d_ctr + 8;
   a.table = B->d_table; a.Kp = B->Kp; a.codes = B->d_codes;
-  a.ring = B->d_lring; a.colck = B->d_lcol; a.wpl = B->d_wpl;
+  a.ring = B->d_lring; a.colck = B->d_lring; a.wpl = B->d_wpl;
   a.pd = B->d_pairs; a.fo = B->d_fo; a.res = B->d_res; a.cig = B->d_cig;
   a.open = B->p.gap_open; a.ext = B->p.gap_extend;
   a.ckpt_on = B->p.traceback;

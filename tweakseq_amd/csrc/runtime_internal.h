@@ -115,10 +115,18 @@ inline int tune_key(const ta_params *p, int bucket) {
 // `force`: use this tuning instead of the context's table (the autotuner).
 // `res`: the pairs are resident sequences (resident_resolve) and `pairs` is
 // unused.
+// `admitted`: bytes the batch was admitted for (batch_tb_estimate), within
+// which its long pairs keep; -1: no limit.
 int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32_t n, hipStream_t stream,
-                    ta_batch **out, const ta_tuning *force = nullptr, const ResidentBatch *res = nullptr);
-// Direction-plane bytes a batch of these pairs would allocate (admission).
-int64_t batch_tb_estimate(const ta_params *p, const ta_pair *pairs, int32_t n);
+                    ta_batch **out, const ta_tuning *force = nullptr, const ResidentBatch *res = nullptr,
+                    int64_t admitted = -1);
+// Traceback memory of a batch of these pairs, for admission: what it cannot do
+// without, and what it takes where there is room (long pairs side by side and
+// with regions ahead; for score-only long pairs their rows).
+struct AdmitBytes {
+  int64_t least = 0, full = 0;
+};
+AdmitBytes batch_tb_estimate(const ta_params *p, const ta_pair *pairs, int32_t n);
 // Results of a finished batch with the CIGAR text in one string
 // (ta_result::cigar_off indexes `text`): ta_batch_results in one pass.
 int batch_results_text(ta_ctx *ctx, ta_batch *B, std::vector<ta_result> &out, std::string &text);

@@ -37,7 +37,11 @@ struct Request {
   uint64_t ticket = 0;
   ta_params p{};
   std::vector<std::string> a, b;
-  int64_t tb_bytes = 0;
+  AdmitBytes tb;
+  // Counted against the budget while in flight: all it can use, or the whole
+  // budget if that is less (it then runs alone, in less).
+  int64_t counted = 0;
+  void count(int64_t budget) { counted = std::max(tb.least, std::min(tb.full, budget)); }
   RState state = RState::Pending;
   int err = 0;
   bool walk_failed = false;    // a pair's walk gave up: delivered with TA_E_WALK
@@ -105,13 +109,14 @@ void Serve::admit_dq() {
     if (r->state == RState::Cancelled) { it = pending.erase(it); continue; }
     if (r->dq < 0) r->dq = devq_eligible(dq, &r->p, r->a, r->b) ? 1 : 0;
     if (!r->dq) { ++it; continue; }
-    if (r->tb_bytes > budget) {  // the budget was lowered below it: it can never run
+    if (r->tb.least > budget) {  // the budget was lowered below it: it can never run
       r->state = RState::Failed;
       r->err = TA_E_BUDGET;
       it = pending.erase(it);
       continue;
     }
-    if (used + r->tb_bytes > budget) break;
+    r->count(budget);
+    if (used + r->counted > budget) break;
     DevqJob *job = nullptr;
     const int rc = devq_admit(dq, &r->p, r->a, r->b, &job);
     if (rc == TA_E_PENDING) break;  // device memory or slots: wait for completions
@@ -123,7 +128,7 @@ void Serve::admit_dq() {
     }
     r->job = job;
     r->state = RState::InFlight;
-    used += r->tb_bytes;
+    used += r->counted;
     dq_jobs.push_back(r);
     any = true;
   }
@@ -164,7 +169,7 @@ void Serve::dq_loop() {
     lk.lock();
     for (size_t k = 0; k < fin.size(); ++k) {
       Request *r = fin[k];
-      used -= r->tb_bytes;
+      used -= r->counted;
       if (r->state == RState::Cancelled) {
         all.erase(r->ticket);
         delete r;
@@ -217,12 +222,14 @@ void Serve::run_requests(Request *const *reqs, size_t n, hipStream_t st) {
         pairs.push_back({r->a[k].data(), (int32_t)r->a[k].size(), r->b[k].data(), (int32_t)r->b[k].size()});
     }
   }
+  int64_t admitted = 0;
+  for (size_t q = 0; q < n; ++q) admitted += reqs[q]->counted;
   const int32_t np = resident ? (int32_t)rb.la.size() : (int32_t)pairs.size();
   ta_batch *B = nullptr;
   std::vector<ta_result> res;
   std::string text;
-  int rc = resident ? batch_create_on(ctx, &reqs[0]->p, nullptr, np, st, &B, nullptr, &rb)
-                    : batch_create_on(ctx, &reqs[0]->p, pairs.data(), np, st, &B);
+  int rc = resident ? batch_create_on(ctx, &reqs[0]->p, nullptr, np, st, &B, nullptr, &rb, admitted)
+                    : batch_create_on(ctx, &reqs[0]->p, pairs.data(), np, st, &B, nullptr, nullptr, admitted);
   if (!rc) rc = ta_batch_run(ctx, B);
   if (!rc) rc = ta_batch_wait(ctx, B);
   if (!rc) rc = batch_results_text(ctx, B, res, text);
@@ -330,7 +337,7 @@ void Serve::loop() {
         Request *r = *it;
         if (r->state == RState::Cancelled) { it = pending.erase(it); continue; }
         if (r->dq == 1) { ++it; continue; }  // waits for room in the device queue
-        if (r->tb_bytes > budget) {  // the budget was lowered below it: it can never run
+        if (r->tb.least > budget) {  // the budget was lowered below it: it can never run
           r->state = RState::Failed;
           r->err = TA_E_BUDGET;
           it = pending.erase(it);
@@ -341,8 +348,9 @@ void Serve::loop() {
           ++it;
           continue;
         }
-        if (used + g.tb + r->tb_bytes > budget) break;
-        g.tb += r->tb_bytes;
+        r->count(budget);
+        if (used + g.tb + r->counted > budget) break;
+        g.tb += r->counted;
         r->state = RState::InFlight;
         g.reqs.push_back(r);
         it = pending.erase(it);
@@ -424,7 +432,7 @@ int ta_submit(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32_t n, 
   Serve *s = serve_of(ctx);
   Request *r = new Request();
   r->p = *p;
-  r->tb_bytes = batch_tb_estimate(p, pairs, n);
+  r->tb = batch_tb_estimate(p, pairs, n);
   r->a.reserve(n);
   r->b.reserve(n);
   for (int32_t k = 0; k < n; ++k) {
@@ -432,7 +440,7 @@ int ta_submit(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32_t n, 
     r->b.emplace_back(pairs[k].b, (size_t)pairs[k].lb);
   }
   std::lock_guard<std::mutex> g(s->mu);
-  if (r->tb_bytes > s->budget) {
+  if (r->tb.least > s->budget) {
     delete r;
     return TA_E_BUDGET;
   }
@@ -458,10 +466,10 @@ int ta_submit_resident(ta_ctx *ctx, const ta_params *p, const ta_seq_pair *pairs
   r->dq = 0;  // batches only: the device queue stages letters from host memory
   std::vector<ta_pair> lens((size_t)n);
   for (int32_t k = 0; k < n; ++k) lens[k] = ta_pair{nullptr, r->rb.la[k], nullptr, r->rb.lb[k]};
-  r->tb_bytes = batch_tb_estimate(p, lens.data(), n);
+  r->tb = batch_tb_estimate(p, lens.data(), n);
   Serve *s = serve_of(ctx);
   std::lock_guard<std::mutex> g(s->mu);
-  if (r->tb_bytes > s->budget) {
+  if (r->tb.least > s->budget) {
     delete r;
     return TA_E_BUDGET;
   }
