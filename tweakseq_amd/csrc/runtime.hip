@@ -1035,6 +1035,8 @@ struct ta_batch {
   hipGraphExec_t gexec = nullptr;
   // timing
   hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
+  std::vector<hipEvent_t> gev;  // around the tracebacks of all long groups but the last
+  bool gev_timed = false;       // by the last run
   double ms[4] = {0, 0, 0, 0};
   // plain (one launch per pair) resources, built on first use
   bool plain_ready = false;
@@ -1101,6 +1103,8 @@ void ta_batch_destroy(ta_batch *B) {
   dfree(B->d_plain_tasks); dfree(B->d_prow); dfree(B->d_pcol); dfree(B->d_pring);
   dfree(B->d_ptbuf); dfree(B->d_pptb); dfree(B->d_plain_rtasks); dfree(B->d_pptb_r);
   for (auto &e : B->ev)
+    if (e) (void)hipEventDestroy(e);
+  for (auto &e : B->gev)
     if (e) (void)hipEventDestroy(e);
   if (B->gexec) (void)hipGraphExecDestroy(B->gexec);
   if (B->graph) (void)hipGraphDestroy(B->graph);
@@ -1776,6 +1780,9 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
   }
   for (auto &e : B->ev)
     if (!rc && hipEventCreate(&e) != hipSuccess) rc = TA_E_DEVICE;
+  if (p->traceback && B->lgroups.size() > 1) B->gev.assign(2 * (B->lgroups.size() - 1), nullptr);
+  for (auto &e : B->gev)
+    if (!rc && hipEventCreate(&e) != hipSuccess) rc = TA_E_DEVICE;
   tr.mark("allocations");
   // Drained on every path: the blocks of a failed creation go back to the
   // cache only after the copies queued into them.  The letter check comes
@@ -2086,7 +2093,9 @@ int launch_init(ta_batch *B) {
   return TA_OK;
 }
 
-int launch_fills(ta_ctx *ctx, ta_batch *B) {
+// `timed`: the tracebacks among them are timed by themselves (not while a
+// graph is captured).
+int launch_fills(ta_ctx *ctx, ta_batch *B, bool timed) {
   const Plan &pl = B->plan;
   const int n2[3] = {(int)pl.list2[0].spans.size(), (int)pl.list2[1].spans.size(), (int)pl.list2[2].spans.size()};
   const int n1[3] = {(int)pl.list1[0].spans.size(), (int)pl.list1[1].spans.size(), 0};
@@ -2099,7 +2108,10 @@ int launch_fills(ta_ctx *ctx, ta_batch *B) {
   for (size_t g = 0; !rc && g < B->lgroups.size(); ++g) {
     const LongGroup &L = B->lgroups[g];
     rc = launch_long_fwd(ctx, B, L.it0, L.nitems, 0, L.ring_n);
-    if (!rc && g + 1 < B->lgroups.size()) rc = launch_long_tb(ctx, B, L.lp0, L.npairs, B->lahead > 0);
+    if (rc || g + 1 == B->lgroups.size() || B->gev.empty()) continue;
+    if (timed) HIPCHK(hipEventRecord(B->gev[2 * g], B->stream));
+    rc = launch_long_tb(ctx, B, L.lp0, L.npairs, B->lahead > 0);
+    if (timed) HIPCHK(hipEventRecord(B->gev[2 * g + 1], B->stream));
   }
   return rc;
 }
@@ -2129,7 +2141,7 @@ int run_graph(ta_ctx *ctx, ta_batch *B) {
   if (!B->gexec) {
     HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
     int rc = launch_init(B);
-    if (!rc) rc = launch_fills(ctx, B);
+    if (!rc) rc = launch_fills(ctx, B, false);
     if (!rc) rc = launch_tracebacks(ctx, B);
     hipGraph_t g = nullptr;
     const hipError_t e = hipStreamEndCapture(st, &g);
@@ -2157,7 +2169,7 @@ int ta_batch_run(ta_ctx *ctx, ta_batch *B) {
   int rc = launch_init(B);
   if (rc) return rc;
   HIPCHK(hipEventRecord(B->ev[0], st));
-  rc = launch_fills(ctx, B);
+  rc = launch_fills(ctx, B, true);
   if (rc) return rc;
   HIPCHK(hipEventRecord(B->ev[1], st));
   if (B->may_saturate) {
@@ -2170,7 +2182,7 @@ int ta_batch_run(ta_ctx *ctx, ta_batch *B) {
   rc = launch_tracebacks(ctx, B);
   if (rc) return rc;
   HIPCHK(hipEventRecord(B->ev[3], st));
-  B->phases_timed = true;
+  B->phases_timed = B->gev_timed = true;
   return TA_OK;
 }
 
@@ -2189,6 +2201,12 @@ int ta_batch_wait(ta_ctx *ctx, ta_batch *B) {
     if (hipEventElapsedTime(&t, B->ev[0], B->ev[1]) == hipSuccess) B->ms[0] = t;
     if (hipEventElapsedTime(&t, B->ev[1], B->ev[2]) == hipSuccess) B->ms[1] = t;
     if (hipEventElapsedTime(&t, B->ev[2], B->ev[3]) == hipSuccess) B->ms[2] = t;
+    // long groups but the last are walked back among the fills
+    for (size_t g = 0; B->gev_timed && g + 1 < B->gev.size(); g += 2) {
+      if (hipEventElapsedTime(&t, B->gev[g], B->gev[g + 1]) != hipSuccess) continue;
+      B->ms[0] -= t;
+      B->ms[2] += t;
+    }
   }
   if (hipEventElapsedTime(&t, B->ev[0], B->ev[3]) == hipSuccess) B->ms[3] = t;
   if (!B->longs.empty() || B->ncoop2 || B->ncoop1 || B->strips) {
@@ -2608,6 +2626,7 @@ int ta_batch_run_plain(ta_ctx *ctx, ta_batch *B, int32_t first, int32_t count) {
     B->plain_rerun = rerun_of;
     B->plain_ready = true;
   }
+  B->gev_timed = false;
   HIPCHK(hipEventRecord(B->ev[0], st));
   // the counters and the error word (d_ctr[10]) start at 0, as init_kernel
   // leaves them for a batch run
