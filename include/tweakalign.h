@@ -227,7 +227,9 @@ typedef struct {
 int ta_tune_bucket(const ta_pair *pairs, int32_t n);
 /* Times candidate tunings on these pairs (best of `repeats` runs each),
  * stores the fastest in the context for this kind of batch and returns it;
- * ta_batch_create / ta_align_batch / serving on this context then use it. */
+ * ta_batch_create / ta_align_batch / serving on this context then use it.
+ * (Batches of few pairs run pair by pair all over the GPU, whatever the
+ * tuning; candidates are timed in the form that larger ones take.) */
 int ta_autotune(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32_t n, int32_t repeats,
                 ta_tuning *best, double *best_ms);
 /* Set / read the context's tuning for (p's mode, traceback, alphabet, bucket)

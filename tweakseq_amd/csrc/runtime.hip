@@ -1549,7 +1549,8 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
   }
 
   tr.mark("pairs");
-  plan_strips(ctx, B);
+  // (a tuning is a shape of the task form, so candidates are timed in it)
+  if (!force) plan_strips(ctx, B);
   // Couples: local pairs pad to the longer column count; global couples
   // need equal column counts (so H(m, n) of both sits in the last column).
   Plan &pl = B->plan;
