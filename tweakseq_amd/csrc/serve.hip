@@ -75,6 +75,7 @@ struct Serve {
   int max_inflight = 4, inflight = 0;
   uint64_t next_ticket = 1;
   uint64_t changes = 0;         // bumped whenever admission may change its mind
+  uint64_t arrivals = 0;        // requests submitted
   bool stop = false, stop_workers = false;
   std::thread th;
   std::vector<std::thread> workers;
@@ -90,7 +91,19 @@ struct Serve {
   void run_requests(Request *const *reqs, size_t n, hipStream_t st);
   void dq_loop();
   void admit_dq();
+  bool room_for_first();
 };
+
+// Whether the first request that waits for a batch fits beside those in
+// flight (lock held).
+bool Serve::room_for_first() {
+  for (Request *r : pending) {
+    if (r->state == RState::Cancelled || r->dq == 1 || r->tb.least > budget) continue;
+    r->count(budget);
+    return used + r->counted <= budget;
+  }
+  return false;
+}
 
 // Requests the device queue can take, in arrival order, while it has room
 // (lock held).  The queue is created on first use; without it (not asked for
@@ -317,19 +330,24 @@ void Serve::loop() {
     // requests with the parameters of the first admitted one form the batch.
     if (!pending.empty() && inflight < max_inflight) {
       // Requests of a burst come microseconds apart: as long as the next comes
-      // within 20 us, for 500 us at most, they join the batch.  (A batch runs
-      // as long as its longest pair, so a burst's first few, admitted one by
-      // one, would hold every slot meanwhile: 64 requests submitted together
-      // 2.6-3.2 ms so, 2.05 gathered; 2.4 with 10 us and 100 us.  A lone
-      // request waits the 20 us.)
+      // within 20 us, for 500 us at most, they join the batch, unless there is no
+      // room for the first anyway.  (A batch runs as long as its longest pair,
+      // so a burst's first few, admitted one by one, would hold every slot
+      // meanwhile: 64 requests submitted together from Python 2.6-3.2 ms so,
+      // 2.15 gathered; 2.4 with 10 us and 100 us, or with the window opened only
+      // while batches run or several wait.  A lone request waits the 20 us, of
+      // 270.  p50 with / without where nothing runs, one pair a request:
+      // 2,000/s 250 / 242 us, 10,000/s 303 / 306, 40,000/s 430 / 426, 80,000/s
+      // 531 / 492; 8 pairs of up to 2,500 each, 2,000/s 861 / 854.)
       using Clock = std::chrono::steady_clock;
       const Clock::time_point t0 = Clock::now();
-      for (uint64_t n = changes;; n = changes) {
+      while (!stop && room_for_first()) {
+        const uint64_t n = arrivals;
         lk.unlock();
         const Clock::time_point t1 = Clock::now();
         while (Clock::now() - t1 < std::chrono::microseconds(20)) std::this_thread::yield();
         lk.lock();
-        if (changes == n || stop || Clock::now() - t0 > std::chrono::microseconds(500)) break;
+        if (arrivals == n || Clock::now() - t0 > std::chrono::microseconds(500)) break;
       }
       if (stop) break;
       Group g;
@@ -449,6 +467,7 @@ int ta_submit(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32_t n, 
   s->pending.push_back(r);
   *ticket = r->ticket;
   ++s->changes;
+  ++s->arrivals;
   s->cv.notify_all();
   return TA_OK;
 }
@@ -478,6 +497,7 @@ int ta_submit_resident(ta_ctx *ctx, const ta_params *p, const ta_seq_pair *pairs
   s->pending.push_back(r);
   *ticket = r->ticket;
   ++s->changes;
+  ++s->arrivals;
   s->cv.notify_all();
   return TA_OK;
 }
