@@ -98,7 +98,7 @@ struct Serve {
 // flight (lock held).
 bool Serve::room_for_first() {
   for (Request *r : pending) {
-    if (r->state == RState::Cancelled || r->dq == 1 || r->tb.least > budget) continue;
+    if (r->state == RState::Cancelled || r->dq == 1 || (dq && r->dq < 0) || r->tb.least > budget) continue;
     r->count(budget);
     return used + r->counted <= budget;
   }
@@ -354,7 +354,8 @@ void Serve::loop() {
       for (auto it = pending.begin(); it != pending.end();) {
         Request *r = *it;
         if (r->state == RState::Cancelled) { it = pending.erase(it); continue; }
-        if (r->dq == 1) { ++it; continue; }  // waits for room in the device queue
+        // waits for room in the device queue, or came after it was last asked
+        if (r->dq == 1 || (dq && r->dq < 0)) { ++it; continue; }
         if (r->tb.least > budget) {  // the budget was lowered below it: it can never run
           r->state = RState::Failed;
           r->err = TA_E_BUDGET;
