@@ -1,11 +1,13 @@
 """Device-queue serving beside batches: requests that the queue takes go there
-also while a batch gathers."""
+also while a batch gathers, and letter requests through the queue mix with
+requests on resident sequences, which go to batches."""
 import random
 import time
 
 import pytest
 
 import tweakseq_amd as ta
+import test_gpu_resident
 from test_gpu_parity import compare, mutate, oracle_results, rand_prot
 
 pytestmark = pytest.mark.gpu
@@ -44,5 +46,15 @@ def test_a_gathering_batch_leaves_queue_requests_alone(monkeypatch):
             long_res = eng.poll(*first)
             assert time.time() - t0 < 60
         assert long_res == eng.align(long_pairs, params)
+    finally:
+        eng.close()
+
+
+@pytest.mark.parametrize("queue", ["0", "1"])
+def test_resident_beside_letter_requests(queue, monkeypatch):
+    monkeypatch.setenv("TWEAKALIGN_DEVICE_QUEUE", queue)
+    eng = ta.Engine(0)
+    try:
+        test_gpu_resident.test_served_resident_requests_equal_oracle(eng)
     finally:
         eng.close()
