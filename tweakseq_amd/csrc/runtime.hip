@@ -941,8 +941,8 @@ __global__ void patch_ptb_kernel(const PtbPatch *p, int n, PairTB *ptb) {
 }
 
 // Start of a run: work-queue counters to 0, fill outputs to their initial
-// values (empty pairs keep theirs), long-pair progress counters to 0.  A
-// kernel rather than memset / memcpy nodes, so a captured run is all kernels.
+// values (empty pairs keep theirs).  A kernel rather than memset / memcpy
+// nodes, so a captured run is all kernels.
 __global__ void init_kernel(int32_t *ctr, int nctr, FillOut *fo, const FillOut *fo_init, int n) {
   const int tid = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
   for (int k = tid; k < nctr; k += stride) ctr[k] = 0;
