@@ -194,7 +194,7 @@ int ta_align_resident(ta_ctx *ctx, const ta_params *p, const ta_seq_pair *pairs,
  * A request counts 4 bits a cell of its pairs; long pairs (TA_F_LONG) count
  * the checkpoints and traceback regions they hold, up to all pairs side by
  * side.  TA_E_BUDGET: more than the budget even with its long pairs one after
- * the other.  Score-only requests are never refused (long pairs among them
+ * the other.  Global score-only requests are never refused (long pairs among them
  * wait for room for their rows). */
 int ta_serve_config(ta_ctx *ctx, int64_t tb_budget_bytes, int32_t max_inflight);
 int ta_submit(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32_t n,
