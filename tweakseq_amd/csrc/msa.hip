@@ -100,6 +100,10 @@ __host__ __device__ inline int join_steps(int lb) { return (lb + 63 + 7) & ~7; }
 __host__ __device__ inline int join_strips(int la) { return (la + JRS - 1) / JRS; }
 // LDS of the int32 ring: a column's bottom row at entry column + 64.
 __host__ __device__ inline int join_ring(int lb) { return join_steps(lb) + 80; }
+// Bytes of the ring of a join with lb columns (int64: H and F of every column).
+inline int64_t join_ring_bytes(int lb, bool wide) {
+  return wide ? 2 * (int64_t)sizeof(int64_t) * (lb + 2) : (int64_t)sizeof(int2) * join_ring(lb);
+}
 
 __device__ __forceinline__ const int4 *join_row(const JoinSide &s, const int4 *leaf, int c) {
   return s.code ? leaf + s.code[c] * CI : s.rows + (int64_t)c * CI;
@@ -202,6 +206,8 @@ struct JoinIO : StripGroupIO {
 
 // LDS words of the sync area: a progress counter per wave, then as in StripGroupIO.
 enum { JS_PROG = 0, JS_STATUS = 16, JS_READY = 17, JS_RUNS = 18, JS_ZERO = 32, JS_EDGE = 48, JS_WORDS = 64 };
+// A join's LDS beside the ring: the sync area and the walk's window.
+constexpr int64_t JOIN_LDS = 4 * (JS_WORDS + StripWindow<JR>::WL * StripWindow<JR>::WD);
 
 // The strips of a join in int64, plain recurrence: H, E, F with a column test
 // a step; direction codes as strip.h's.
@@ -596,6 +602,9 @@ int ta_msa(ta_ctx *ctx, const ta_params *p, const char *const *seqs, const int32
       strips = (int32_t)std::max<int64_t>(strips, S);
       tiles = (int32_t)std::max<int64_t>(tiles, S * ((T + 63) / 64));
     }
+    // The ring holds a bottom row of every column: 20,017 of them fit a CU's
+    // LDS (10,078 in int64).  A larger launch would take the whole queue down.
+    if (join_ring_bytes(max_lb, wide) + JOIN_LDS > ctx->lds_max) return TA_E_INVALID;
     const bool root = L == top;
     int32_t *d_map = (int32_t *)hold(sizeof(int32_t) * (size_t)col_total);
     int4 *d_out = root ? nullptr : (int4 *)device_alloc(sizeof(int4) * CI * (size_t)col_total);
@@ -631,7 +640,7 @@ int ta_msa(ta_ctx *ctx, const ta_params *p, const char *const *seqs, const int32
       const dim3 grid((unsigned)nj, (unsigned)std::min(tiles, 65535));
       if (!rc) hipLaunchKernelGGL(m24 ? msa_scores_kernel<true> : msa_scores_kernel<false>, grid, dim3(256), 0, st, a,
                                   wide ? 0 : -p->gap_open - p->gap_extend, wide ? 0 : p->gap_extend - p->gap_open);
-      const size_t lds = wide ? 2 * sizeof(int64_t) * (size_t)(max_lb + 2) : sizeof(int2) * (size_t)join_ring(max_lb);
+      const size_t lds = (size_t)join_ring_bytes(max_lb, wide);
       if (!rc) hipLaunchKernelGGL(wide ? msa_join_kernel<true> : msa_join_kernel<false>, dim3((unsigned)nj),
                                   dim3(64 * std::min(strips, JWMAX)), lds, st, a);
       if (rc || hipGetLastError() != hipSuccess ||
