@@ -1256,9 +1256,11 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
   // sequence also gets the sum over its residues of the best score the
   // residue can reach against any letter (0 if none is positive): no local
   // alignment of it scores more, which decides whether int16 can saturate.
-  int best[32] = {0};
+  int best[32] = {0}, maxbest = 0;
   for (int r = 0; r < B->alph.K; ++r)
     for (int c = 0; c < B->alph.K; ++c) best[r] = std::max<int>(best[r], B->alph.S[r * B->alph.K + c]);
+  for (int r = 0; r < B->alph.K; ++r) maxbest = std::max(maxbest, best[r]);
+  const int64_t sat_limit = 32767 - 2L * B->alph.maxS;
   // Unique sequences (by pointer and length) and their offsets in the code
   // array.  Pointers are split by hash over the host threads; each thread
   // scans every pair and keeps a table for its share only (a few hundred KB,
@@ -1326,6 +1328,7 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
   std::vector<Uniq> &uq = tl_uq;
   size_t ctotal = 0;  // bytes of the unique sequences' codes
   std::vector<int32_t> base(T + 1, 0);  // first unique entry of each thread's share
+  std::vector<char> sums(T, 0);         // whether a share has a sequence whose bound must be summed
   if (!res) {
     ua.resize((size_t)n);
     ub.resize((size_t)n);
@@ -1372,8 +1375,9 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
     });
     tr.mark("dedupe hash");
     // Global order: partition by partition; each sequence starts 16-byte
-    // aligned (walker windows).  Offsets and the flat array, per partition on
-    // the threads, from the partitions' counts and byte totals.
+    // aligned (walker windows).  Offsets, bounds from the lengths alone and the
+    // flat array, per partition on the threads, from the partitions' counts and
+    // byte totals.
     std::vector<size_t> bbase(T + 1, 0);
     for (int t = 0; t < T; ++t) {
       base[t + 1] = base[t] + (int32_t)part[t].size();
@@ -1388,6 +1392,10 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
       for (const Uniq &e : part[t]) {
         *dst = e;
         dst->off = at;
+        if (local) {
+          dst->bound = (int64_t)e.len * maxbest;
+          if (dst->bound > sat_limit) sums[t] = 1;
+        }
         at += ((size_t)e.len + 15) & ~(size_t)15;
         ++dst;
       }
@@ -1430,13 +1438,11 @@ int batch_create_on(ta_ctx *ctx, const ta_params *p, const ta_pair *pairs, int32
   // (0 if none is positive) bounds any local alignment of it; it decides
   // whether int16 can saturate, which only a sequence longer than
   // limit / (best of all letters) can reach, so only such sequences are summed.
-  int maxbest = 0;
-  for (int r = 0; r < B->alph.K; ++r) maxbest = std::max(maxbest, best[r]);
-  const int64_t sat_limit = 32767 - 2L * B->alph.maxS;
-  if (local && !res)
+  // (A pass of the host threads that finds none costs small batches 30-45 us: 256
+  // pairs of up to 20 residues 251-271 us a call with it, 207-220 without.)
+  if (std::any_of(sums.begin(), sums.end(), [](char x) { return x != 0; }))
     parallel_for(uq.size(), [&](size_t u) {
       Uniq &e = uq[u];
-      e.bound = (int64_t)e.len * maxbest;
       if (e.bound <= sat_limit) return;
       int64_t sum = 0;
       const unsigned char *src = (const unsigned char *)e.s;
